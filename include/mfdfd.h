@@ -88,7 +88,7 @@ typedef struct {
     int32_t method;           /* MFD_SQMR, MFD_COCG, MFD_BICGSTAB, or -1 (SQMR; BiCGSTAB with a complex Bloch phase) */
     double inner_tol;         /* mixed: tightest inner reduction per FP32 cycle (1e-5) */
     int32_t check_every;      /* iterations between host convergence checks (32) */
-    int32_t use_graph;        /* capture a chunk of iterations in a hipGraph */
+    int32_t use_graph;        /* capture a chunk of iterations in a hipGraph (not needed by the one-kernel solver) */
 } mfd_solve_opts;
 
 typedef struct {
@@ -249,7 +249,8 @@ int mfd_op_autotune(mfd_op *op, int64_t nrhs, int iters, int tile64[3], int tile
  * to 4 and 1) while a launch would have fewer than 256 tiles, TY = 8 for
  * full ε on a one-cell z axis where that still gives 256 tiles, and 32-wide
  * tiles (xcd_order 3) when that stencil serves and they leave fewer lanes of
- * the last x tile idle than 64-wide ones. */
+ * the last x tile idle than 64-wide ones.  Small SQMR solves do not use the
+ * tiles (one kernel keeps the whole grid on chip) unless they were set here. */
 int mfd_op_set_tile(mfd_op *op, int prec, int ty, int kz, int xcd_order);
 /* Average device time (ms) of one apply of the solver's stencil kernel
  * (MFD_FP64: A; MFD_MIXED: the complex-FP32 inner operator) */
@@ -296,8 +297,9 @@ int mfd_solve_dev_noalloc(mfd_op *op, const void *b, void *e, int64_t nrhs, cons
                           mfd_solve_stats *st);
 /* Solve `count` independent systems A_p e_p = b_p, one RHS each (every
  * problem keeps its own grid, ε and ω; all operators share one context).
- * Each chunk of iterations of all unconverged problems is one hipGraph launch
- * whose per-problem branches run concurrently.  b[p], e[p]: host arrays of
+ * Each round gives every unconverged problem one launch (a chunk of iterations
+ * as its own hipGraph, or, small problems, the one-kernel solver's) and reads
+ * all results back at once.  b[p], e[p]: host arrays of
  * 3·M_p values (e holds the initial guess); st: `count` entries or null.
  * b = 0, NaN residuals and unconverged problems are handled per problem as
  * mfd_solve handles its columns.

@@ -13,7 +13,7 @@
 // the positive end, Cₘ backward differences with the ghost at the negative
 // end; a Bloch ghost is the wrapped value times e^{∓ikL}, a non-Bloch ghost
 // is zero.
-#include "op.hpp"
+#include "resident.hpp"
 #include "assembly.hpp"
 #include <cmath>
 #include <cstring>
@@ -22,18 +22,7 @@
 
 namespace mfd {
 
-constexpr int NPART = 16384;  // max blocks per reduction (per RHS)
-constexpr int NGRID_MAX = 2048;   // grid cap of the grid-stride vector kernels
-constexpr int BS = 256;
-enum { MODE_A = 0, MODE_P = 1 };
-enum { EPI_STORE = 0, EPI_RESID = 1, EPI_DOT = 2 };
-
 // --------------------------------------------------------------- helpers
-
-template <typename R>
-__device__ inline cx<R> czero() { return mk<R>((R)0, (R)0); }
-template <typename R>
-__device__ inline cx<R> cone() { return mk<R>((R)1, (R)0); }
 
 template <typename R>
 __device__ inline void cell3(const DGrid<R> &g, int64_t p, int &i, int &j, int &k) {
@@ -163,26 +152,6 @@ __device__ inline cx<R> ccdiag(const DGrid<R> &g, const OpData<R> &od, int u, in
     return s;
 }
 
-// block reduction of NV doubles; result valid in thread 0
-template <int NV>
-__device__ inline void block_sum(double (&v)[NV]) {
-    __shared__ double sh[8][NV];
-#pragma unroll
-    for (int a = 0; a < NV; ++a)
-        for (int o = 32; o > 0; o >>= 1) v[a] += __shfl_down(v[a], o, 64);
-    int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0)
-        for (int a = 0; a < NV; ++a) sh[wv][a] = v[a];
-    __syncthreads();
-    if (threadIdx.x == 0)
-        for (int a = 0; a < NV; ++a) {
-            double s = 0;
-            for (int b = 0; b < (int)(blockDim.x >> 6); ++b) s += sh[b][a];
-            v[a] = s;
-        }
-    __syncthreads();
-}
-
 // write this block's partial (block bid of nb); returns true in every thread of
 // the last block to arrive, which then holds the fixed-order total in tot
 // (thread 0) and re-arms the counter
@@ -214,26 +183,6 @@ __device__ inline bool reduce_last_n(double (&v)[NV], double *part, unsigned *cn
 template <int NV>
 __device__ inline bool reduce_last(double (&v)[NV], double *part, unsigned *cnt, double (&tot)[NV]) {
     return reduce_last_n<NV>(v, part, cnt, tot, (int)blockIdx.x, (int)gridDim.x);
-}
-
-// Grid reductions on the solver's hot path: every block writes its partial
-// sums with plain stores and a one-block finish kernel, launched next on the
-// same stream, adds them in a fixed order (deterministic) and updates the
-// solver scalars.  The kernel boundary orders the two, so no block needs a
-// device-scope fence or a shared counter.
-template <int NV>
-__device__ inline void block_partial(double (&v)[NV], double *part, int bid) {
-    block_sum<NV>(v);
-    if (threadIdx.x == 0)
-        for (int a = 0; a < NV; ++a) part[4 * bid + a] = v[a];
-}
-// fixed-order sum of nb partials by one block; result in thread 0
-template <int NV>
-__device__ inline void sum_partials(const double *part, int nb, double (&tot)[NV]) {
-    for (int a = 0; a < NV; ++a) tot[a] = 0;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x)
-        for (int a = 0; a < NV; ++a) tot[a] += part[4 * b + a];
-    block_sum<NV>(tot);
 }
 
 // after the stencil with EPI_DOT: σ = qᵀPq, α = ρ/σ (one block per RHS)
@@ -673,25 +622,7 @@ __global__ __launch_bounds__(BS) void k_fin_r(const double *part, int nb, Scal *
     double tot[3];
     sum_partials<3>(part + (size_t)rhs * NPART * 4, nb, tot);
     if (threadIdx.x != 0) return;
-    double rn = sqrt(tot[0]);
-    double th1 = rn / S.tau, c = 1.0 / sqrt(1.0 + th1 * th1);
-    S.c2t2 = c * c * S.theta * S.theta;
-    S.c2a_re = c * c * S.alpha_re;
-    S.c2a_im = c * c * S.alpha_im;
-    S.tau = S.tau * th1 * c;
-    c64 rho1 = mk<double>(tot[1], tot[2]);
-    if (S.rho_re == 0.0 && S.rho_im == 0.0) { S.beta_re = S.beta_im = 0; S.breakdown = 1; S.conv = 1; }
-    else {
-        c64 b = cdiv(rho1, mk<double>(S.rho_re, S.rho_im));
-        S.beta_re = b.re;
-        S.beta_im = b.im;
-    }
-    S.rho_re = rho1.re;
-    S.rho_im = rho1.im;
-    S.theta = th1;
-    S.rnorm2 = tot[0];
-    S.it += 1;
-    if (S.tau <= S.target || S.it >= S.itmax || rn == 0.0) S.conv = 1;
+    sqmr_advance(S, tot);
 }
 
 // d = c²θ² d + c²α q;  z += d;  q = r + β q
@@ -2158,6 +2089,7 @@ int op_set_tile_impl(mfd_op *op, int prec, int ty, int kz, int xcd) {
     t[0] = ty;
     t[1] = kz;
     t[2] = xcd;
+    op->tile_set = 1;
     op->ws.release();
     return MFD_OK;
 }
@@ -2182,6 +2114,41 @@ static void trace_progress(const Scal *scal_h, int64_t nrhs, long long done_it, 
     fprintf(stderr, "[mfd step] it %lld recurrence tau/cn %.3e\n", it, worst);
 }
 
+// steps of one resident launch: whole chunks, up to 512, to the next multiple of
+// 512 steps (the FP32 probes, the trace) and to the step `upto` if given
+static int resident_span(int chunk, long long done_it, long long upto) {
+    const long long probe = std::max<long long>(chunk, 512) / chunk * chunk;
+    long long n = probe - done_it % probe;
+    if (upto > done_it) n = std::min(n, upto - done_it);
+    return (int)((n + chunk - 1) / chunk * chunk);
+}
+
+// the workspace's graph of `chunk` SQMR steps, captured when it holds another
+template <typename R>
+static int chunk_graph(mfd_op *op, int64_t nrhs, int chunk) {
+    Workspace &w = op->ws;
+    const int kind = sizeof(R) == 4 ? 1 : 3;
+    if (w.graph_iters == chunk && w.graph_kind == kind) return MFD_OK;
+    if (w.graph) { hipGraphExecDestroy(w.graph); w.graph = nullptr; }
+    w.graph_iters = 0;
+    hipGraph_t gr;
+    MFD_HIP(hipStreamBeginCapture(op->stream, hipStreamCaptureModeThreadLocal));
+    for (int it = 0; it < chunk; ++it) launch_iter<R>(op, nrhs);
+    MFD_HIP(hipStreamEndCapture(op->stream, &gr));
+    const hipError_t e = hipGraphInstantiate(&w.graph, gr, nullptr, nullptr, 0);
+    hipGraphDestroy(gr);
+    MFD_HIP(e);
+    w.graph_iters = chunk;
+    w.graph_kind = kind;
+    return MFD_OK;
+}
+
+static int resident_check(const Scal *scal_h, int64_t nrhs) {
+    for (int64_t r = 0; r < nrhs; ++r)
+        if (scal_h[r].stag == RESIDENT_TIMEOUT) { set_error("resident solver: blocks of one launch did not meet"); return MFD_ERR_HIP; }
+    return MFD_OK;
+}
+
 // stalled (optional): set when an FP32 cycle ended because its probes stopped
 // improving, rather than at its target or budget
 template <typename R>
@@ -2201,18 +2168,8 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     MFD_HIP(hipGetLastError());
     int chunk = o->check_every > 0 ? o->check_every : 32;
     bool use_graph = o->use_graph != 0;
-    const int kind = sizeof(R) == 4 ? 1 : 3;
-    if (use_graph && (w.graph_iters != chunk || w.graph_kind != kind)) {
-        if (w.graph) { hipGraphExecDestroy(w.graph); w.graph = nullptr; }
-        hipGraph_t gr;
-        MFD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (int it = 0; it < chunk; ++it) launch_iter<R>(op, nrhs);
-        MFD_HIP(hipStreamEndCapture(s, &gr));
-        MFD_HIP(hipGraphInstantiate(&w.graph, gr, nullptr, nullptr, 0));
-        hipGraphDestroy(gr);
-        w.graph_iters = chunk;
-        w.graph_kind = kind;
-    }
+    const bool res = resident_ok<R>(op, nrhs);
+    if (use_graph && !res) MFD_TRY(chunk_graph<R>(op, nrhs, chunk));
     long long done_it = 0;
     // FP32 cycles probe the true FP64 residual every `probe` steps and end after
     // two probes in a row that fail to halve it
@@ -2228,15 +2185,31 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     // soon as it is ≤ 0.9 tol for every RHS (the outer loop recomputes it the
     // same way).  A probe costs about one step.
     const long long probe64 = std::max<long long>(chunk, 256) / chunk * chunk;
-    long long next64 = 0;
+    long long next64 = 0, it_seen = 0;
     while (true) {
-        if (use_graph) MFD_HIP(hipGraphLaunch(w.graph, s));
+        int steps = chunk;
+        if (res) {
+            // one right-hand side: several chunks per launch, up to the next
+            // point at which this loop would do more than go on
+            double near = 0;
+            if (nrhs == 1) {
+                const bool p64 = sizeof(R) == 8 && b && e && tol > 0 && cyc_res > 0;
+                if (p64 && done_it >= next64) near = 3.0 * (tol / cyc_res);
+                steps = resident_span(chunk, done_it, p64 && done_it < next64 ? next64 : 0);
+            }
+            MFD_TRY(resident_steps<R>(op, nrhs, steps, chunk, near));
+        } else if (use_graph) MFD_HIP(hipGraphLaunch(w.graph, s));
         else
             for (int it = 0; it < chunk; ++it) launch_iter<R>(op, nrhs);
         MFD_HIP(hipGetLastError());
         MFD_HIP(hipMemcpyAsync(w.scal_h, w.scal, sizeof(Scal) * nrhs, hipMemcpyDeviceToHost, s));
         MFD_HIP(hipStreamSynchronize(s));
-        done_it += chunk;
+        if (res) {
+            MFD_TRY(resident_check(w.scal_h, nrhs));
+            if (nrhs == 1 && !w.scal_h[0].conv) steps = (int)(w.scal_h[0].it - it_seen);   // it may have stopped early
+            it_seen = w.scal_h[0].it;
+        }
+        done_it += steps;
         bool all = true;
         long long mx = 0;
         for (int64_t r = 0; r < nrhs; ++r) {
@@ -2362,10 +2335,7 @@ __global__ __launch_bounds__(BS) void k_bi_fin1(const double *part, int nb, Scal
     double tot[2];
     sum_partials<2>(part + (size_t)rhs * NPART * 4, nb, tot);
     if (threadIdx.x != 0) return;
-    if (tot[0] == 0.0 && tot[1] == 0.0) { S.breakdown = 1; S.conv = 1; S.alpha_re = S.alpha_im = 0; return; }
-    c64 a = cdiv(mk<double>(S.rho_re, S.rho_im), mk<double>(tot[0], tot[1]));
-    S.alpha_re = a.re;
-    S.alpha_im = a.im;
+    bi_alpha(S, tot);
 }
 
 // s = r − α v
@@ -2426,21 +2396,7 @@ __global__ __launch_bounds__(BS) void k_bi_fin3(const double *part, int nb, Scal
     double tot[3];
     sum_partials<3>(part + (size_t)rhs * NPART * 4, nb, tot);
     if (threadIdx.x != 0) return;
-    c64 rho1 = mk<double>(tot[0], tot[1]), om = mk<double>(S.om_re, S.om_im);
-    S.tau = sqrt(tot[2]);
-    S.it += 1;
-    if ((S.rho_re == 0.0 && S.rho_im == 0.0) || (om.re == 0.0 && om.im == 0.0)) {
-        S.breakdown = 1;
-        S.conv = 1;
-        S.beta_re = S.beta_im = 0;
-    } else {
-        c64 b = cdiv(rho1, mk<double>(S.rho_re, S.rho_im)) * cdiv(mk<double>(S.alpha_re, S.alpha_im), om);
-        S.beta_re = b.re;
-        S.beta_im = b.im;
-    }
-    S.rho_re = rho1.re;
-    S.rho_im = rho1.im;
-    if (S.tau <= S.target || S.it >= S.itmax || S.tau == 0.0) S.conv = 1;
+    bi_advance(S, tot);
 }
 
 // p = r + β (p − ω v)
@@ -2761,15 +2717,21 @@ struct BatchProb {
     double best = HUGE_VAL;    // smallest FP64 residual at a cycle start (iterate kept in ebest)
     int stall = 0;
     long long it_total = 0, it32 = 0, cycles = 0, next_probe = 0, next64 = 0;
+    long long it_seen = 0;     // steps of the cycle at the last readback
     bool conv = false, done = false, stalled32 = false;   // stalled32: an FP32 cycle stagnated
+    bool res() const { return prec == MFD_MIXED ? resident_ok<float>(op, 1) : resident_ok<double>(op, 1); }
 };
 }  // namespace
 
 // Independent problems (own grid, ε, ω; one RHS each) solved in lockstep: each
-// chunk of SQMR iterations of every live problem is one hipGraph launch whose
-// per-problem branches run on separate streams; between chunks the host reads
-// all solver scalars in one copy and runs the FP64 refinement step of each
+// round queues a chunk of SQMR iterations of every live problem, resident
+// where the problem fits the chip and as its own chunk graph (kept in its
+// workspace from call to call) otherwise; between rounds the host reads all
+// solver scalars in one copy and runs the FP64 refinement step of each
 // problem whose inner cycle ended (same rules as solve_dev_impl's SQMR path).
+// One graph with a branch and a stream per problem was captured and
+// instantiated on every call, and its branches did not overlap: eight
+// problems of 20³ to 64³ took 312 µs per step, the sum of their own steps.
 int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, void *const *e,
                          const mfd_solve_opts *oin, mfd_solve_stats *st) {
     if (count < 1 || count > 1024 || !ops || !b || !e) { set_error("count must be in [1, 1024] with non-null arrays"); return MFD_ERR_ARG; }
@@ -2793,22 +2755,13 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
         P[p].prec = prec0;
         MFD_TRY(ws_ensure(ops[p], 1, prec0));
     }
-    const int nstreams = std::min(count, 32);
-    std::vector<hipStream_t> streams(nstreams, nullptr);
-    std::vector<hipEvent_t> joins(nstreams, nullptr);
-    hipEvent_t fork = nullptr, tev0 = nullptr, tev1 = nullptr;
+    hipEvent_t tev0 = nullptr, tev1 = nullptr;
     Scal **src_d = nullptr;
     Scal *all_d = nullptr, *all_h = nullptr;
-    hipGraphExec_t gexec = nullptr;
     int rc = MFD_OK;
     auto fail = [&](hipError_t err) { set_error(hipGetErrorString(err)); rc = MFD_ERR_HIP; };
 #define BCHK(x) do { hipError_t err_ = (x); if (err_ != hipSuccess) { fail(err_); goto cleanup; } } while (0)
     {
-        for (int i = 0; i < nstreams; ++i) {
-            BCHK(hipStreamCreateWithFlags(&streams[i], hipStreamNonBlocking));
-            BCHK(hipEventCreateWithFlags(&joins[i], hipEventDisableTiming));
-        }
-        BCHK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
         BCHK(hipEventCreate(&tev0));
         BCHK(hipEventCreate(&tev1));
         BCHK(hipMalloc(&src_d, sizeof(Scal *) * count));
@@ -2892,6 +2845,7 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
             B.stall = 0;
             B.next_probe = probe_every;
             B.next64 = 0;
+            B.it_seen = 0;
             return MFD_OK;
         };
         // end of an inner cycle: e += (Q T⁻¹) z in FP64
@@ -2907,57 +2861,36 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
             int r = start_cycle(P[p]);
             if (r) { rc = r; goto cleanup; }
         }
-        std::vector<int> cap_prec;   // precision each problem was captured with (-1: not in the graph)
-        int cap_live = 0;
         while (true) {
-            int live = 0;
-            bool recap = gexec == nullptr;
+            bool live = false;
             for (int p = 0; p < count; ++p) {
-                if (P[p].done) continue;
-                ++live;
-                if (cap_prec.empty() || cap_prec[p] != P[p].prec) recap = true;
-            }
-            if (live == 0) break;
-            if (live < (3 * cap_live) / 4) recap = true;
-            if (recap) {
-                if (gexec) { hipGraphExecDestroy(gexec); gexec = nullptr; }
-                cap_prec.assign(count, -1);
-                hipGraph_t gr;
-                BCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                hipEventRecord(fork, s);
-                int k = 0;
-                for (int p = 0; p < count; ++p) {
-                    if (P[p].done) continue;
-                    hipStream_t sp = streams[k % nstreams];
-                    if (k < nstreams) hipStreamWaitEvent(sp, fork, 0);
-                    ++k;
-                    P[p].op->stream = sp;
-                    for (int it = 0; it < chunk; ++it) {
-                        if (P[p].prec == MFD_MIXED) launch_iter<float>(P[p].op, 1);
-                        else launch_iter<double>(P[p].op, 1);
+                BatchProb &B = P[p];
+                if (B.done) continue;
+                live = true;
+                int r;
+                if (B.res()) {   // as in run_inner: up to the next step at which the problem is looked at
+                    if (B.prec == MFD_MIXED) r = resident_steps<float>(B.op, 1, resident_span(chunk, B.it_seen, B.next_probe), chunk, 0);
+                    else {
+                        const bool look = !B.op->gd && B.it_seen >= B.next64;
+                        r = resident_steps<double>(B.op, 1, resident_span(chunk, B.it_seen, look ? 0 : B.next64), chunk,
+                                                   look ? 3.0 * o.tol / B.worst : 0.0);
                     }
-                    P[p].op->stream = s;
-                    cap_prec[p] = P[p].prec;
+                } else {
+                    r = B.prec == MFD_MIXED ? chunk_graph<float>(B.op, 1, chunk) : chunk_graph<double>(B.op, 1, chunk);
+                    if (!r) BCHK(hipGraphLaunch(B.op->ws.graph, s));
                 }
-                for (int i = 0; i < std::min(k, nstreams); ++i) {
-                    hipEventRecord(joins[i], streams[i]);
-                    hipStreamWaitEvent(s, joins[i], 0);
-                }
-                hipError_t ce = hipStreamEndCapture(s, &gr);
-                BCHK(ce);
-                ce = hipGraphInstantiate(&gexec, gr, nullptr, nullptr, 0);
-                hipGraphDestroy(gr);
-                BCHK(ce);
-                cap_live = live;
+                if (r) { rc = r; goto cleanup; }
             }
-            BCHK(hipGraphLaunch(gexec, s));
+            if (!live) break;
             k_gather_scal<<<(count + 63) / 64, 64, 0, s>>>(src_d, all_d, count);
             BCHK(hipMemcpyAsync(all_h, all_d, sizeof(Scal) * count, hipMemcpyDeviceToHost, s));
             BCHK(hipStreamSynchronize(s));
             for (int p = 0; p < count; ++p) {
                 BatchProb &B = P[p];
-                if (B.done || cap_prec[p] != B.prec) continue;
+                if (B.done) continue;
                 const Scal &S = all_h[p];
+                if (int r = resident_check(&S, 1)) { rc = r; goto cleanup; }
+                B.it_seen = S.it;
                 bool end = S.conv != 0;
                 if (!end && B.prec == MFD_MIXED && S.it >= B.next_probe) {
                     // true FP64 residual of e + (Q T⁻¹) z: the FP32 cycle ends
@@ -2997,14 +2930,6 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
                     end_cycle(B, S.it);
                     int r = start_cycle(B);
                     if (r) { rc = r; goto cleanup; }
-                    if (B.done) {
-                        // the captured graph may still hold this problem's
-                        // branch: its kernels skip a problem marked done
-                        const int one = 1;
-                        BCHK(hipMemcpyAsync(B.op->ws.active, &one, sizeof(int), hipMemcpyHostToDevice, s));
-                        k_set_done<<<1, 64, 0, s>>>(B.op->ws.scal, B.op->ws.active, 1);
-                        BCHK(hipStreamSynchronize(s));   // the pageable `one`
-                    }
                 }
             }
         }
@@ -3028,14 +2953,7 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
     }
 cleanup:
 #undef BCHK
-    for (int p = 0; p < count; ++p) ops[p]->stream = s;
     hipStreamSynchronize(s);
-    if (gexec) hipGraphExecDestroy(gexec);
-    for (int i = 0; i < nstreams; ++i) {
-        if (streams[i]) hipStreamDestroy(streams[i]);
-        if (joins[i]) hipEventDestroy(joins[i]);
-    }
-    if (fork) hipEventDestroy(fork);
     if (tev0) hipEventDestroy(tev0);
     if (tev1) hipEventDestroy(tev1);
     if (src_d) hipFree(src_d);

@@ -66,7 +66,7 @@ void ws_carve(Workspace &w, void *base, int64_t n, int64_t nrhs);
 
 struct mfd_op {
     mfd_ctx *ctx;
-    hipStream_t stream = nullptr;   // the context's stream; a batched solve re-points it while capturing
+    hipStream_t stream = nullptr;   // the context's stream
     mfd::DevGrid G;
     mfd::c64 omega;
     int full = 0, has_mu = 0;
@@ -80,6 +80,7 @@ struct mfd_op {
     // selects the direct kernel
     int tile64[3] = {4, 16, 1};
     int tile32[3] = {4, 16, 1};
+    int tile_set = 0;         // the caller fixed the tile shape: the marching stencil runs with it
     int sym = 1;              // complex-symmetric up to S_E (no complex Bloch phase)
     int gd = 0;               // grad-div augmented inner operator in use
     int gd_ok = 0;            // eligible (diagonal ε, μ = 1)
