@@ -1,0 +1,21 @@
+// Launches of the operator's stencils and of the sparse product.
+#pragma once
+#include "krylov_dev.hpp"
+
+namespace mfd {
+
+// launch one operator apply; returns the number of partial sums per RHS its
+// reduction wrote (finish = false leaves them to the next kernel)
+template <typename R, int MODE, int EPI>
+int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrhs, double *part, Scal *scal, double *rn,
+                 const int *mask = nullptr, hipEvent_t after_main = nullptr, bool finish = true);
+// finish kernel of a stencil epilogue with a reduction (nb partials per RHS)
+template <int EPI>
+void launch_finish(hipStream_t s, int nb, int64_t nrhs, double *part, Scal *scal, double *rn, const int *mask);
+// COCG's fused stencil: p = r + β p_old formed while staging (stored in pn),
+// the deferred it += α_prev p_old, t = P p and the pᵀt partials
+template <typename R>
+void launch_cocg_stencil(mfd_op *op, dim3 grid, int ty, int kz, int nch, int xr, const cx<R> *po, cx<R> *t,
+                         const cx<R> *rr, cx<R> *pn, cx<R> *xi);
+
+}  // namespace mfd

@@ -1,0 +1,9 @@
+// P on FP64 vectors without a reduction (BiCGSTAB, timing).
+#include "stencil_impl.hpp"
+
+namespace mfd {
+#define MFD_APPLY(R, MODE, EPI)                                                                                      \
+    template int launch_apply<R, MODE, EPI>(mfd_op *, const cx<R> *, cx<R> *, const c64 *, int64_t, double *, Scal *, \
+                                            double *, const int *, hipEvent_t, bool)
+MFD_APPLY(double, MODE_P, EPI_STORE);
+}  // namespace mfd
