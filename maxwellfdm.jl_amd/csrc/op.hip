@@ -209,7 +209,7 @@ __global__ __launch_bounds__(BS) void k_upd_r_dot(cx<R> *__restrict__ rall, cons
             S.conv = 1;
             S.alpha_re = S.alpha_im = 0;
             S.apend_re = S.apend_im = 0;
-            // k_fin_r skips a converged RHS, so k_upd_dzq would otherwise
+            // k_fin_r skips a converged RHS, so the d, z updates would otherwise
             // apply the previous step's coefficients once more: d = 0, z kept
             S.c2t2 = 0;
             S.c2a_re = S.c2a_im = 0;
@@ -236,39 +236,99 @@ __global__ __launch_bounds__(BS) void k_upd_r_dot(cx<R> *__restrict__ rall, cons
     block_partial<3>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
 }
 
+// d and z updates put off: the coefficients of a step's d = c²θ² d + c²α q,
+// kept until the updates run (on = 0: the step moved nothing)
+struct DzCoef {
+    double c2t2, c2a_re, c2a_im;
+    int on, pad;
+};
+constexpr int DZ_MAX = 4;   // steps put off at most, this one included
+// a right-hand side's coefficients lie behind its partial sums of the r update
+__device__ inline DzCoef *dz_coef(double *part, int rhs) {
+    return (DzCoef *)(part + (size_t)rhs * NPART * 4 + 4 * NGRID_MAX);
+}
+static_assert(DZ_MAX * sizeof(DzCoef) <= (NPART - NGRID_MAX) * 4 * sizeof(double), "");
+
 // after k_upd_r_dot: ||r||, θ, c, τ, β, ρ of the SQMR step (one block per RHS)
-__global__ __launch_bounds__(BS) void k_fin_r(const double *part, int nb, Scal *scal) {
+// and the coefficients of its d, z updates
+__global__ __launch_bounds__(BS) void k_fin_r(double *part, int nb, Scal *scal, int slot) {
     const int rhs = blockIdx.x;
     Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
+    DzCoef &C = dz_coef(part, rhs)[slot];
+    if (S.done || S.conv) {
+        if (threadIdx.x == 0) C.on = 0;
+        return;
+    }
     double tot[3];
     sum_partials<3>(part + (size_t)rhs * NPART * 4, nb, tot);
     if (threadIdx.x != 0) return;
     sqmr_advance(S, tot);
+    C = DzCoef{S.c2t2, S.c2a_re, S.c2a_im, 1, 0};
 }
 
-// d = c²θ² d + c²α q;  z += d;  q = r + β q
+// The end of an SQMR step: q' = r + β q and, with P > 0, the d, z updates of
+// the last P steps from their kept q, one step after the other:
+// d = c²θ² d + c²α q, z += d.  All of it is memory traffic, and d and z are
+// read by nothing until the host looks at z: put off over four steps a step
+// moves 4.75 vectors instead of 7.  Measured on 128³ (µs): 101 every step →
+// 41.2 with P = 0 and 140.7 with P = 4, 66 on average (7.3 TB/s of a
+// vector's 101 MB, part of it from the Infinity Cache); 640×522 cells 11.0 →
+// 7.8.  The scalars' finish stays a kernel of one block: done by every block
+// here it cost 13–15 µs (640×522: 20.5 µs with P = 0 against 5.5 + 4.5).
 // QNT: the new q is streamed too (the q vectors of all RHS exceed the cache,
 // so keeping them there only evicts other data)
-template <typename R, bool NT, bool QNT = false>
-__global__ __launch_bounds__(BS) void k_upd_dzq(cx<R> *__restrict__ dall, cx<R> *__restrict__ zall,
-                                                cx<R> *__restrict__ qall, const cx<R> *__restrict__ rall, int64_t n,
-                                                int64_t vs, const Scal *scal) {
+template <typename R>
+struct QArgs {
+    const cx<R> *q[DZ_MAX];   // q of the steps not yet applied, oldest first (P = 0: only this step's)
+    cx<R> *qn;                // the new q (may be q[0])
+    cx<R> *d, *z;
+    const cx<R> *r;
+    int64_t n;
+    double *part;             // the r update's partials, before the coefficients
+    const Scal *scal;
+    int slot;                 // of this step
+};
+template <typename R, bool NT, bool QNT, int P>
+__global__ __launch_bounds__(BS) void k_upd_q(QArgs<R> A) {
+    constexpr int NQ = P > 0 ? P : 1;
     const int rhs = blockIdx.y;
-    const Scal &S = scal[rhs];
-    if (S.done) return;
-    cx<R> *d = dall + rhs * vs, *z = zall + rhs * vs, *q = qall + rhs * vs;
-    const cx<R> *r = rall + rhs * vs;
-    double c2t2 = S.c2t2;
-    c64 c2a = mk<double>(S.c2a_re, S.c2a_im), be = mk<double>(S.beta_re, S.beta_im);
-    for (int64_t e = blockIdx.x * (int64_t)BS + threadIdx.x; e < n; e += (int64_t)gridDim.x * BS) {
-        c64 qe = cvt<double>(vld<NT>(&q[e]));
-        c64 de = c2t2 * cvt<double>(vld<NT>(&d[e])) + c2a * qe;
-        vst<NT>(&d[e], cvt<R>(de));
-        vst<NT>(&z[e], cvt<R>(cvt<double>(vld<NT>(&z[e])) + de));
-        const cx<R> qn = cvt<R>(cvt<double>(vld<NT>(&r[e])) + be * qe);   // read next by the stencil
-        if (QNT) vst<true>(&q[e], qn);
-        else q[e] = qn;
+    const Scal &S = A.scal[rhs];
+    const DzCoef *coef = dz_coef(A.part, rhs) + (P > 0 ? 0 : A.slot);
+    DzCoef c[NQ];
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+        c[k] = coef[k];
+        any = any || c[k].on;
+    }
+    if (!any) return;   // a finished right-hand side: nothing moves
+    const c64 be = mk<double>(S.beta_re, S.beta_im);
+    const int64_t off = (int64_t)rhs * A.n;
+    const cx<R> *r = A.r + off;
+    cx<R> *qn = A.qn + off, *d = A.d + off, *z = A.z + off;
+    const cx<R> *q[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) q[k] = A.q[k] + off;
+    const int64_t step = (int64_t)gridDim.x * BS;
+    for (int64_t e = blockIdx.x * (int64_t)BS + threadIdx.x; e < A.n; e += step) {
+        cx<R> qv[NQ], dv, zv;
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) qv[k] = vld<NT>(&q[k][e]);
+        const cx<R> rv = vld<NT>(&r[e]);
+        if (P > 0) {
+            dv = vld<NT>(&d[e]);
+            zv = vld<NT>(&z[e]);
+#pragma unroll
+            for (int k = 0; k < P; ++k)
+                if (c[k].on) {
+                    const c64 de = c[k].c2t2 * cvt<double>(dv) + mk<double>(c[k].c2a_re, c[k].c2a_im) * cvt<double>(qv[k]);
+                    dv = cvt<R>(de);
+                    zv = cvt<R>(cvt<double>(zv) + de);
+                }
+            vst<NT>(&d[e], dv);
+            vst<NT>(&z[e], zv);
+        }
+        vst<QNT>(&qn[e], cvt<R>(cvt<double>(rv) + be * cvt<double>(qv[NQ - 1])));   // read next by the stencil
     }
 }
 
@@ -642,17 +702,6 @@ static int ws_ensure(mfd_op *op, int64_t nrhs, int prec) {
     return MFD_OK;
 }
 
-template <typename R>
-static void launch_upd_dzq(dim3 gv, hipStream_t s, cx<R> *d, cx<R> *z, cx<R> *q, const cx<R> *r, int64_t n,
-                           const Scal *scal, bool nt) {
-    // the new q of every RHS fits the 256 MB Infinity Cache: keep it there for
-    // the next stencil; otherwise stream it as well
-    const bool qnt = nt && (double)n * gv.y * sizeof(cx<R>) > 256.0 * 1024 * 1024;
-    if (qnt) k_upd_dzq<R, true, true><<<gv, BS, 0, s>>>(d, z, q, r, n, n, scal);
-    else if (nt) k_upd_dzq<R, true><<<gv, BS, 0, s>>>(d, z, q, r, n, n, scal);
-    else k_upd_dzq<R, false><<<gv, BS, 0, s>>>(d, z, q, r, n, n, scal);
-}
-
 // Whether one SQMR step's vectors (r, q, t, d, z of every RHS) and the
 // stencil's operator data (qs) exceed the Infinity Cache (256 MB on MI355X):
 // then the vector updates stream non-temporally (measured on 128³ FP64: step
@@ -663,32 +712,77 @@ static bool stream_nt(int64_t n, int64_t nrhs, size_t vbytes) {
     return foot > 256.0 * 1024 * 1024;
 }
 
-// One SQMR step: stencil t = P q with qᵀt partials, r update (with the α
-// finish folded in), finish of ||r||, rᵀr, d/z/q update.  E (optional): six
-// events around the main kernels, for timing in context.
+// The grid of an SQMR step's vector kernels: about two blocks per CU over all
+// right-hand sides, so that every RHS streams at once (with a full grid per RHS
+// the launch ran as nrhs successive rounds, 24% slower per RHS at 4 RHS) and
+// the r update's blocks, which all sum the stencil's partials, are few.
+// 2,048 → 512 blocks: the r update on 128³ 49.9 → 46.8 µs and on 640×522 cells
+// 11.0 → 9.2 µs, the q, d, z update on 128³ 147.9 → 140.7 µs.
+static dim3 grid_rhs(int64_t n, int64_t nrhs) {
+    const int64_t full = ngrid(n);
+    return dim3((unsigned)std::min(full, std::max(512 / nrhs, std::min<int64_t>(full, 64))), (unsigned)nrhs);
+}
+
+// `steps` SQMR steps, step by step: stencil t = P q with qᵀt partials, r update
+// (with the α finish folded in), the scalars' finish, then q and, every DZ_MAX
+// steps and at the end, the d and z updates of the steps since.  Between calls
+// the state is that of whole steps (w.q, w.d, w.z, w.scal).  Inside, q moves
+// through w.q, w.et2, w.et and w.r64 (the probe and residual vectors, free
+// inside a cycle).  E (optional): six events per step around the kernels, for
+// timing in context.
 template <typename R>
-static void launch_iter(mfd_op *op, int64_t nrhs, hipEvent_t *E = nullptr) {
+static void launch_steps(mfd_op *op, int64_t nrhs, int steps, hipEvent_t *E = nullptr) {
     Workspace &w = op->ws;
-    int64_t n = w.n;
+    const int64_t n = w.n;
     hipStream_t s = op->stream;
-    // about one resident round of blocks in total: every RHS streams at once
-    // (with ngrid(n) blocks per RHS the launch ran as nrhs successive rounds,
-    // measured 24% slower per RHS for the FP64 d/z/q update at 4 RHS)
-    const unsigned gx = std::max<unsigned>(ngrid(n) / (unsigned)nrhs, std::min<unsigned>(ngrid(n), 64u));
-    dim3 gv(gx, (unsigned)nrhs);
-    size_t pslot = (size_t)nrhs * NPART * 4;
+    double *rpart = w.part + (size_t)nrhs * NPART * 4;
     const bool nt = stream_nt(n, nrhs, sizeof(cx<R>));
-    if (E) hipEventRecord(E[0], s);
-    const int nbd = launch_apply<R, MODE_P, EPI_DOT>(op, (const cx<R> *)w.q, (cx<R> *)w.t, nullptr, nrhs, w.part,
-                                                     w.scal, nullptr, nullptr, E ? E[1] : nullptr, false);
-    if (E) hipEventRecord(E[2], s);
-    if (nt) k_upd_r_dot<R, true><<<gv, BS, 0, s>>>((cx<R> *)w.r, (const cx<R> *)w.t, n, n, w.part, nbd, w.part + pslot, w.scal);
-    else k_upd_r_dot<R, false><<<gv, BS, 0, s>>>((cx<R> *)w.r, (const cx<R> *)w.t, n, n, w.part, nbd, w.part + pslot, w.scal);
-    if (E) hipEventRecord(E[3], s);
-    k_fin_r<<<(unsigned)nrhs, BS, 0, s>>>(w.part + pslot, (int)gv.x, w.scal);
-    if (E) hipEventRecord(E[4], s);
-    launch_upd_dzq<R>(gv, s, (cx<R> *)w.d, (cx<R> *)w.z, (cx<R> *)w.q, (const cx<R> *)w.r, n, w.scal, nt);
-    if (E) hipEventRecord(E[5], s);
+    // the new q of every RHS fits the 256 MB Infinity Cache: it stays there for
+    // the next stencil; otherwise it is streamed as well
+    const bool qnt = nt && (double)n * nrhs * sizeof(cx<R>) > 256.0 * 1024 * 1024;
+    const dim3 gv = grid_rhs(n, nrhs);
+    cx<R> *ring[DZ_MAX] = {(cx<R> *)w.q, (cx<R> *)w.et2, (cx<R> *)w.et, (cx<R> *)w.r64};
+    QArgs<R> A;
+    A.d = (cx<R> *)w.d;
+    A.z = (cx<R> *)w.z;
+    A.r = (const cx<R> *)w.r;
+    A.n = n;
+    A.part = rpart;
+    A.scal = w.scal;
+    int slot = 0;   // steps not yet applied to d and z before this one
+    for (int it = 0; it < steps; ++it, E = E ? E + 6 : nullptr) {
+        const cx<R> *q = ring[slot];
+        if (E) hipEventRecord(E[0], s);
+        const int nbd = launch_apply<R, MODE_P, EPI_DOT>(op, q, (cx<R> *)w.t, nullptr, nrhs, w.part, w.scal, nullptr,
+                                                         nullptr, E ? E[1] : nullptr, false);
+        if (E) hipEventRecord(E[2], s);
+        if (nt) k_upd_r_dot<R, true><<<gv, BS, 0, s>>>((cx<R> *)w.r, (const cx<R> *)w.t, n, n, w.part, nbd, rpart, w.scal);
+        else k_upd_r_dot<R, false><<<gv, BS, 0, s>>>((cx<R> *)w.r, (const cx<R> *)w.t, n, n, w.part, nbd, rpart, w.scal);
+        if (E) hipEventRecord(E[3], s);
+        k_fin_r<<<(unsigned)nrhs, BS, 0, s>>>(rpart, (int)gv.x, w.scal, slot);
+        if (E) hipEventRecord(E[4], s);
+        const bool flush = it + 1 == steps || slot + 1 == DZ_MAX;
+        A.slot = slot;
+        for (int k = 0; k <= slot; ++k) A.q[k] = ring[k];
+        if (!flush) A.q[0] = q;
+        A.qn = flush ? ring[0] : ring[slot + 1];
+#define MFD_UPD_Q(P)                                                        \
+    do {                                                                    \
+        if (qnt) k_upd_q<R, true, true, P><<<gv, BS, 0, s>>>(A);            \
+        else if (nt) k_upd_q<R, true, false, P><<<gv, BS, 0, s>>>(A);       \
+        else k_upd_q<R, false, false, P><<<gv, BS, 0, s>>>(A);              \
+    } while (0)
+        switch (flush ? slot + 1 : 0) {
+        case 0: MFD_UPD_Q(0); break;
+        case 1: MFD_UPD_Q(1); break;
+        case 2: MFD_UPD_Q(2); break;
+        case 3: MFD_UPD_Q(3); break;
+        default: MFD_UPD_Q(4); break;
+        }
+#undef MFD_UPD_Q
+        if (E) hipEventRecord(E[5], s);
+        slot = flush ? 0 : slot + 1;
+    }
 }
 
 }  // namespace mfd
@@ -1115,14 +1209,14 @@ int op_bench_iteration_impl(mfd_op *op, int64_t nrhs, int prec, int iters, doubl
     int rc = MFD_OK;
     for (auto &e : ev)
         if (hipEventCreate(&e) != hipSuccess) { rc = MFD_ERR_HIP; break; }
-    auto iteration = [&](hipEvent_t *E) {
-        if (prec == MFD_FP64) launch_iter<double>(op, nrhs, E);
-        else launch_iter<float>(op, nrhs, E);
+    auto run = [&](int steps, hipEvent_t *E) {
+        if (prec == MFD_FP64) launch_steps<double>(op, nrhs, steps, E);
+        else launch_steps<float>(op, nrhs, steps, E);
     };
     if (!rc) {
         k_bench_scal<<<(unsigned)((nrhs + 63) / 64), 64, 0, s>>>(w.scal, nrhs);
-        for (int k = 0; k < 3; ++k) iteration(nullptr);
-        for (int it = 0; it < iters; ++it) iteration(&ev[6 * (size_t)it]);
+        run(4, nullptr);
+        run(iters, ev.data());
         if (hipStreamSynchronize(s) != hipSuccess) rc = MFD_ERR_HIP;
     }
     if (!rc) {
@@ -1620,7 +1714,7 @@ static int chunk_graph(mfd_op *op, int64_t nrhs, int chunk) {
     w.graph_iters = 0;
     hipGraph_t gr;
     MFD_HIP(hipStreamBeginCapture(op->stream, hipStreamCaptureModeThreadLocal));
-    for (int it = 0; it < chunk; ++it) launch_iter<R>(op, nrhs);
+    launch_steps<R>(op, nrhs, chunk);
     MFD_HIP(hipStreamEndCapture(op->stream, &gr));
     const hipError_t e = hipGraphInstantiate(&w.graph, gr, nullptr, nullptr, 0);
     hipGraphDestroy(gr);
@@ -1686,8 +1780,7 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
             }
             MFD_TRY(resident_steps<R>(op, nrhs, steps, chunk, near));
         } else if (use_graph) MFD_HIP(hipGraphLaunch(w.graph, s));
-        else
-            for (int it = 0; it < chunk; ++it) launch_iter<R>(op, nrhs);
+        else launch_steps<R>(op, nrhs, chunk);
         MFD_HIP(hipGetLastError());
         MFD_HIP(hipMemcpyAsync(w.scal_h, w.scal, sizeof(Scal) * nrhs, hipMemcpyDeviceToHost, s));
         MFD_HIP(hipStreamSynchronize(s));
