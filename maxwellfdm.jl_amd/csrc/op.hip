@@ -619,6 +619,46 @@ void Workspace::release() {
     nrhs = 0;
 }
 
+// Rows and planes per tile.  The stencils hold two waves per SIMD (their
+// registers), so a CU runs two 4-row blocks or one 8-row block at a time, and
+// a launch takes as many rounds of them as the fullest CU has: with 64×4 tiles
+// of 16 planes 144×120×100 is 630 tiles, three on some CUs, where 20 planes
+// make it 450, two on each.  A block costs its planes and about two more (the
+// first plane's halo and the prologue); one 4-row block alone on a CU takes
+// 0.7 of the time of two (0.5 with μ ≠ 1, where 4-row blocks never share a
+// CU); 8-row blocks read fewer halo rows.  Measured on 14 grids of 52 to 203
+// cells an axis, FP64 and FP32, one and three right-hand sides, against the
+// fastest of 26 to 52 shapes: within 2.5%, where 4 × 16 with planes halved
+// while a launch had fewer than 256 tiles lost up to 20% (µs per step: full ε
+// 144×120×100 330.6 → 274.7, μ ≠ 1 80×76×70 96.2 → 80.0, boundft HEE 100×90×96
+// 127.1 → 107.5, 110×112×90 138.6 → 121.0, 56×58×52 41.7 → 37.8).  More than
+// 20 planes lose again (203×180×151: 24 planes 618 µs, 20 planes 593).
+Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs) {
+    const int *t = fp64 ? op->tile64 : op->tile32;
+    Tile best = {t[0], t[1], t[2]};
+    if (best.ty == 0 || op->tile_set[fp64 ? 0 : 1]) return best;
+    const int32_t *N = op->G.d64.N;
+    const bool narrow = (best.xr & 2) != 0;
+    const double alone = op->has_mu || op->gd ? 0.5 : 0.7;
+    double least = 1e300;
+    for (int ty = 8; ty >= 4; ty /= 2) {
+        if (ty == 8 && op->gd) continue;
+        const int rows = narrow ? 2 * ty : ty, per = 8 / ty;   // per: blocks of a CU at a time
+        const int64_t cols = (int64_t)((N[0] + (narrow ? 31 : 63)) / (narrow ? 32 : 64)) * ((N[1] + rows - 1) / rows);
+        for (int kz = 1; kz <= std::min<int>(N[2], 20); ++kz) {
+            const int64_t most = (cols * ((N[2] + kz - 1) / kz) * nrhs + 255) / 256;
+            const double rounds = (double)(most / per) + (most % per ? alone : 0.0);
+            const double cost = rounds * (kz + 2) * (ty == 8 ? 0.97 : 1.0);
+            if (cost < least) {
+                least = cost;
+                best.ty = ty;
+                best.kz = kz;
+            }
+        }
+    }
+    return best;
+}
+
 // scratch of the two-pass direct kernel for nrhs right-hand sides (operators
 // the tiled stencils do not serve); allocated outside any graph capture
 static int hbuf_ensure(mfd_op *op, int64_t nrhs) {
@@ -887,26 +927,10 @@ int op_create_impl(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const
     op->gd_ok = !full && !op->has_mu && op->ee_all && !(om2.re == 0.0 && om2.im == 0.0);
     if (!op->ee_all && !op->rev) op->tile64[0] = op->tile32[0] = 0;   // the direct kernel serves mixed boundaries
     else {
-        // default tile (until mfd_op_autotune or mfd_op_set_tile): 4 rows x 16
-        // planes, with fewer planes and then fewer rows per block on grids too
-        // small for that to give one tile per CU (256); 32-wide tiles (of
-        // twice the rows) where they leave fewer x lanes idle than 64-wide ones
+        // 32-wide tiles (of twice the rows) where they leave fewer x lanes idle
+        // than 64-wide ones; rows and planes are chosen at each launch
         const int64_t N0 = op->G.h.N[0];
         const bool narrow = !full && !op->has_mu && !op->rev && 64 * ((N0 + 63) / 64) - N0 > 32 * ((N0 + 31) / 32) - N0;
-        const int64_t nx = narrow ? (N0 + 31) / 32 : (N0 + 63) / 64;
-        auto tiles = [&](int ty, int kz) {
-            const int rows = narrow ? 2 * ty : ty;
-            return nx * ((op->G.h.N[1] + rows - 1) / rows) * ((op->G.h.N[2] + kz - 1) / kz);
-        };
-        int ty = 4, kz = 16;
-        while (kz > 4 && tiles(ty, kz) < 256) kz /= 2;
-        while (ty > 1 && tiles(ty, kz) < 256) ty /= 2;
-        // a one-cell z axis with full ε (the smoothed 2D models): each tile
-        // marches a single plane, and the 8-row tile is the faster one
-        // wherever it still gives a tile per CU (2D TE 1024²: 8.67 → 8.31 s)
-        if (full && op->G.h.N[2] == 1 && ty == 4 && tiles(8, kz) >= 256) ty = 8;
-        op->tile64[0] = op->tile32[0] = ty;
-        op->tile64[1] = op->tile32[1] = kz;
         op->tile64[2] = op->tile32[2] = narrow ? 3 : 1;
     }
     op->gd = 0;   // opt-in: it helps small PML-dominated grids and slows larger ones
@@ -1261,24 +1285,26 @@ int op_autotune_impl(mfd_op *op, int64_t nrhs, int iters, int *best64, int *best
     double bestms[2] = {1e30, 1e30};
     int bt[2][3] = {{4, 16, 1}, {4, 16, 1}};
     const int its = std::max(2, std::min(iters, 50));
-    for (int prec = 0; prec < 2; ++prec)
-        for (int a = 0; a < 4; ++a)
-            for (int b = 0; b < 4; ++b)
+    for (int prec = 0; prec < 2; ++prec) {
+        int *tile = prec == 0 ? op->tile64 : op->tile32;
+        op->tile_set[prec] = 0;
+        const Tile rule = stencil_tile(op, prec == 0, nrhs);   // a candidate as well
+        op->tile_set[prec] = 2;
+        for (int a = -1; a < 4; ++a)
+            for (int b = 0; b < (a < 0 ? 1 : 4); ++b)
                 for (int xo = 0; xo < norders; ++xo) {
-                    int *tile = prec == 0 ? op->tile64 : op->tile32;
-                    tile[0] = tys[a];
-                    tile[1] = kzs[b];
+                    tile[0] = a < 0 ? rule.ty : tys[a];
+                    tile[1] = a < 0 ? rule.kz : kzs[b];
                     tile[2] = xo;
                     double part[3] = {0, 0, 0};
                     MFD_TRY(op_bench_iteration_impl(op, nrhs, prec == 0 ? MFD_FP64 : MFD_MIXED, its, part));
                     const double ms = part[0] + part[1] + part[2];
                     if (ms < bestms[prec]) {
                         bestms[prec] = ms;
-                        bt[prec][0] = tys[a];
-                        bt[prec][1] = kzs[b];
-                        bt[prec][2] = xo;
+                        for (int k = 0; k < 3; ++k) bt[prec][k] = tile[k];
                     }
                 }
+    }
     for (int k = 0; k < 3; ++k) {
         op->tile64[k] = bt[0][k];
         op->tile32[k] = bt[1][k];
@@ -1460,11 +1486,11 @@ static void launch_cocg_iter(mfd_op *op, int64_t nrhs, int par) {
     size_t pslot = (size_t)nrhs * NPART * 4;
     cx<R> *po = cocg_p<R>(w, par), *pn = cocg_p<R>(w, par ^ 1);
     const DGrid<R> &g = op->G.view<R>();
-    int ty = std::is_same<R, double>::value ? op->tile64[0] : op->tile32[0];
+    // the fused COCG stencil is built 64-wide only: the narrow-tile bit is ignored
+    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
+    const int ty = tile.ty, xr = tile.xr & 1;
     if (!op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win && ty > 0) {
-        int kz = std::is_same<R, double>::value ? op->tile64[1] : op->tile32[1];
-        // the fused COCG stencil is built 64-wide only: the narrow-tile bit is ignored
-        int xr = (std::is_same<R, double>::value ? op->tile64[2] : op->tile32[2]) & 1;
+        int kz = tile.kz;
         int nx = (g.N[0] + 63) / 64, ny = (g.N[1] + ty - 1) / ty, nch = (g.N[2] + kz - 1) / kz;
         while ((int64_t)nx * ny * nch > NPART) { kz *= 2; nch = (g.N[2] + kz - 1) / kz; }
         dim3 grid(nx, ny, (unsigned)(nch * nrhs));
@@ -1670,7 +1696,7 @@ int op_set_tile_impl(mfd_op *op, int prec, int ty, int kz, int xcd) {
     t[0] = ty;
     t[1] = kz;
     t[2] = xcd;
-    op->tile_set = 1;
+    op->tile_set[prec == MFD_FP64 ? 0 : 1] = 1;
     op->ws.release();
     return MFD_OK;
 }

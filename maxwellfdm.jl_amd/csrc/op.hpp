@@ -80,7 +80,10 @@ struct mfd_op {
     // selects the direct kernel
     int tile64[3] = {4, 16, 1};
     int tile32[3] = {4, 16, 1};
-    int tile_set = 0;         // the caller fixed the tile shape: the marching stencil runs with it
+    // per precision (FP64, FP32): 0 = shape chosen at each launch (stencil_tile),
+    // 1 = fixed by the caller, whose solves then march through the tiles even
+    // where the resident kernel would serve, 2 = fixed by the autotuner
+    int tile_set[2] = {0, 0};
     int sym = 1;              // complex-symmetric up to S_E (no complex Bloch phase)
     int gd = 0;               // grad-div augmented inner operator in use
     int gd_ok = 0;            // eligible (diagonal ε, μ = 1)

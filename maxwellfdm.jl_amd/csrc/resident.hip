@@ -760,7 +760,7 @@ static int res_xch(const Workspace &w, const ResPlan &P, int64_t n, int64_t nrhs
 
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs) {
-    if (op->tile_set || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
+    if (op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
     if (op->G.d64.M > (1 << 22)) return false;   // 32-bit byte offsets (and far above any capacity)
     const ResPlan P = res_plan<R>(op);
     return P.nb <= P.cap && res_xch<R>(op->ws, P, op->n, nrhs) != 0;

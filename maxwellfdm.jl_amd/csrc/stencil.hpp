@@ -4,6 +4,12 @@
 
 namespace mfd {
 
+// the tile shape of a stencil launch over nrhs right-hand sides
+struct Tile {
+    int ty, kz, xr;   // rows, planes, order (bit 0: XCD runs, bit 1: 32-wide); ty = 0: the direct kernel
+};
+Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs);
+
 // launch one operator apply; returns the number of partial sums per RHS its
 // reduction wrote (finish = false leaves them to the next kernel)
 template <typename R, int MODE, int EPI>

@@ -266,16 +266,12 @@ void launch_finish(hipStream_t s, int nb, int64_t nrhs, double *part, Scal *scal
 // launch one operator apply; returns the number of partial sums per RHS its
 // reduction wrote (finish = false leaves them to the next kernel)
 template <typename R, int MODE, int EPI>
-int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrhs, double *part,
-                        Scal *scal, double *rn, const int *mask, hipEvent_t after_main,
-                 bool finish) {
+int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrhs, double *part, Scal *scal, double *rn,
+                 const int *mask, hipEvent_t after_main, bool finish) {
     const DGrid<R> &g = op->G.view<R>();
     const OpData<R> &od = opd<R>(op);
     int64_t vs = op->n;
     hipStream_t s = op->stream;
-    int ty = std::is_same<R, double>::value ? op->tile64[0] : op->tile32[0];
-    int kz = std::is_same<R, double>::value ? op->tile64[1] : op->tile32[1];
-    int xr = std::is_same<R, double>::value ? op->tile64[2] : op->tile32[2];
     if (op->csr) {   // an operator built from a caller's CSC matrix
         dim3 grid(ngrid(vs), (unsigned)nrhs);
         k_spmv<R, MODE, EPI><<<grid, BS, 0, s>>>(vs, op->csr_rowptr, op->csr_colind, op->csr_val, op->d64.qs,
@@ -284,6 +280,8 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
         if (finish) launch_finish<EPI>(s, (int)grid.x, nrhs, part, scal, rn, mask);
         return (int)grid.x;
     }
+    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
+    int ty = tile.ty, kz = tile.kz, xr = tile.xr;
     if (MODE == MODE_P && op->gd && ty == 8) ty = 4;   // the grad-div tile keeps two more LDS planes
     // μ ≠ 1 has a tiled form with diagonal ε (the grad-div form is never on with μ)
     if ((op->ee_all || op->rev) && ty > 0 && !(op->has_mu && op->full)) {

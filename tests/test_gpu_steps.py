@@ -37,3 +37,20 @@ def test_deferred_updates(check_every, precision, pkg, O):
     assert st.converged and not e[1].any()
     for r in (0, 2):
         assert np.linalg.norm(b[r] - A @ e[r]) <= 1.01 * TOL * np.linalg.norm(b[r])
+
+
+@pytest.mark.parametrize("N", [(70, 37, 45), (64, 130, 31), (33, 9, 90), (150, 21, 1)])
+@pytest.mark.parametrize("scene", ["diag", "mu", "full"])
+def test_launch_tiles(N, scene, pkg):
+    """Tiles chosen at the launch (short last chunks, several right-hand sides)
+    against a fixed shape: each value is formed from the same terms in the same
+    order whatever the tile, so they agree to the last bits."""
+    m, rng = system(pkg, N, (False, False, N[2] == 1), (0, 0, 0), scene, 4)
+    x = rng.normal(size=(3, 3 * int(np.prod(N)))) + 1j * rng.normal(size=(3, 3 * int(np.prod(N))))
+    op = pkg.MaxwellOperator(m, OM)
+    say("tiles", N, scene)
+    y = [op.apply(x), op.apply(x[0])]
+    op.set_tile("fp64", 4, 16, 1)
+    z = op.apply(x)
+    op.close()
+    assert np.abs(y[0] - z).max() <= 1e-15 * np.abs(z).max() and np.abs(y[1] - z[0]).max() <= 1e-15 * np.abs(z).max()
