@@ -57,135 +57,163 @@ struct EList {
     }
 };
 
-// Column (w, p) of Cₑ (which = 0) or Cₘ (which = 1).  Row generation of a
-// curl row H_u(r) = ∂_v F_w − ∂_w F_v, v = u+1, w = u+2: diagonal term first,
-// then the neighbour term; a non-Bloch ghost is zero.
+// The entries of column (w, p) of Cₑ (which = 0) or Cₘ (which = 1) in the row
+// component u = w+1+t: at p itself (va) and, when there is a neighbour (return
+// true), at p's neighbour along the difference axis v (index qb on that axis,
+// cell pb, value vb).  Row generation of a curl row H_u(r) = ∂_v F_w − ∂_w F_v,
+// v = u+1, w = u+2; a non-Bloch ghost is zero.
+__device__ inline bool curl_pair(const DGrid<double> &g, int which, int w, int t, const int q[3], int64_t p, c64 &va,
+                                 int &qb, int64_t &pb, c64 &vb) {
+    const int v = t == 0 ? (w + 2) % 3 : (w + 1) % 3;
+    const double sg = t == 0 ? 1.0 : -1.0;
+    const bool isfwd = which == 0 ? (g.bft[v] == EE) : (g.bft[v] == HH);
+    const c64 *inv = g.sdlinv[g0type(g.bft, which == 0 ? HH : EE, v)][v];
+    const int Nv = g.N[v], i = q[v];
+    const int64_t st = stride3(g, v);
+    qb = i;
+    pb = p;
+    vb = mk<double>(0.0, 0.0);
+    if (isfwd) {
+        va = -(sg * inv[i]);
+        if (i > 0) {
+            qb = i - 1;
+            pb = p - st;
+            vb = sg * inv[i - 1];
+            return true;
+        }
+        if (!g.bloch[v]) return false;
+        const c64 val = (sg * inv[Nv - 1]) * g.ph[v];
+        if (Nv == 1) { va = va + val; return false; }
+        qb = Nv - 1;
+        pb = p + (int64_t)(Nv - 1) * st;
+        vb = val;
+        return true;
+    }
+    va = sg * inv[i];
+    if (i < Nv - 1) {
+        qb = i + 1;
+        pb = p + st;
+        vb = -(sg * inv[i + 1]);
+        return true;
+    }
+    if (!g.bloch[v]) return false;
+    const c64 val = (-(sg * inv[0])) * g.phinv[v];
+    if (Nv == 1) { va = va + val; return false; }
+    qb = 0;
+    pb = p - (int64_t)(Nv - 1) * st;
+    vb = val;
+    return true;
+}
+
+// column (w, p) of Cₑ (which = 0) or Cₘ (which = 1)
 __device__ void curl_col(const DGrid<double> &g, int which, int w, int64_t p, EList<4> &L) {
     int q[3];
     unc3(g, p, q);
-    int ftout = which == 0 ? HH : EE;
     for (int t = 0; t < 2; ++t) {
-        int u = t == 0 ? (w + 1) % 3 : (w + 2) % 3;
-        int v = t == 0 ? (w + 2) % 3 : (w + 1) % 3;
-        double sg = t == 0 ? 1.0 : -1.0;
-        int isfwd = which == 0 ? (g.bft[v] == EE) : (g.bft[v] == HH);
-        int gi = g0type(g.bft, ftout, v);
-        const c64 *inv = g.sdlinv[gi][v];
-        int Nv = g.N[v];
-        int64_t st = stride3(g, v);
-        int key = 0;
-        if (isfwd) {
-            c64 dg = -(sg * inv[q[v]]);
-            if (q[v] > 0) {
-                L.push(dofidx(g, u, p), key, dg);
-                L.push(dofidx(g, u, p - st), key + 1, sg * inv[q[v] - 1]);
-            } else if (g.bloch[v]) {
-                c64 val = (sg * inv[Nv - 1]) * g.ph[v];
-                int64_t r = p + (int64_t)(Nv - 1) * st;
-                if (Nv == 1) L.push(dofidx(g, u, p), key, dg + val);
-                else { L.push(dofidx(g, u, p), key, dg); L.push(dofidx(g, u, r), key + 1, val); }
-            } else L.push(dofidx(g, u, p), key, dg);
-        } else {
-            c64 dg = sg * inv[q[v]];
-            if (q[v] < Nv - 1) {
-                L.push(dofidx(g, u, p), key, dg);
-                L.push(dofidx(g, u, p + st), key + 1, -(sg * inv[q[v] + 1]));
-            } else if (g.bloch[v]) {
-                c64 val = (-(sg * inv[0])) * g.phinv[v];
-                int64_t r = p - (int64_t)(Nv - 1) * st;
-                if (Nv == 1) L.push(dofidx(g, u, p), key, dg + val);
-                else { L.push(dofidx(g, u, p), key, dg); L.push(dofidx(g, u, r), key + 1, val); }
-            } else L.push(dofidx(g, u, p), key, dg);
-        }
+        const int u = (w + 1 + t) % 3;
+        c64 va, vb;
+        int qb;
+        int64_t pb;
+        const bool two = curl_pair(g, which, w, t, q, p, va, qb, pb, vb);
+        L.push(dofidx(g, u, p), 0, va);
+        if (two) L.push(dofidx(g, u, pb), 1, vb);
     }
     L.sort_merge();
 }
 
-// Corners that the field value F_w(qc) contributes to, with their weights:
-// the ∆l-weighted average along w (direction isfwd_in[w]; weights s∆l at the
-// field planes over 2 s∆l at the corner planes) that create_mean performs for
-// Pε/Pμ and for create_Mcs (model.jl:287-306).  Returns the entry count (1 or 2).
-__device__ inline int corner_entries(const DGrid<double> &g, int which, int w, int64_t qc, int64_t cor[2],
-                                     c64 wt[2]) {
-    int ft = which == 0 ? EE : HH;
-    int q[3];
-    unc3(g, qc, q);
-    int gc = g0type(g.bft, ft, w), gf = 1 - gc;
-    int fwd_in_w = which == 0 ? (g.bft[w] != EE) : (g.bft[w] != HH);
-    int Nw = g.N[w];
-    int64_t stw = stride3(g, w);
-    int n = 0;
-    for (int ic = 0; ic < 2; ++ic) {
-        int64_t c = qc;
-        int cw = q[w], fi = q[w];
-        c64 phin = mk<double>(1.0, 0.0);
-        if (ic == 1) {
-            if (!fwd_in_w) {   // corner c takes fields c and c - ŵ: q is the c - ŵ of c = q + ŵ
-                if (q[w] < Nw - 1) { c = qc + stw; cw = q[w] + 1; }
-                else if (g.bloch[w]) { c = qc - (int64_t)(Nw - 1) * stw; cw = 0; phin = g.phinv[w]; }
-                else continue;
-            } else {           // corner c takes fields c and c + ŵ
-                if (q[w] > 0) { c = qc - stw; cw = q[w] - 1; }
-                else if (g.bloch[w]) { c = qc + (int64_t)(Nw - 1) * stw; cw = Nw - 1; phin = g.ph[w]; }
-                else continue;
-            }
+// The corner that the field value F_w(qc) contributes to at its own position
+// (ic = 0) or one cell off along w (ic = 1; false when there is none), with the
+// weight of the ∆l-weighted average along w (direction isfwd_in[w]; weights s∆l
+// at the field planes over 2 s∆l at the corner planes) that create_mean
+// performs for Pε/Pμ and for create_Mcs (model.jl:287-306); cw: its w index.
+__device__ inline bool corner_entry(const DGrid<double> &g, int which, int w, int ic, const int q[3], int64_t qc,
+                                    int64_t &c, int &cw, c64 &wt) {
+    const int ft = which == 0 ? EE : HH;
+    const int gc = g0type(g.bft, ft, w), gf = 1 - gc;
+    const bool fwd_in_w = which == 0 ? (g.bft[w] != EE) : (g.bft[w] != HH);
+    const int Nw = g.N[w], fi = q[w];
+    const int64_t stw = stride3(g, w);
+    c64 phin = mk<double>(1.0, 0.0);
+    bool ok = true;
+    c = qc;
+    cw = fi;
+    if (ic == 1) {
+        if (!fwd_in_w) {   // corner c takes fields c and c - ŵ: q is the c - ŵ of c = q + ŵ
+            if (fi < Nw - 1) { c = qc + stw; cw = fi + 1; }
+            else if (g.bloch[w]) { c = qc - (int64_t)(Nw - 1) * stw; cw = 0; phin = g.phinv[w]; }
+            else ok = false;
+        } else {           // corner c takes fields c and c + ŵ
+            if (fi > 0) { c = qc - stw; cw = fi - 1; }
+            else if (g.bloch[w]) { c = qc + (int64_t)(Nw - 1) * stw; cw = Nw - 1; phin = g.ph[w]; }
+            else ok = false;
         }
-        cor[n] = c;
-        wt[n] = ((0.5 * g.sdl[gf][w][fi]) * g.sdlinv[gc][w][cw]) * phin;
-        ++n;
     }
-    return n;
+    wt = ((0.5 * g.sdl[gf][w][fi]) * g.sdlinv[gc][w][cw]) * phin;
+    return ok;
 }
 
 // Column (w, q) of the corner-mean operator Mcₑ (which = 0) or Mcₘ (which = 1):
 // F_w at q goes to the w-component slot of its corners.
 __device__ void mean_col(const DGrid<double> &g, int which, int w, int64_t qc, EList<2> &L) {
-    int64_t cor[2];
-    c64 wt[2];
-    int n = corner_entries(g, which, w, qc, cor, wt);
-    for (int x = 0; x < n; ++x) L.push(dofidx(g, w, cor[x]), x, wt[x]);
+    int q[3];
+    unc3(g, qc, q);
+    for (int ic = 0; ic < 2; ++ic) {
+        int64_t c;
+        int cw;
+        c64 wt;
+        if (corner_entry(g, which, w, ic, q, qc, c, cw, wt)) L.push(dofidx(g, w, c), ic, wt);
+    }
     L.sort_merge();
+}
+
+// The row cell that corner c (indices cq) gives to F_v at its own position
+// (oc = 0) or one cell off along v (oc = 1; false when there is none), with the
+// half weight and phase of that average.
+__device__ inline bool param_out(const DGrid<double> &g, int which, int v, int oc, const int cq[3], int64_t c,
+                                 int64_t &pr, c64 &fo) {
+    const bool fwd_in_v = which == 0 ? (g.bft[v] != EE) : (g.bft[v] != HH);
+    const int Nv = g.N[v];
+    const int64_t stv = stride3(g, v);
+    pr = c;
+    fo = mk<double>(0.5, 0.0);
+    if (oc == 0) return true;
+    if (!fwd_in_v) {   // row p takes corners p and p + v̂
+        if (cq[v] > 0) pr = c - stv;
+        else if (g.bloch[v]) { pr = c + (int64_t)(Nv - 1) * stv; fo = 0.5 * g.ph[v]; }
+        else return false;
+    } else {           // row p takes corners p and p - v̂
+        if (cq[v] < Nv - 1) pr = c + stv;
+        else if (g.bloch[v]) { pr = c - (int64_t)(Nv - 1) * stv; fo = 0.5 * g.phinv[v]; }
+        else return false;
+    }
+    return true;
 }
 
 // Column (w, q) of Pε (which = 0) or Pμ (which = 1).  The off-diagonal block
 // (v, w) takes F_w to the corners of grid g0 with a ∆l-weighted average along
-// w (direction isfwd_in[w]; weights s∆l at the field planes over 2 s∆l at the
-// corner planes), multiplies by parr(v,w) at the corner, and takes the corner
-// values to F_v by a half-half average along v in the other direction.
+// w, multiplies by parr(v,w) at the corner, and takes the corner values to F_v
+// by a half-half average along v in the other direction.
 __device__ void param_col(const DGrid<double> &g, int which, const c64 *parr, int full, int w, int64_t qc,
                           EList<9> &L) {
     int64_t M = g.M;
     L.push(dofidx(g, w, qc), 0, parr[qc + M * (w + 3 * w)]);
     if (!full) return;
-    int64_t cor[2];
-    c64 wt[2];
-    const int ncor = corner_entries(g, which, w, qc, cor, wt);
-    for (int ic = 0; ic < ncor; ++ic) {
-        const int64_t c = cor[ic];
-        const c64 wi = wt[ic];
+    int q[3];
+    unc3(g, qc, q);
+    for (int ic = 0; ic < 2; ++ic) {
+        int64_t c;
+        int cw;
+        c64 wi;
+        if (!corner_entry(g, which, w, ic, q, qc, c, cw, wi)) continue;
         int cq[3];
         unc3(g, c, cq);
         for (int v = 0; v < 3; ++v) {
             if (v == w) continue;
-            int fwd_in_v = which == 0 ? (g.bft[v] != EE) : (g.bft[v] != HH);
-            int Nv = g.N[v];
-            int64_t stv = stride3(g, v);
             c64 ec = parr[c + M * (v + 3 * w)];
             for (int oc = 0; oc < 2; ++oc) {
-                int64_t pr = c;
-                c64 fo = mk<double>(0.5, 0.0);
-                if (oc == 1) {
-                    if (!fwd_in_v) {   // row p takes corners p and p + v̂
-                        if (cq[v] > 0) pr = c - stv;
-                        else if (g.bloch[v]) { pr = c + (int64_t)(Nv - 1) * stv; fo = 0.5 * g.ph[v]; }
-                        else continue;
-                    } else {           // row p takes corners p and p - v̂
-                        if (cq[v] < Nv - 1) pr = c + stv;
-                        else if (g.bloch[v]) { pr = c - (int64_t)(Nv - 1) * stv; fo = 0.5 * g.phinv[v]; }
-                        else continue;
-                    }
-                }
-                L.push(dofidx(g, v, pr), 1 + 2 * oc + ic, ec * (fo * wi));
+                int64_t pr;
+                c64 fo;
+                if (param_out(g, which, v, oc, cq, c, pr, fo)) L.push(dofidx(g, v, pr), 1 + 2 * oc + ic, ec * (fo * wi));
             }
         }
     }
@@ -240,64 +268,195 @@ __global__ void k_param(DGrid<double> g, int which, const c64 *parr, const int *
 // Column of A = Cₘ (Pμ \ Cₑ) − ω² Pε (ft = EE, model.jl:235-237) or
 // A = Cₑ (Pε \ Cₘ) − ω² Pμ (ft = HH, model.jl:238-240).  The product is
 // accumulated in the order of Gustavson's algorithm (inner-factor column
-// entries by row, then outer-factor column entries by row), then rows are
-// sorted; the ω² term is subtracted with zero results dropped (skipped when
-// ω = 0, as the reference does).  `dv` is the diagonal divisor array (μ for
-// EE, ε for HH) and `pw` the parameter array of the ω² term.
-template <bool FILL>
-__global__ void k_A(DGrid<double> g, int ft, const c64 *pw, const c64 *dv, const int *full, c64 om2, int omz,
-                    int64_t n, int64_t *cnt, const int64_t *colptr, int64_t *rowval, c64 *nzval) {
-    int64_t col = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (col >= n) return;
+// entries by row, then outer-factor column entries by row); the ω² term is
+// subtracted with zero results dropped (skipped when ω = 0, as the reference
+// does).  `dv` is the diagonal divisor array (μ for EE, ε for HH) and `pw` the
+// parameter array of the ω² term.
+//
+// Every list is a fixed set of slots in registers (16 products, 9 parameter
+// entries; an absent one has the row NONE): equal rows are found by comparing
+// slot pairs, and an entry's place in the column is the number of entries with
+// a smaller row, so nothing is indexed at run time.  Lists indexed at run time
+// lay in scratch memory (1,040 bytes a thread), which bound the kernel: on
+// 56×48×50 cells, full ε, 1.07 ms to count and 1.17 ms to fill; now 0.10 and
+// 0.14 ms (the fill writes about 126 MB there).
+// Rows fit 32 bits: the two 9M-value parameter arrays that an assembly uploads
+// would need 412 GB at M = 2³²/3.
+constexpr uint32_t NONE = 0xffffffffu;
+template <bool FILL, int W>
+__device__ __forceinline__ void A_col(const DGrid<double> &g, int ft, const c64 *pw, const c64 *dv, int full, c64 om2,
+                                      int omz, int64_t p, int64_t *cnt, const int64_t *colptr, int64_t *rowval,
+                                      c64 *nzval) {
     const int inner = ft == EE ? 0 : 1;   // Cₑ first for EE, Cₘ first for HH
-    int w;
-    int64_t p;
-    col2cp(g, col, w, p);
-    EList<4> ce;
-    curl_col(g, inner, w, p, ce);
-    EList<16> acc;
-    for (int k = 0; k < ce.n; ++k) {
-        int u;
-        int64_t r;
-        col2cp(g, ce.e[k].row, u, r);
-        c64 b = cdiv(ce.e[k].v, dv[r + g.M * (u + 3 * u)]);
-        EList<4> cm;
-        curl_col(g, 1 - inner, u, r, cm);
-        for (int x = 0; x < cm.n; ++x) {
-            c64 prod = cm.e[x].v * b;
-            int f = -1;
-            for (int y = 0; y < acc.n; ++y)
-                if (acc.e[y].row == cm.e[x].row) { f = y; break; }
-            if (f >= 0) acc.e[f].v = acc.e[f].v + prod;
-            else acc.push(cm.e[x].row, acc.n, prod);
-        }
-    }
-    acc.sort_merge();
-    int64_t o = FILL ? colptr[col] : 0;
-    int m = 0;
-    if (omz) {
-        for (int x = 0; x < acc.n; ++x) {
-            if (FILL) { rowval[o + m] = acc.e[x].row + 1; nzval[o + m] = acc.e[x].v; }
-            ++m;
-        }
-    } else {
-        EList<9> pe;
-        param_col(g, inner, pw, *full, w, p, pe);
-        int a = 0, b = 0;
-        while (a < acc.n || b < pe.n) {
-            int64_t ra = a < acc.n ? acc.e[a].row : INT64_MAX, rb = b < pe.n ? pe.e[b].row : INT64_MAX;
-            c64 v;
-            int64_t r;
-            if (ra == rb) { v = acc.e[a].v - om2 * pe.e[b].v; r = ra; ++a; ++b; }
-            else if (ra < rb) { v = acc.e[a].v - mk<double>(0.0, 0.0); r = ra; ++a; }
-            else { v = mk<double>(0.0, 0.0) - om2 * pe.e[b].v; r = rb; ++b; }
-            if (!iszero(v)) {
-                if (FILL) { rowval[o + m] = r + 1; nzval[o + m] = v; }
-                ++m;
+    int q[3];
+    unc3(g, p, q);
+    uint32_t row[16], key[4];
+    c64 val[16];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int u = (W + 1 + t) % 3, v = t == 0 ? (W + 2) % 3 : (W + 1) % 3;
+        c64 e[2];
+        int qb;
+        int64_t pb;
+        const bool two = curl_pair(g, inner, W, t, q, p, e[0], qb, pb, e[1]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {   // inner-factor entry in row (u, r)
+            const int s = 2 * t + h;
+            const bool on = h == 0 || two;
+            const int64_t r = h == 0 ? p : pb;
+            int qr[3] = {q[0], q[1], q[2]};
+            if (h == 1) qr[v] = qb;
+            const c64 b = cdiv(e[h], dv[r + g.M * (u + 3 * u)]);
+            key[s] = on ? (uint32_t)dofidx(g, u, r) : NONE;
+#pragma unroll
+            for (int t2 = 0; t2 < 2; ++t2) {
+                const int u2 = (u + 1 + t2) % 3;
+                c64 va, vb;
+                int qn;
+                int64_t pn;
+                const bool two2 = curl_pair(g, 1 - inner, u, t2, qr, r, va, qn, pn, vb);
+                row[4 * s + 2 * t2] = on ? (uint32_t)dofidx(g, u2, r) : NONE;
+                val[4 * s + 2 * t2] = va * b;
+                row[4 * s + 2 * t2 + 1] = on && two2 ? (uint32_t)dofidx(g, u2, pn) : NONE;
+                val[4 * s + 2 * t2 + 1] = vb * b;
             }
         }
     }
-    if (!FILL) cnt[col] = m;
+    // the four inner-factor entries by row (all distinct), their products with them
+    auto order = [&](int a, int b) {
+        const bool sw = key[b] < key[a];
+        const uint32_t ka = key[a], kb = key[b];
+        key[a] = sw ? kb : ka;
+        key[b] = sw ? ka : kb;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const uint32_t ra = row[4 * a + x], rb = row[4 * b + x];
+            const c64 xa = val[4 * a + x], xb = val[4 * b + x];
+            row[4 * a + x] = sw ? rb : ra;
+            row[4 * b + x] = sw ? ra : rb;
+            val[4 * a + x] = sw ? xb : xa;
+            val[4 * b + x] = sw ? xa : xb;
+        }
+    };
+    order(0, 1);
+    order(2, 3);
+    order(0, 2);
+    order(1, 3);
+    order(1, 2);
+#pragma unroll
+    for (int i = 4; i < 16; ++i)
+#pragma unroll
+        for (int j = 0; j < (i & ~3); ++j)   // the four of one group lie in different rows
+            if (row[i] == row[j] && row[i] != NONE) {
+                val[j] = val[j] + val[i];
+                row[i] = NONE;
+            }
+    uint32_t prow[9];
+    c64 pval[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) prow[i] = NONE;
+    if (!omz) {
+        prow[0] = (uint32_t)dofidx(g, W, p);
+        pval[0] = pw[p + g.M * (W + 3 * W)];
+        if (full) {
+#pragma unroll
+            for (int ic = 0; ic < 2; ++ic) {
+                int64_t c;
+                int cw;
+                c64 wi;
+                const bool on = corner_entry(g, inner, W, ic, q, p, c, cw, wi);
+                int cq[3] = {q[0], q[1], q[2]};
+                cq[W] = cw;
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const int v = (W + 1 + x) % 3;
+                    const c64 ec = pw[c + g.M * (v + 3 * W)];
+#pragma unroll
+                    for (int oc = 0; oc < 2; ++oc) {   // in the order in which equal rows add up
+                        int64_t pr;
+                        c64 fo;
+                        const bool to = param_out(g, inner, v, oc, cq, c, pr, fo);
+                        const int i = 1 + 4 * x + 2 * oc + ic;
+                        prow[i] = on && to ? (uint32_t)dofidx(g, v, pr) : NONE;
+                        pval[i] = ec * (fo * wi);
+                    }
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < i; ++j) {
+                        const int a = 1 + 4 * x + j, b = 1 + 4 * x + i;
+                        if (prow[a] == prow[b] && prow[b] != NONE) {
+                            pval[a] = pval[a] + pval[b];
+                            prow[b] = NONE;
+                        }
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            c64 d = mk<double>(0.0, 0.0);
+#pragma unroll
+            for (int j = 0; j < 9; ++j)
+                if (row[i] == prow[j] && row[i] != NONE) {
+                    d = om2 * pval[j];
+                    prow[j] = NONE;
+                }
+            val[i] = val[i] - d;
+            if (iszero(val[i])) row[i] = NONE;
+        }
+#pragma unroll
+        for (int j = 0; j < 9; ++j)
+            if (prow[j] != NONE) {
+                pval[j] = mk<double>(0.0, 0.0) - om2 * pval[j];
+                if (iszero(pval[j])) prow[j] = NONE;
+            }
+    }
+    const int64_t col = dofidx(g, W, p);
+    if (!FILL) {
+        int m = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m += row[i] != NONE;
+#pragma unroll
+        for (int j = 0; j < 9; ++j) m += prow[j] != NONE;
+        cnt[col] = m;
+        return;
+    }
+    const int64_t o = colptr[col];
+    auto place = [&](uint32_t r, c64 v) {
+        if (r == NONE) return;
+        int at = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) at += row[i] < r;
+#pragma unroll
+        for (int j = 0; j < 9; ++j) at += prow[j] < r;
+        rowval[o + at] = (int64_t)r + 1;
+        nzval[o + at] = v;
+    };
+#pragma unroll
+    for (int i = 0; i < 16; ++i) place(row[i], val[i]);
+#pragma unroll
+    for (int j = 0; j < 9; ++j) place(prow[j], pval[j]);
+}
+
+// One component w per block, so that every table and axis is known when the
+// code is compiled; the three blocks of a run of cells lie 8 apart, on one XCD
+// (blocks go to the XCDs in turn), whose L2 joins the pieces of a line that
+// their interleaved columns write.
+constexpr int A_BS = 128;
+static unsigned A_grid(int64_t M) { return (unsigned)(((M + 8 * A_BS - 1) / (8 * A_BS)) * 24); }
+template <bool FILL>
+__global__ __launch_bounds__(A_BS, 2) void k_A(DGrid<double> g, int ft, const c64 *pw, const c64 *dv, const int *full,
+                                            c64 om2, int omz, int64_t *cnt, const int64_t *colptr, int64_t *rowval,
+                                            c64 *nzval) {
+    const int w = (blockIdx.x >> 3) % 3;
+    const int64_t p = ((int64_t)(blockIdx.x / 24) * 8 + (blockIdx.x & 7)) * A_BS + threadIdx.x;
+    if (p >= g.M) return;
+    if (w == 0) A_col<FILL, 0>(g, ft, pw, dv, *full, om2, omz, p, cnt, colptr, rowval, nzval);
+    else if (w == 1) A_col<FILL, 1>(g, ft, pw, dv, *full, om2, omz, p, cnt, colptr, rowval, nzval);
+    else A_col<FILL, 2>(g, ft, pw, dv, *full, om2, omz, p, cnt, colptr, rowval, nzval);
 }
 
 // any nonzero off-diagonal entry in a (Nx,Ny,Nz,3,3) array
@@ -438,8 +597,8 @@ int A_csc(mfd_ctx *ctx, const DevGrid &G, int ft, mfd_c64 omega, const mfd_c64 *
     c64 om2 = om * om;
     int omz = (omega.re == 0.0 && omega.im == 0.0);
     return csc_drive(s, n, nnz, colptr, rowval, nzval,
-                     [&](int64_t *cnt) { k_A<false><<<nblk(n, 128), 128, 0, s>>>(g, ft, pa, da, full, om2, omz, n, cnt, nullptr, nullptr, nullptr); },
-                     [&](int64_t *cp, int64_t *rv, c64 *nz) { k_A<true><<<nblk(n, 128), 128, 0, s>>>(g, ft, pa, da, full, om2, omz, n, nullptr, cp, rv, nz); });
+                     [&](int64_t *cnt) { k_A<false><<<A_grid(g.M), A_BS, 0, s>>>(g, ft, pa, da, full, om2, omz, cnt, nullptr, nullptr, nullptr); },
+                     [&](int64_t *cp, int64_t *rv, c64 *nz) { k_A<true><<<A_grid(g.M), A_BS, 0, s>>>(g, ft, pa, da, full, om2, omz, nullptr, cp, rv, nz); });
 }
 
 
