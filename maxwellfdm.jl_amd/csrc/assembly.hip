@@ -477,52 +477,33 @@ static inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) 
 
 // count -> scan -> fill -> copy out (1-based) driver shared by all operators
 template <typename CountF, typename FillF>
-static int csc_drive(hipStream_t s, int64_t n, int64_t *nnz_out, int64_t *colptr_h, int64_t *rowval_h,
+static int csc_drive(mfd_ctx *ctx, int64_t n, int64_t *nnz_out, int64_t *colptr_h, int64_t *rowval_h,
                      mfd_c64 *nzval_h, CountF count, FillF fill) {
-    int64_t *cnt = nullptr, *colptr = nullptr, *rowval = nullptr;
-    c64 *nzval = nullptr;
-    void *tmp = nullptr;
+    hipStream_t s = ctx->stream;
+    Scratch C, P, T, R, Z;
     size_t tmpb = 0;
-    int rc = MFD_OK;
-    auto fail = [&](hipError_t e) {
-        set_error(std::string("HIP error in CSC assembly: ") + hipGetErrorString(e));
-        rc = MFD_ERR_HIP;
-    };
-    hipError_t e;
-    if ((e = hipMalloc(&cnt, sizeof(int64_t) * (n + 1))) != hipSuccess) { fail(e); goto done; }
-    if ((e = hipMalloc(&colptr, sizeof(int64_t) * (n + 1))) != hipSuccess) { fail(e); goto done; }
+    MFD_TRY(C.get(ctx, sizeof(int64_t) * (n + 1)));
+    MFD_TRY(P.get(ctx, sizeof(int64_t) * (n + 1)));
+    int64_t *cnt = (int64_t *)C.p, *colptr = (int64_t *)P.p;
     count(cnt);
-    if ((e = hipGetLastError()) != hipSuccess) { fail(e); goto done; }
+    MFD_HIP(hipGetLastError());
     hipcub::DeviceScan::ExclusiveSum(nullptr, tmpb, cnt, colptr, n + 1, s);
-    if ((e = hipMalloc(&tmp, tmpb)) != hipSuccess) { fail(e); goto done; }
-    if ((e = hipMemsetAsync(cnt + n, 0, sizeof(int64_t), s)) != hipSuccess) { fail(e); goto done; }
-    hipcub::DeviceScan::ExclusiveSum(tmp, tmpb, cnt, colptr, n + 1, s);
-    {
-        int64_t nnz = 0;
-        if ((e = hipMemcpyAsync(&nnz, colptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, s)) != hipSuccess) { fail(e); goto done; }
-        if ((e = hipStreamSynchronize(s)) != hipSuccess) { fail(e); goto done; }
-        *nnz_out = nnz;
-        if (!colptr_h) goto done;   // size query only
-        if ((e = hipMalloc(&rowval, sizeof(int64_t) * (nnz ? nnz : 1))) != hipSuccess) { fail(e); goto done; }
-        if ((e = hipMalloc(&nzval, sizeof(c64) * (nnz ? nnz : 1))) != hipSuccess) { fail(e); goto done; }
-        fill(colptr, rowval, nzval);
-        k_colptr1<<<nblk(n + 1, 256), 256, 0, s>>>(colptr, n);
-        if ((e = hipGetLastError()) != hipSuccess) { fail(e); goto done; }
-        if ((e = hipMemcpyAsync(colptr_h, colptr, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost, s)) != hipSuccess) { fail(e); goto done; }
-        if (nnz) {
-            if ((e = hipMemcpyAsync(rowval_h, rowval, sizeof(int64_t) * nnz, hipMemcpyDeviceToHost, s)) != hipSuccess) { fail(e); goto done; }
-            if ((e = hipMemcpyAsync(nzval_h, nzval, sizeof(c64) * nnz, hipMemcpyDeviceToHost, s)) != hipSuccess) { fail(e); goto done; }
-        }
-        if ((e = hipStreamSynchronize(s)) != hipSuccess) { fail(e); goto done; }
-    }
-done:
-    hipStreamSynchronize(s);
-    if (cnt) hipFree(cnt);
-    if (colptr) hipFree(colptr);
-    if (rowval) hipFree(rowval);
-    if (nzval) hipFree(nzval);
-    if (tmp) hipFree(tmp);
-    return rc;
+    MFD_TRY(T.get(ctx, tmpb));
+    MFD_HIP(hipMemsetAsync(cnt + n, 0, sizeof(int64_t), s));
+    hipcub::DeviceScan::ExclusiveSum(T.p, tmpb, cnt, colptr, n + 1, s);
+    int64_t nnz = 0;
+    MFD_HIP(hipMemcpyAsync(&nnz, colptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    MFD_HIP(hipStreamSynchronize(s));
+    *nnz_out = nnz;
+    if (!colptr_h) return MFD_OK;   // size query only
+    MFD_TRY(R.get(ctx, sizeof(int64_t) * nnz));
+    MFD_TRY(Z.get(ctx, sizeof(c64) * nnz));
+    fill(colptr, (int64_t *)R.p, (c64 *)Z.p);
+    k_colptr1<<<nblk(n + 1, 256), 256, 0, s>>>(colptr, n);
+    MFD_HIP(hipGetLastError());
+    MFD_TRY(copy_out(ctx, colptr_h, colptr, sizeof(int64_t) * (n + 1)));
+    MFD_TRY(copy_out(ctx, rowval_h, R.p, sizeof(int64_t) * nnz));
+    return copy_out(ctx, nzval_h, Z.p, sizeof(c64) * nnz);
 }
 
 int curl_csc(mfd_ctx *ctx, const DevGrid &G, int which, int64_t *nnz, int64_t *colptr, int64_t *rowval,
@@ -530,7 +511,7 @@ int curl_csc(mfd_ctx *ctx, const DevGrid &G, int which, int64_t *nnz, int64_t *c
     const DGrid<double> &g = G.d64;
     int64_t n = 3 * g.M;
     hipStream_t s = ctx->stream;
-    return csc_drive(s, n, nnz, colptr, rowval, nzval,
+    return csc_drive(ctx, n, nnz, colptr, rowval, nzval,
                      [&](int64_t *cnt) { k_curl<false><<<nblk(n, 256), 256, 0, s>>>(g, which, n, cnt, nullptr, nullptr, nullptr); },
                      [&](int64_t *cp, int64_t *rv, c64 *nz) { k_curl<true><<<nblk(n, 256), 256, 0, s>>>(g, which, n, nullptr, cp, rv, nz); });
 }
@@ -540,18 +521,16 @@ int mean_csc(mfd_ctx *ctx, const DevGrid &G, int which, int64_t *nnz, int64_t *c
     const DGrid<double> &g = G.d64;
     int64_t n = 3 * g.M;
     hipStream_t s = ctx->stream;
-    return csc_drive(s, n, nnz, colptr, rowval, nzval,
+    return csc_drive(ctx, n, nnz, colptr, rowval, nzval,
                      [&](int64_t *cnt) { k_mean<false><<<nblk(n, 256), 256, 0, s>>>(g, which, n, cnt, nullptr, nullptr, nullptr); },
                      [&](int64_t *cp, int64_t *rv, c64 *nz) { k_mean<true><<<nblk(n, 256), 256, 0, s>>>(g, which, n, nullptr, cp, rv, nz); });
 }
 
-DevArray::~DevArray() { if (p) hipFree(p); }
-
-int upload_param(mfd_ctx *ctx, const DevGrid &G, const mfd_c64 *parr, DevArray &d, int *full_h) {
+int upload_param(mfd_ctx *ctx, const DevGrid &G, const mfd_c64 *parr, Scratch &d, int *full_h) {
     int64_t M = G.d64.M;
     size_t bytes = sizeof(c64) * 9 * M + 64;
-    MFD_HIP(hipMalloc(&d.p, bytes));
-    MFD_HIP(hipMemcpyAsync(d.p, parr, sizeof(c64) * 9 * M, hipMemcpyHostToDevice, ctx->stream));
+    MFD_TRY(d.get(ctx, bytes));
+    MFD_TRY(copy_in(ctx, d.p, parr, sizeof(c64) * 9 * M));
     int *flag = (int *)((char *)d.p + sizeof(c64) * 9 * M);
     MFD_HIP(hipMemsetAsync(flag, 0, sizeof(int), ctx->stream));
     k_offdiag<<<nblk(9 * M, 256), 256, 0, ctx->stream>>>((const c64 *)d.p, M, flag);
@@ -568,11 +547,11 @@ int param_csc(mfd_ctx *ctx, const DevGrid &G, int which, const mfd_c64 *parr, in
     const DGrid<double> &g = G.d64;
     int64_t n = 3 * g.M;
     hipStream_t s = ctx->stream;
-    DevArray P;
+    Scratch P;
     MFD_TRY(upload_param(ctx, G, parr, P, nullptr));
     const c64 *pa = (const c64 *)P.p;
     const int *full = (const int *)((const char *)P.p + sizeof(c64) * 9 * g.M);
-    return csc_drive(s, n, nnz, colptr, rowval, nzval,
+    return csc_drive(ctx, n, nnz, colptr, rowval, nzval,
                      [&](int64_t *cnt) { k_param<false><<<nblk(n, 256), 256, 0, s>>>(g, which, pa, full, n, cnt, nullptr, nullptr, nullptr); },
                      [&](int64_t *cp, int64_t *rv, c64 *nz) { k_param<true><<<nblk(n, 256), 256, 0, s>>>(g, which, pa, full, n, nullptr, cp, rv, nz); });
 }
@@ -582,7 +561,7 @@ int A_csc(mfd_ctx *ctx, const DevGrid &G, int ft, mfd_c64 omega, const mfd_c64 *
     const DGrid<double> &g = G.d64;
     int64_t n = 3 * g.M;
     hipStream_t s = ctx->stream;
-    DevArray Dv, Pw;   // divisor (diagonal) and ω²-term parameter arrays
+    Scratch Dv, Pw;   // divisor (diagonal) and ω²-term parameter arrays
     int dfull = 0;
     MFD_TRY(upload_param(ctx, G, ft == EE ? mu : eps, Dv, &dfull));
     if (dfull) {
@@ -596,7 +575,7 @@ int A_csc(mfd_ctx *ctx, const DevGrid &G, int ft, mfd_c64 omega, const mfd_c64 *
     c64 om = mk<double>(omega.re, omega.im);
     c64 om2 = om * om;
     int omz = (omega.re == 0.0 && omega.im == 0.0);
-    return csc_drive(s, n, nnz, colptr, rowval, nzval,
+    return csc_drive(ctx, n, nnz, colptr, rowval, nzval,
                      [&](int64_t *cnt) { k_A<false><<<A_grid(g.M), A_BS, 0, s>>>(g, ft, pa, da, full, om2, omz, cnt, nullptr, nullptr, nullptr); },
                      [&](int64_t *cp, int64_t *rv, c64 *nz) { k_A<true><<<A_grid(g.M), A_BS, 0, s>>>(g, ft, pa, da, full, om2, omz, nullptr, cp, rv, nz); });
 }
@@ -652,11 +631,9 @@ int csc_upload(mfd_ctx *ctx, const mfd_csc *h, const char *name, DevCsc &d) {
     d.rowval = (int64_t *)((char *)d.buf + off_rv);
     d.nzval = (c64 *)((char *)d.buf + off_nz);
     int *flag = (int *)((char *)d.buf + off_fl);
-    MFD_HIP(hipMemcpyAsync(d.colptr, h->colptr, bcp, hipMemcpyHostToDevice, s));
-    if (h->nnz) {
-        MFD_HIP(hipMemcpyAsync(d.rowval, h->rowval, brv, hipMemcpyHostToDevice, s));
-        MFD_HIP(hipMemcpyAsync(d.nzval, h->nzval, bnz, hipMemcpyHostToDevice, s));
-    }
+    MFD_TRY(copy_in(ctx, d.colptr, h->colptr, bcp));
+    MFD_TRY(copy_in(ctx, d.rowval, h->rowval, brv));
+    MFD_TRY(copy_in(ctx, d.nzval, h->nzval, bnz));
     MFD_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
     if (h->n) k_csc_check<<<nblk(h->n, 256), 256, 0, s>>>(h->m, h->n, d.colptr, d.rowval, flag);
     MFD_HIP(hipGetLastError());
@@ -859,9 +836,9 @@ static int square_n(const mfd_csc *const *ms, const char *const *names, int cnt,
 }
 
 // diagonal of the divisor `P` of `P \ C`, refused unless diagonal and nonsingular
-static int divisor_diag(mfd_ctx *ctx, const DevCsc &P, const char *what, DevArray &d) {
+static int divisor_diag(mfd_ctx *ctx, const DevCsc &P, const char *what, Scratch &d) {
     hipStream_t s = ctx->stream;
-    MFD_HIP(hipMalloc(&d.p, sizeof(c64) * P.n + 256));
+    MFD_TRY(d.get(ctx, sizeof(c64) * P.n + 256));
     int *flag = (int *)((char *)d.p + sizeof(c64) * P.n);
     MFD_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
     if (P.n) k_csc_diag<<<nblk(P.n, 256), 256, 0, s>>>(P.view(), (c64 *)d.p, flag);
@@ -890,18 +867,17 @@ int A_from_csc(mfd_ctx *ctx, int ft, mfd_c64 omega, const mfd_csc *Pe, const mfd
     MFD_TRY(csc_upload(ctx, Y, ft == EE ? "Cₑ" : "Cₘ", dY));
     MFD_TRY(csc_upload(ctx, D, ft == EE ? "Pμ" : "Pε", dD));
     MFD_TRY(csc_upload(ctx, S, ft == EE ? "Pε" : "Pμ", dS));
-    DevArray dd;
+    Scratch dd;
     MFD_TRY(divisor_diag(ctx, dD, ft == EE ? "Pμ" : "Pε", dd));
     hipStream_t s = ctx->stream;
     const c64 om = mk<double>(omega.re, omega.im), s2 = om * om;
     const int sub = !(omega.re == 0.0 && omega.im == 0.0);
-    int *flag = nullptr;
-    MFD_HIP(hipMalloc(&flag, sizeof(int)));
-    DevArray fguard;
-    fguard.p = flag;
+    Scratch F;
+    MFD_TRY(F.get(ctx, sizeof(int)));
+    int *flag = (int *)F.p;
     MFD_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
     const c64 *dv = (const c64 *)dd.p;
-    int rc = csc_drive(s, n, nnz, colptr, rowval, nzval,
+    int rc = csc_drive(ctx, n, nnz, colptr, rowval, nzval,
                        [&](int64_t *cnt) { k_spgemm<false><<<nblk(n, 128), 128, 0, s>>>(dX.view(), dY.view(), dv, dS.view(), s2, sub, n, cnt, nullptr, nullptr, nullptr, flag); },
                        [&](int64_t *cp, int64_t *rv, c64 *nz) { k_spgemm<true><<<nblk(n, 128), 128, 0, s>>>(dX.view(), dY.view(), dv, dS.view(), s2, sub, n, nullptr, cp, rv, nz, flag); });
     int f = 0;
@@ -928,16 +904,16 @@ int b_from_csc(mfd_ctx *ctx, int ft, mfd_c64 omega, const mfd_csc *Pe, const mfd
     DevCsc dX, dD;
     MFD_TRY(csc_upload(ctx, X, ft == EE ? "Cₘ" : "Cₑ", dX));
     MFD_TRY(csc_upload(ctx, D, ft == EE ? "Pμ" : "Pε", dD));
-    DevArray dd;
+    Scratch dd;
     MFD_TRY(divisor_diag(ctx, dD, ft == EE ? "Pμ" : "Pε", dd));
     DevCsr R;
     MFD_TRY(csr_of(ctx, dX, R));
     hipStream_t s = ctx->stream;
-    DevArray V;
-    MFD_HIP(hipMalloc(&V.p, sizeof(c64) * 3 * n + 64));
+    Scratch V;
+    MFD_TRY(V.get(ctx, sizeof(c64) * 3 * n + 64));
     c64 *y = (c64 *)V.p, *jdd = y + n, *jwd = y + 2 * n;
-    MFD_HIP(hipMemcpyAsync(jdd, jd, sizeof(c64) * n, hipMemcpyHostToDevice, s));
-    MFD_HIP(hipMemcpyAsync(jwd, jw, sizeof(c64) * n, hipMemcpyHostToDevice, s));
+    MFD_TRY(copy_in(ctx, jdd, jd, sizeof(c64) * n));
+    MFD_TRY(copy_in(ctx, jwd, jw, sizeof(c64) * n));
     const c64 om = mk<double>(omega.re, omega.im), iw = om * mk<double>(0.0, 1.0);
     const int omz = omega.re == 0.0 && omega.im == 0.0;
     if (n) {
@@ -947,9 +923,7 @@ int b_from_csc(mfd_ctx *ctx, int ft, mfd_c64 omega, const mfd_csc *Pe, const mfd
         k_b_finish<<<nblk(n, 256), 256, 0, s>>>(n, y, ft == EE, iw, omz, jwd);
     }
     MFD_HIP(hipGetLastError());
-    MFD_HIP(hipMemcpyAsync(b, y, sizeof(c64) * n, hipMemcpyDeviceToHost, s));
-    MFD_HIP(hipStreamSynchronize(s));
-    return MFD_OK;
+    return copy_out(ctx, b, y, sizeof(c64) * n);
 }
 
 int field_from_csc(mfd_ctx *ctx, int which, mfd_c64 omega, const mfd_csc *P, const mfd_csc *Cx,
@@ -964,16 +938,16 @@ int field_from_csc(mfd_ctx *ctx, int which, mfd_c64 omega, const mfd_csc *P, con
     DevCsc dP, dC;
     MFD_TRY(csc_upload(ctx, P, pn, dP));
     MFD_TRY(csc_upload(ctx, Cx, cn, dC));
-    DevArray dd;
+    Scratch dd;
     MFD_TRY(divisor_diag(ctx, dP, pn, dd));
     DevCsr R;
     MFD_TRY(csr_of(ctx, dC, R));
     hipStream_t s = ctx->stream;
-    DevArray V;
-    MFD_HIP(hipMalloc(&V.p, sizeof(c64) * 3 * n + 64));
+    Scratch V;
+    MFD_TRY(V.get(ctx, sizeof(c64) * 3 * n + 64));
     c64 *vin = (c64 *)V.p, *vsrc = vin + n, *vout = vin + 2 * n;
-    MFD_HIP(hipMemcpyAsync(vin, in, sizeof(c64) * n, hipMemcpyHostToDevice, s));
-    if (src) MFD_HIP(hipMemcpyAsync(vsrc, src, sizeof(c64) * n, hipMemcpyHostToDevice, s));
+    MFD_TRY(copy_in(ctx, vin, in, sizeof(c64) * n));
+    if (src) MFD_TRY(copy_in(ctx, vsrc, src, sizeof(c64) * n));
     // h = (i/ω) (Pμ \ (Cₑ e + jₘ));  e = (−i/ω) (Pε \ (Cₘ h − jₑ))
     const c64 om = mk<double>(omega.re, omega.im);
     const c64 f = cdiv(mk<double>(0.0, which == 0 ? 1.0 : -1.0), om);
@@ -981,9 +955,7 @@ int field_from_csc(mfd_ctx *ctx, int which, mfd_c64 omega, const mfd_csc *P, con
         k_csr_mv<<<nblk(n, 256), 256, 0, s>>>(n, R.rowptr, R.colind, R.val, vin, src ? vsrc : nullptr,
                                                mk<double>(which == 0 ? 1.0 : -1.0, 0), (const c64 *)dd.p, f, 1, vout);
     MFD_HIP(hipGetLastError());
-    MFD_HIP(hipMemcpyAsync(out, vout, sizeof(c64) * n, hipMemcpyDeviceToHost, s));
-    MFD_HIP(hipStreamSynchronize(s));
-    return MFD_OK;
+    return copy_out(ctx, out, vout, sizeof(c64) * n);
 }
 
 }  // namespace mfd

@@ -65,6 +65,12 @@ int mfd_ctx_create(int device, mfd_ctx **out) {
         set_error("hipStreamCreate failed");
         return MFD_ERR_HIP;
     }
+    c->mem = ctxmem_create(device);
+    if (!c->mem) {
+        hipStreamDestroy(c->stream);
+        delete c;
+        return MFD_ERR_ALLOC;
+    }
     *out = c;
     return MFD_OK;
 }
@@ -73,6 +79,7 @@ int mfd_ctx_destroy(mfd_ctx *ctx) {
     if (!ctx) return MFD_OK;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
+    ctxmem_destroy(ctx->mem);
     hipStreamDestroy(ctx->stream);
     delete ctx;
     return MFD_OK;

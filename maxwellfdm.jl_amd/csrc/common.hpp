@@ -129,7 +129,9 @@ void set_error(const std::string &msg);
 
 }  // namespace mfd
 
+namespace mfd { struct CtxMem; }
 struct mfd_ctx {
     int device;
     hipStream_t stream;
+    mfd::CtxMem *mem = nullptr;   // scratch memory and copy slots (ctxmem.hpp)
 };

@@ -673,7 +673,7 @@ static int hbuf_ensure(mfd_op *op, int64_t nrhs) {
         op->hbuf = nullptr;
         op->hbuf_bytes = 0;
     }
-    if (hipMalloc(&op->hbuf, need) != hipSuccess) {
+    if (ctx_malloc(op->ctx, &op->hbuf, need) != hipSuccess) {
         (void)hipGetLastError();   // clear it: the single-pass kernel serves without the scratch
         op->hbuf = nullptr;
         return MFD_OK;
@@ -733,7 +733,7 @@ static int ws_ensure(mfd_op *op, int64_t nrhs, int prec) {
     if (w.buf && w.nrhs == nrhs && w.prec == prec) return MFD_OK;
     w.release();
     const size_t bytes = ws_bytes(n, nrhs);
-    MFD_HIP(hipMalloc(&w.buf, bytes));
+    MFD_HIP(ctx_malloc(op->ctx, &w.buf, bytes));
     ws_carve(w, w.buf, n, nrhs);
     MFD_HIP(hipMemsetAsync(w.cnt, 0, sizeof(unsigned) * 3 * nrhs, op->stream));
     MFD_HIP(hipHostMalloc((void **)&w.scal_h, sizeof(Scal) * nrhs, hipHostMallocDefault));
@@ -860,7 +860,7 @@ int op_create_impl(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const
     op->n = 3 * M;
     op->omega = mk<double>(omega.re, omega.im);
     c64 om2 = op->omega * op->omega;
-    DevArray E, U;
+    Scratch E, U;
     int full = 0, mufull = 0;
     auto bail = [&](int code) { delete op; return code; };
     if ((rc = upload_param(ctx, op->G, eps_arr, E, &full))) return bail(rc);
@@ -891,7 +891,7 @@ int op_create_impl(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const
     size_t n3 = 3 * (size_t)M;
     size_t b64 = sizeof(c64) * n3, b32 = sizeof(c32) * n3;
     size_t bytes = 4 * (b64 + b32) + b64 + (b64 + b32) / 3 + 512;
-    if (hipMalloc(&op->buf, bytes) != hipSuccess) { set_error("hipMalloc failed for operator arrays"); return bail(MFD_ERR_ALLOC); }
+    if (ctx_malloc(ctx, &op->buf, bytes) != hipSuccess) { set_error("hipMalloc failed for operator arrays"); return bail(MFD_ERR_ALLOC); }
     char *p = (char *)op->buf;
     c64 *epsd = (c64 *)p; p += b64;
     c64 *epso = (c64 *)p; p += b64;
@@ -1016,7 +1016,7 @@ int op_create_csc_impl(mfd_ctx *ctx, const mfd_csc *A, mfd_op **out) {
     op->omega = mk<double>(0, 0);
     const size_t b64 = sizeof(c64) * n, b32 = sizeof(c32) * n;
     // q, qs, qo, T, T⁻¹ (FP64), q (FP32), flags
-    if (hipMalloc(&op->buf, 5 * b64 + b32 + 256) != hipSuccess) { set_error("hipMalloc failed for operator arrays"); return bail(MFD_ERR_ALLOC); }
+    if (ctx_malloc(ctx, &op->buf, 5 * b64 + b32 + 256) != hipSuccess) { set_error("hipMalloc failed for operator arrays"); return bail(MFD_ERR_ALLOC); }
     c64 *q = (c64 *)op->buf, *qs = q + n, *qo = q + 2 * n, *t = q + 3 * n, *tinv = q + 4 * n;
     c32 *q32 = (c32 *)(q + 5 * n);
     int *flag = (int *)((char *)op->buf + 5 * b64 + b32 + 64);
@@ -1149,18 +1149,12 @@ int op_apply_dev_impl(mfd_op *op, const void *x, void *y, int64_t nrhs, int prec
 int op_apply_impl(mfd_op *op, const mfd_c64 *x, mfd_c64 *y, int64_t nrhs) {
     int64_t n = op->n;
     size_t b = sizeof(c64) * n * nrhs;
-    void *dx = nullptr, *dy = nullptr;
-    MFD_HIP(hipMalloc(&dx, b));
-    if (hipMalloc(&dy, b) != hipSuccess) { hipFree(dx); set_error("hipMalloc failed"); return MFD_ERR_ALLOC; }
-    hipStream_t s = op->stream;
-    int rc = MFD_OK;
-    if (hipMemcpyAsync(dx, x, b, hipMemcpyHostToDevice, s) != hipSuccess) rc = MFD_ERR_HIP;
-    if (!rc) rc = op_apply_dev_impl(op, dx, dy, nrhs, MFD_FP64);
-    if (!rc && (hipMemcpyAsync(y, dy, b, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess))
-        rc = MFD_ERR_HIP;
-    hipFree(dx);
-    hipFree(dy);
-    return rc;
+    Scratch dx, dy;
+    MFD_TRY(dx.get(op->ctx, b));
+    MFD_TRY(dy.get(op->ctx, b));
+    MFD_TRY(copy_in(op->ctx, dx.p, x, b));
+    MFD_TRY(op_apply_dev_impl(op, dx.p, dy.p, nrhs, MFD_FP64));
+    return copy_out(op->ctx, y, dy.p, b);
 }
 
 // average ms of one stencil launch (EPI_STORE): MODE_A or MODE_P, FP64 or FP32 vectors
@@ -2574,48 +2568,40 @@ int solve_batch_impl(int count, mfd_op *const *ops, const mfd_c64 *const *b, mfd
     if (count < 1 || count > 1024 || !ops || !b || !e) { set_error("count must be in [1, 1024] with non-null arrays"); return MFD_ERR_ARG; }
     for (int p = 0; p < count; ++p)
         if (!ops[p] || !b[p] || !e[p]) { set_error("batched solve: null operator or array"); return MFD_ERR_ARG; }
-    hipStream_t s = ops[0]->ctx->stream;
+    mfd_ctx *ctx = ops[0]->ctx;
     std::vector<void *> db(count, nullptr), de(count, nullptr);
-    int rc = MFD_OK;
-    for (int p = 0; p < count && !rc; ++p) {
-        size_t bytes = sizeof(c64) * ops[p]->n;
-        if (hipMalloc(&db[p], bytes) != hipSuccess || hipMalloc(&de[p], bytes) != hipSuccess) { set_error("hipMalloc failed"); rc = MFD_ERR_ALLOC; break; }
-        if (hipMemcpyAsync(db[p], b[p], bytes, hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipMemcpyAsync(de[p], e[p], bytes, hipMemcpyHostToDevice, s) != hipSuccess) { set_error("copy to device failed"); rc = MFD_ERR_HIP; }
-    }
-    if (!rc) rc = solve_batch_dev_impl(count, ops, db.data(), de.data(), o, st);
-    if (rc == MFD_OK || rc == MFD_ERR_NOCONV) {
-        for (int p = 0; p < count; ++p) {
-            size_t bytes = sizeof(c64) * ops[p]->n;
-            if (hipMemcpyAsync(e[p], de[p], bytes, hipMemcpyDeviceToHost, s) != hipSuccess) rc = MFD_ERR_HIP;
-        }
-        if (hipStreamSynchronize(s) != hipSuccess) rc = MFD_ERR_HIP;
-    }
+    std::vector<size_t> at(count);
+    size_t total = 0;
     for (int p = 0; p < count; ++p) {
-        if (db[p]) hipFree(db[p]);
-        if (de[p]) hipFree(de[p]);
+        at[p] = total;
+        total += (sizeof(c64) * ops[p]->n + 255) / 256 * 256;
     }
+    Scratch B, E;
+    MFD_TRY(B.get(ctx, total));
+    MFD_TRY(E.get(ctx, total));
+    for (int p = 0; p < count; ++p) {
+        const size_t bytes = sizeof(c64) * ops[p]->n;
+        db[p] = (char *)B.p + at[p];
+        de[p] = (char *)E.p + at[p];
+        MFD_TRY(copy_in(ctx, db[p], b[p], bytes));
+        MFD_TRY(copy_in(ctx, de[p], e[p], bytes));
+    }
+    const int rc = solve_batch_dev_impl(count, ops, db.data(), de.data(), o, st);
+    if (rc == MFD_OK || rc == MFD_ERR_NOCONV)
+        for (int p = 0; p < count; ++p) MFD_TRY(copy_out(ctx, e[p], de[p], sizeof(c64) * ops[p]->n));
     return rc;
 }
 
 int solve_impl(mfd_op *op, const mfd_c64 *b, mfd_c64 *e, int64_t nrhs, const mfd_solve_opts *o, mfd_solve_stats *st) {
     int64_t n = op->n;
     size_t bytes = sizeof(c64) * n * nrhs;
-    void *db = nullptr, *de = nullptr;
-    MFD_HIP(hipMalloc(&db, bytes));
-    if (hipMalloc(&de, bytes) != hipSuccess) { hipFree(db); set_error("hipMalloc failed"); return MFD_ERR_ALLOC; }
-    hipStream_t s = op->stream;
-    int rc = MFD_OK;
-    if (hipMemcpyAsync(db, b, bytes, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(de, e, bytes, hipMemcpyHostToDevice, s) != hipSuccess)
-        rc = MFD_ERR_HIP;
-    if (!rc) rc = solve_dev_impl(op, db, de, nrhs, o, st);
-    if (rc == MFD_OK || rc == MFD_ERR_NOCONV) {
-        if (hipMemcpyAsync(e, de, bytes, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-            rc = MFD_ERR_HIP;
-    }
-    hipFree(db);
-    hipFree(de);
+    Scratch db, de;
+    MFD_TRY(db.get(op->ctx, bytes));
+    MFD_TRY(de.get(op->ctx, bytes));
+    MFD_TRY(copy_in(op->ctx, db.p, b, bytes));
+    MFD_TRY(copy_in(op->ctx, de.p, e, bytes));
+    const int rc = solve_dev_impl(op, db.p, de.p, nrhs, o, st);
+    if (rc == MFD_OK || rc == MFD_ERR_NOCONV) MFD_TRY(copy_out(op->ctx, e, de.p, bytes));
     return rc;
 }
 
@@ -2627,25 +2613,19 @@ int solve_adjoint_impl(mfd_op *op, const mfd_c64 *gvec, mfd_c64 *lam, const mfd_
     }
     int64_t n = 3 * op->G.h.M;
     size_t bytes = sizeof(c64) * n;
-    void *db = nullptr, *de = nullptr;
-    MFD_HIP(hipMalloc(&db, bytes));
-    if (hipMalloc(&de, bytes) != hipSuccess) { hipFree(db); return MFD_ERR_ALLOC; }
+    Scratch db, de;
+    MFD_TRY(db.get(op->ctx, bytes));
+    MFD_TRY(de.get(op->ctx, bytes));
     hipStream_t s = op->stream;
-    int rc = MFD_OK;
     // Aᵀ λ = g  <=>  A (S⁻¹ λ) = S⁻¹ g
-    if (hipMemcpyAsync(db, gvec, bytes, hipMemcpyHostToDevice, s) != hipSuccess || hipMemsetAsync(de, 0, bytes, s) != hipSuccess)
-        rc = MFD_ERR_HIP;
-    if (!rc) {
-        k_scale_S<<<ngrid(n), BS, 0, s>>>(op->G.d64, (c64 *)db, n, 1);
-        rc = solve_dev_impl(op, db, de, 1, o, st);
-    }
+    MFD_TRY(copy_in(op->ctx, db.p, gvec, bytes));
+    MFD_HIP(hipMemsetAsync(de.p, 0, bytes, s));
+    k_scale_S<<<ngrid(n), BS, 0, s>>>(op->G.d64, (c64 *)db.p, n, 1);
+    const int rc = solve_dev_impl(op, db.p, de.p, 1, o, st);
     if (rc == MFD_OK || rc == MFD_ERR_NOCONV) {
-        k_scale_S<<<ngrid(n), BS, 0, s>>>(op->G.d64, (c64 *)de, n, 0);
-        if (hipMemcpyAsync(lam, de, bytes, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-            rc = MFD_ERR_HIP;
+        k_scale_S<<<ngrid(n), BS, 0, s>>>(op->G.d64, (c64 *)de.p, n, 0);
+        MFD_TRY(copy_out(op->ctx, lam, de.p, bytes));
     }
-    hipFree(db);
-    hipFree(de);
     return rc;
 }
 
@@ -2737,54 +2717,36 @@ int field_convert_impl(mfd_op *op, int which, const mfd_c64 *in, const mfd_c64 *
     int64_t n = 3 * op->G.h.M;
     size_t bytes = sizeof(c64) * n;
     hipStream_t s = op->stream;
-    void *din = nullptr, *dsrc = nullptr, *dout = nullptr;
-    MFD_HIP(hipMalloc(&din, bytes));
-    int rc = MFD_OK;
-    if (hipMalloc(&dout, bytes) != hipSuccess || (src && hipMalloc(&dsrc, bytes) != hipSuccess)) { set_error("hipMalloc failed"); rc = MFD_ERR_ALLOC; }
-    if (!rc && (hipMemcpyAsync(din, in, bytes, hipMemcpyHostToDevice, s) != hipSuccess ||
-                (src && hipMemcpyAsync(dsrc, src, bytes, hipMemcpyHostToDevice, s) != hipSuccess)))
-        rc = MFD_ERR_HIP;
-    if (!rc) {
-        c64 iw = cdiv(mk<double>(0.0, 1.0), op->omega);   // i/ω
-        unsigned gr = ngrid(op->G.h.M);
-        if (which == 0) {
-            if (op->has_mu) k_h_from_e<true><<<gr, BS, 0, s>>>(op->G.d64, op->d64, (const c64 *)din, (const c64 *)dsrc, (c64 *)dout, iw);
-            else k_h_from_e<false><<<gr, BS, 0, s>>>(op->G.d64, op->d64, (const c64 *)din, (const c64 *)dsrc, (c64 *)dout, iw);
-        } else {
-            k_e_from_h<<<gr, BS, 0, s>>>(op->G.d64, op->d64, (const c64 *)din, (const c64 *)dsrc, (c64 *)dout,
-                                         mk<double>(-iw.re, -iw.im));
-        }
-        if (hipGetLastError() != hipSuccess || hipMemcpyAsync(out, dout, bytes, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            rc = MFD_ERR_HIP;
-    }
-    hipFree(din);
-    if (dout) hipFree(dout);
-    if (dsrc) hipFree(dsrc);
-    return rc;
+    Scratch din, dsrc, dout;
+    MFD_TRY(din.get(op->ctx, bytes));
+    MFD_TRY(dout.get(op->ctx, bytes));
+    if (src) MFD_TRY(dsrc.get(op->ctx, bytes));
+    MFD_TRY(copy_in(op->ctx, din.p, in, bytes));
+    if (src) MFD_TRY(copy_in(op->ctx, dsrc.p, src, bytes));
+    const c64 iw = cdiv(mk<double>(0.0, 1.0), op->omega);   // i/ω
+    const unsigned gr = ngrid(op->G.h.M);
+    const c64 *di = (const c64 *)din.p, *ds = (const c64 *)dsrc.p;
+    c64 *dd = (c64 *)dout.p;
+    if (which == 1) k_e_from_h<<<gr, BS, 0, s>>>(op->G.d64, op->d64, di, ds, dd, mk<double>(-iw.re, -iw.im));
+    else if (op->has_mu) k_h_from_e<true><<<gr, BS, 0, s>>>(op->G.d64, op->d64, di, ds, dd, iw);
+    else k_h_from_e<false><<<gr, BS, 0, s>>>(op->G.d64, op->d64, di, ds, dd, iw);
+    MFD_HIP(hipGetLastError());
+    return copy_out(op->ctx, out, dout.p, bytes);
 }
 
 int adjoint_grad_impl(mfd_op *op, const mfd_c64 *e, const mfd_c64 *lam, double *grad) {
     if (op->csr) { set_error("adjoint_grad: needs an operator built from a model (ω and the grid)"); return MFD_ERR_UNSUPPORTED; }
     if (op->win) { set_error("adjoint_grad: an operator with a component window (2D/1D model) is not supported"); return MFD_ERR_UNSUPPORTED; }
     int64_t n = 3 * op->G.h.M;
-    void *d = nullptr;
-    MFD_HIP(hipMalloc(&d, (2 * sizeof(c64) + sizeof(double)) * n));
-    hipStream_t s = op->stream;
-    c64 *de = (c64 *)d, *dl = de + n;
+    Scratch d;
+    MFD_TRY(d.get(op->ctx, (2 * sizeof(c64) + sizeof(double)) * n));
+    c64 *de = (c64 *)d.p, *dl = de + n;
     double *dg = (double *)(dl + n);
-    int rc = MFD_OK;
-    if (hipMemcpyAsync(de, e, sizeof(c64) * n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(dl, lam, sizeof(c64) * n, hipMemcpyHostToDevice, s) != hipSuccess)
-        rc = MFD_ERR_HIP;
-    if (!rc) {
-        k_grad<<<ngrid(n), BS, 0, s>>>(de, dl, op->omega * op->omega, dg, n);
-        if (hipMemcpyAsync(grad, dg, sizeof(double) * n, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            rc = MFD_ERR_HIP;
-    }
-    hipFree(d);
-    return rc;
+    MFD_TRY(copy_in(op->ctx, de, e, sizeof(c64) * n));
+    MFD_TRY(copy_in(op->ctx, dl, lam, sizeof(c64) * n));
+    k_grad<<<ngrid(n), BS, 0, op->stream>>>(de, dl, op->omega * op->omega, dg, n);
+    MFD_HIP(hipGetLastError());
+    return copy_out(op->ctx, grad, dg, sizeof(double) * n);
 }
 
 // ------------------------------------------------------------- create_b
@@ -2847,30 +2809,21 @@ int create_b_impl(mfd_ctx *ctx, const mfd::DevGrid &G, int ft, mfd_c64 omega, co
     using namespace mfd;
     int64_t M = G.h.M, n = 3 * M;
     hipStream_t s = ctx->stream;
-    DevArray U;
+    Scratch U;
     int pfull = 0;
     MFD_TRY(upload_param(ctx, G, par, U, &pfull));
     if (pfull) {
         set_error(ft == EE ? "create_b: Pμ must be diagonal (Pμ \\ jₘ)" : "create_b: Pε must be diagonal (Pε \\ jₑ)");
         return MFD_ERR_UNSUPPORTED;
     }
-    void *d = nullptr;
-    MFD_HIP(hipMalloc(&d, sizeof(c64) * 3 * n));
-    c64 *dje = (c64 *)d, *djm = dje + n, *db = djm + n;
-    int rc = MFD_OK;
-    if (hipMemcpyAsync(dje, je, sizeof(c64) * n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(djm, jm, sizeof(c64) * n, hipMemcpyHostToDevice, s) != hipSuccess)
-        rc = MFD_ERR_HIP;
-    if (!rc) {
-        c64 iw = mk<double>(-omega.im, omega.re);
-        int omz = omega.re == 0.0 && omega.im == 0.0;
-        k_create_b<<<(unsigned)((M + BS - 1) / BS), BS, 0, s>>>(G.d64, ft, (const c64 *)U.p, dje, djm, iw, omz, db);
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(b, db, sizeof(c64) * n, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            rc = MFD_ERR_HIP;
-    }
-    if (rc) set_error("create_b failed");
-    hipFree(d);
-    return rc;
+    Scratch d;
+    MFD_TRY(d.get(ctx, sizeof(c64) * 3 * n));
+    c64 *dje = (c64 *)d.p, *djm = dje + n, *db = djm + n;
+    MFD_TRY(copy_in(ctx, dje, je, sizeof(c64) * n));
+    MFD_TRY(copy_in(ctx, djm, jm, sizeof(c64) * n));
+    const c64 iw = mk<double>(-omega.im, omega.re);
+    const int omz = omega.re == 0.0 && omega.im == 0.0;
+    k_create_b<<<(unsigned)((M + BS - 1) / BS), BS, 0, s>>>(G.d64, ft, (const c64 *)U.p, dje, djm, iw, omz, db);
+    MFD_HIP(hipGetLastError());
+    return copy_out(ctx, b, db, sizeof(c64) * n);
 }
