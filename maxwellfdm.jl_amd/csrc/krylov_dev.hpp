@@ -9,7 +9,23 @@ constexpr int NPART = 16384;  // max blocks per reduction (per RHS)
 constexpr int NGRID_MAX = 2048;   // grid cap of the grid-stride vector kernels
 constexpr int BS = 256;
 enum { MODE_A = 0, MODE_P = 1 };
-enum { EPI_STORE = 0, EPI_RESID = 1, EPI_DOT = 2 };
+enum { EPI_STORE = 0, EPI_RESID = 1, EPI_DOT = 2, EPI_BDOT = 3, EPI_XDOT = 4 };
+// one value's share of a stencil's reduction: x the operand, y the result, b the
+// other vector of EPI_BDOT
+template <int EPI>
+__device__ inline void epi_add(double *acc, c64 x, c64 y, c64 b) {
+    if (EPI == EPI_DOT) {          // xᵀy
+        acc[0] += x.re * y.re - x.im * y.im;
+        acc[1] += x.re * y.im + x.im * y.re;
+    } else if (EPI == EPI_BDOT) {  // bᴴy
+        acc[0] += b.re * y.re + b.im * y.im;
+        acc[1] += b.re * y.im - b.im * y.re;
+    } else if (EPI == EPI_XDOT) {  // yᴴx, ‖y‖²
+        acc[0] += y.re * x.re + y.im * x.im;
+        acc[1] += y.re * x.im - y.im * x.re;
+        acc[2] += y.re * y.re + y.im * y.im;
+    }
+}
 
 template <typename R>
 __device__ inline cx<R> czero() { return mk<R>((R)0, (R)0); }

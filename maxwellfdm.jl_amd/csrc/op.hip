@@ -1908,72 +1908,64 @@ __global__ __launch_bounds__(BS) void k_bi_init(DGrid<double> g, OpData<double> 
     if (!act || S.cn == 0.0) { S.conv = 1; S.done = 1; }
 }
 
-// partials of aᴴb (and ‖a‖² when NV = 3)
+// The start of a BiCGSTAB vector kernel with the finish of the product before
+// it folded in: the flags, read once per block (a block never splits on a flag
+// that the lead block sets meanwhile), and the sum of the product's partials in
+// every thread.  False: this right-hand side has nothing to do.
 template <int NV>
-__global__ __launch_bounds__(BS) void k_bi_dot(const c64 *__restrict__ aall, const c64 *__restrict__ ball, int64_t n,
-                                               int64_t vs, double *part, const Scal *scal) {
-    const int rhs = blockIdx.y;
-    const Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
-    const c64 *a = aall + rhs * vs, *b = ball + rhs * vs;
-    double acc[NV];
-    for (int k = 0; k < NV; ++k) acc[k] = 0;
-    for (int64_t e = blockIdx.x * (int64_t)BS + threadIdx.x; e < n; e += (int64_t)gridDim.x * BS) {
-        c64 x = a[e], y = b[e];
-        acc[0] += x.re * y.re + x.im * y.im;
-        acc[1] += x.re * y.im - x.im * y.re;
-        if (NV == 3) acc[2] += x.re * x.re + x.im * x.im;
-    }
-    block_partial<NV>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
+__device__ inline bool bi_sum(const Scal &S, const double *part, int nb, double (&tot)[NV]) {
+    __shared__ int off;
+    __shared__ double bc[NV];
+    if (threadIdx.x == 0) off = S.done || S.conv;
+    __syncthreads();
+    if (off) return false;
+    sum_partials<NV>(part, nb, tot);
+    if (threadIdx.x == 0)
+        for (int a = 0; a < NV; ++a) bc[a] = tot[a];
+    __syncthreads();
+    for (int a = 0; a < NV; ++a) tot[a] = bc[a];
+    return true;
 }
 
-// α = ρ / (r̂ᴴv)
-__global__ __launch_bounds__(BS) void k_bi_fin1(const double *part, int nb, Scal *scal) {
-    const int rhs = blockIdx.x;
-    Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
-    double tot[2];
-    sum_partials<2>(part + (size_t)rhs * NPART * 4, nb, tot);
-    if (threadIdx.x != 0) return;
-    bi_alpha(S, tot);
-}
-
-// s = r − α v
+// α = ρ / (r̂ᴴv), s = r − α v
 __global__ __launch_bounds__(BS) void k_bi_s(c64 *__restrict__ sall, const c64 *__restrict__ rall,
-                                             const c64 *__restrict__ vall, int64_t n, int64_t vs, const Scal *scal) {
+                                             const c64 *__restrict__ vall, int64_t n, int64_t vs, const double *part,
+                                             int nb, Scal *scal) {
     const int rhs = blockIdx.y;
-    const Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
+    Scal &S = scal[rhs];
+    const c64 rho = mk<double>(S.rho_re, S.rho_im);
+    double tot[2];
+    if (!bi_sum<2>(S, part + (size_t)rhs * NPART * 4, nb, tot)) return;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    if (tot[0] == 0.0 && tot[1] == 0.0) {   // breakdown: no step
+        if (lead) bi_alpha(S, tot);
+        return;
+    }
+    const c64 al = cdiv(rho, mk<double>(tot[0], tot[1]));
+    if (lead) bi_alpha(S, tot);
     c64 *s = sall + rhs * vs;
     const c64 *r = rall + rhs * vs, *v = vall + rhs * vs;
-    c64 al = mk<double>(S.alpha_re, S.alpha_im);
     for (int64_t e = blockIdx.x * (int64_t)BS + threadIdx.x; e < n; e += (int64_t)gridDim.x * BS) s[e] = r[e] - al * v[e];
 }
 
-// ω = tᴴs / tᴴt
-__global__ __launch_bounds__(BS) void k_bi_fin2(const double *part, int nb, Scal *scal) {
-    const int rhs = blockIdx.x;
-    Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
-    double tot[3];
-    sum_partials<3>(part + (size_t)rhs * NPART * 4, nb, tot);
-    if (threadIdx.x != 0) return;
-    if (tot[2] == 0.0) { S.om_re = S.om_im = 0; return; }   // t = 0: s is the residual, ω unused
-    S.om_re = tot[0] / tot[2];
-    S.om_im = tot[1] / tot[2];
-}
-
-// x += α p + ω s;  r = s − ω t;  partials of r̂ᴴr and ‖r‖²
+// ω = tᴴs / tᴴt;  x += α p + ω s;  r = s − ω t;  partials of r̂ᴴr and ‖r‖²
 __global__ __launch_bounds__(BS) void k_bi_xr(c64 *__restrict__ xall, c64 *__restrict__ rall,
                                               const c64 *__restrict__ pall, const c64 *__restrict__ sall,
                                               const c64 *__restrict__ tall, const c64 *__restrict__ rhall, int64_t n,
-                                              int64_t vs, double *part, const Scal *scal) {
+                                              int64_t vs, const double *tpart, int nb, double *part, Scal *scal) {
     const int rhs = blockIdx.y;
-    const Scal &S = scal[rhs];
-    if (S.done || S.conv) return;
+    Scal &S = scal[rhs];
+    double tot[3];
+    if (!bi_sum<3>(S, tpart + (size_t)rhs * NPART * 4, nb, tot)) return;
+    // t = 0: s is the residual, ω unused
+    const c64 al = mk<double>(S.alpha_re, S.alpha_im),
+              om = tot[2] == 0.0 ? czero<double>() : mk<double>(tot[0] / tot[2], tot[1] / tot[2]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        S.om_re = om.re;
+        S.om_im = om.im;
+    }
     c64 *x = xall + rhs * vs, *r = rall + rhs * vs;
     const c64 *pp = pall + rhs * vs, *s = sall + rhs * vs, *t = tall + rhs * vs, *rh = rhall + rhs * vs;
-    c64 al = mk<double>(S.alpha_re, S.alpha_im), om = mk<double>(S.om_re, S.om_im);
     double acc[3] = {0, 0, 0};
     for (int64_t e = blockIdx.x * (int64_t)BS + threadIdx.x; e < n; e += (int64_t)gridDim.x * BS) {
         c64 se = s[e];
@@ -2012,22 +2004,23 @@ __global__ __launch_bounds__(BS) void k_bi_p(c64 *__restrict__ pall, const c64 *
         pp[e] = r[e] + be * (pp[e] - om * v[e]);
 }
 
+// One BiCGSTAB step.  The products' inner products are formed in their
+// epilogues and finished by the vector kernels after them, six launches in all.
+// With a kernel for each inner product and each finish it was ten; the four
+// more took 24 µs of a step's 91 on 64×60×72 (now 80): they read 13 MB vectors
+// again and waited, one block, for sums that every block forms in 3 µs.
 static void launch_bicgstab_iter(mfd_op *op, int64_t nrhs) {
     Workspace &w = op->ws;
-    int64_t n = w.n;
+    const int64_t n = w.n;
     hipStream_t s = op->stream;
-    dim3 gv(ngrid(n), (unsigned)nrhs);
+    const dim3 gv = grid_rhs(n, nrhs);
     const size_t ps = (size_t)nrhs * NPART * 4;
     c64 *r = (c64 *)w.r, *rh = (c64 *)w.et, *pp = (c64 *)w.q, *v = (c64 *)w.t, *sv = (c64 *)w.d, *t = (c64 *)w.et2,
         *x = (c64 *)w.z;
-    launch_apply<double, MODE_P, EPI_STORE>(op, pp, v, nullptr, nrhs, nullptr, nullptr, nullptr);
-    k_bi_dot<2><<<gv, BS, 0, s>>>(rh, v, n, n, w.part, w.scal);
-    k_bi_fin1<<<(unsigned)nrhs, BS, 0, s>>>(w.part, (int)gv.x, w.scal);
-    k_bi_s<<<gv, BS, 0, s>>>(sv, r, v, n, n, w.scal);
-    launch_apply<double, MODE_P, EPI_STORE>(op, sv, t, nullptr, nrhs, nullptr, nullptr, nullptr);
-    k_bi_dot<3><<<gv, BS, 0, s>>>(t, sv, n, n, w.part + ps, w.scal);
-    k_bi_fin2<<<(unsigned)nrhs, BS, 0, s>>>(w.part + ps, (int)gv.x, w.scal);
-    k_bi_xr<<<gv, BS, 0, s>>>(x, r, pp, sv, t, rh, n, n, w.part + 2 * ps, w.scal);
+    const int nv = launch_apply<double, MODE_P, EPI_BDOT>(op, pp, v, rh, nrhs, w.part, w.scal, nullptr, nullptr, nullptr, false);
+    k_bi_s<<<gv, BS, 0, s>>>(sv, r, v, n, n, w.part, nv, w.scal);
+    const int nt = launch_apply<double, MODE_P, EPI_XDOT>(op, sv, t, nullptr, nrhs, w.part + ps, w.scal, nullptr, nullptr, nullptr, false);
+    k_bi_xr<<<gv, BS, 0, s>>>(x, r, pp, sv, t, rh, n, n, w.part + ps, nt, w.part + 2 * ps, w.scal);
     k_bi_fin3<<<(unsigned)nrhs, BS, 0, s>>>(w.part + 2 * ps, (int)gv.x, w.scal);
     k_bi_p<<<gv, BS, 0, s>>>(pp, r, v, n, n, w.scal);
 }

@@ -44,6 +44,8 @@ static __global__ __launch_bounds__(BS) void k_fin_resid(const double *part, int
 // y = A x (MODE_A) or y = P x (MODE_P) for the RHS blockIdx.y.
 // EPI_STORE: y = op(x).  EPI_RESID: y = b − op(x), reduce ||y||² into rn.
 // EPI_DOT: y = op(x), reduce xᵀy into the solver scalars (σ, α).
+// EPI_BDOT, EPI_XDOT: y = op(x), partials of bᴴy, and of yᴴx and ‖y‖² (summed
+// by the kernel that uses them).
 // H value from the scratch of k_hpass at (i,j,k) with one index possibly −1
 // or N: the Bloch image times the phase, or zero past a non-Bloch end
 template <typename R>
@@ -99,7 +101,9 @@ __global__ __launch_bounds__(BS) void k_apply(DGrid<R> g, OpData<R> od, const cx
         if (scal[rhs].done) return;
         skip = scal[rhs].conv != 0;
     }
-    double acc[2] = {0.0, 0.0};
+    if ((EPI == EPI_BDOT || EPI == EPI_XDOT) && (scal[rhs].done || scal[rhs].conv)) return;
+    constexpr int NA = EPI == EPI_XDOT ? 3 : 2;
+    double acc[NA] = {};
     if (!skip) {
         for (int64_t p = blockIdx.x * (int64_t)BS + threadIdx.x; p < g.M; p += (int64_t)gridDim.x * BS) {
             int i, j, k;
@@ -183,16 +187,13 @@ __global__ __launch_bounds__(BS) void k_apply(DGrid<R> g, OpData<R> od, const cx
                     acc[0] += (double)rr.re * rr.re + (double)rr.im * rr.im;
                 } else {
                     y[e] = out;
-                    if (EPI == EPI_DOT) {
-                        acc[0] += (double)xu.re * out.re - (double)xu.im * out.im;
-                        acc[1] += (double)xu.re * out.im + (double)xu.im * out.re;
-                    }
+                    epi_add<EPI>(acc, cvt<double>(xu), cvt<double>(out), EPI == EPI_BDOT ? ball[rhs * vs + e] : czero<double>());
                 }
             }
         }
     }
     if (EPI == EPI_STORE) return;
-    block_partial<2>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
+    block_partial<NA>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
 }
 
 // Sparse product for an operator built from a caller's CSC matrix A (stored
@@ -217,7 +218,9 @@ __global__ __launch_bounds__(BS) void k_spmv(int64_t m, const int64_t *__restric
         if (scal[rhs].done) return;
         skip = scal[rhs].conv != 0;
     }
-    double acc[2] = {0.0, 0.0};
+    if ((EPI == EPI_BDOT || EPI == EPI_XDOT) && (scal[rhs].done || scal[rhs].conv)) return;
+    constexpr int NA = EPI == EPI_XDOT ? 3 : 2;
+    double acc[NA] = {};
     const int lane = threadIdx.x % LPR;
     if (!skip) {
         for (int64_t i = (blockIdx.x * (int64_t)BS + threadIdx.x) / LPR; i < m; i += (int64_t)gridDim.x * (BS / LPR)) {
@@ -243,15 +246,12 @@ __global__ __launch_bounds__(BS) void k_spmv(int64_t m, const int64_t *__restric
                 acc[0] += rr.re * rr.re + rr.im * rr.im;
             } else {
                 y[i] = cvt<R>(out);
-                if (EPI == EPI_DOT) {
-                    acc[0] += xi.re * out.re - xi.im * out.im;
-                    acc[1] += xi.re * out.im + xi.im * out.re;
-                }
+                epi_add<EPI>(acc, xi, out, EPI == EPI_BDOT ? ball[rhs * vs + i] : czero<double>());
             }
         }
     }
     if (EPI == EPI_STORE) return;
-    block_partial<2>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
+    block_partial<NA>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
 }
 
 #include "stencil_tiled.hpp"
@@ -350,8 +350,8 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
     const bool two = op->hbuf && op->hbuf_bytes >= sizeof(cx<R>) * (size_t)vs * (size_t)nrhs;
     cx<R> *hb = (cx<R> *)op->hbuf;
     if (two) {
-        if (op->has_mu) k_hpass<R, MODE, true><<<grid, BS, 0, s>>>(g, od, x, hb, vs, scal, EPI == EPI_DOT);
-        else k_hpass<R, MODE, false><<<grid, BS, 0, s>>>(g, od, x, hb, vs, scal, EPI == EPI_DOT);
+        if (op->has_mu) k_hpass<R, MODE, true><<<grid, BS, 0, s>>>(g, od, x, hb, vs, scal, EPI >= EPI_DOT);
+        else k_hpass<R, MODE, false><<<grid, BS, 0, s>>>(g, od, x, hb, vs, scal, EPI >= EPI_DOT);
     }
 #define MFD_DIRECT(OFF, MU_)                                                                                   \
     do {                                                                                                       \

@@ -1,4 +1,4 @@
-// P on FP64 vectors without a reduction (BiCGSTAB, timing).
+// P on FP64 vectors without a reduction (timing).
 #include "stencil_impl.hpp"
 
 namespace mfd {

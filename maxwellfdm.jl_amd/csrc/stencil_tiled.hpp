@@ -204,13 +204,15 @@ __global__ __launch_bounds__(TXW * TY, OFFD ? 2 : 1) void k_apply_tiled(DGrid<do
         if (scal[rhs].done) return;
         skip = scal[rhs].conv != 0;
     }
+    if ((EPI == EPI_BDOT || EPI == EPI_XDOT) && (scal[rhs].done || scal[rhs].conv)) return;
     const int tid = threadIdx.x, tx = tid % C::TX, ty = tid / C::TX;
     const int i0 = bx * C::TX, j0 = by * TY;
     const int i = i0 + tx, j = j0 + ty;
     const bool own = i < g.N[0] && j < g.N[1];
     const int k0 = chunk * KZ, k1 = min(k0 + KZ, g.N[2]);
     const int64_t NxNy = (int64_t)g.N[0] * g.N[1];
-    double acc[2] = {0.0, 0.0};
+    constexpr int NA = EPI == EPI_XDOT ? 3 : 2;
+    double acc[NA] = {};
     // the caller's cell of cell (ci, cj, ck) of g: x-y part and z part
     auto gxy = [&](int ci, int cj) -> int64_t {
         if (REV && (g.rmask & 1)) ci = g.N[0] - 1 - ci;
@@ -632,6 +634,11 @@ __global__ __launch_bounds__(TXW * TY, OFFD ? 2 : 1) void k_apply_tiled(DGrid<do
                     cc[2] = cc[2] - ec[2] * (az_k * (Ps[pn][ty][tx] - p0));
                 }
                 int64_t p = i + (int64_t)g.N[0] * j + NxNy * k;
+                c64 bv[3];
+                if (EPI == EPI_BDOT)   // all three loads ahead of the output's arithmetic
+#pragma unroll
+                    for (int u = 0; u < 3; ++u)
+                        bv[u] = inw(u) ? ball[rhs * vs + dofidx(g, u, REV ? gxy(i, j) + gz(k) : p)] : czero<double>();
                 c64 term[3] = {czero<double>(), czero<double>(), czero<double>()};
                 if (OFFD) {
                     // ∆l weights of the corner averages along each axis: x and y
@@ -718,12 +725,10 @@ __global__ __launch_bounds__(TXW * TY, OFFD ? 2 : 1) void k_apply_tiled(DGrid<do
                         if (yall) y[e] = cvt<R>(rr);   // null output: the residual norm only
                         acc[0] += (double)rr.re * rr.re + (double)rr.im * rr.im;
                     } else {
-                        // the dot product xᵀy is the same in either frame
+                        // products of x and y are the same in either frame
                         y[e] = cvt<R>(rsg(u, out));
-                        if (EPI == EPI_DOT) {
-                            acc[0] += (double)xc[u].re * out.re - (double)xc[u].im * out.im;
-                            acc[1] += (double)xc[u].re * out.im + (double)xc[u].im * out.re;
-                        }
+                        if (EPI == EPI_BDOT) epi_add<EPI>(acc, xc[u], rsg(u, out), bv[u]);
+                        else epi_add<EPI>(acc, xc[u], out, czero<double>());
                     }
                 }
             }
@@ -733,5 +738,5 @@ __global__ __launch_bounds__(TXW * TY, OFFD ? 2 : 1) void k_apply_tiled(DGrid<do
     }
     if (EPI == EPI_STORE) return;
     const int bid = bx + (int)nbx * (by + (int)nby * chunk);
-    block_partial<2>(acc, part + (size_t)rhs * NPART * 4, bid);
+    block_partial<NA>(acc, part + (size_t)rhs * NPART * 4, bid);
 }

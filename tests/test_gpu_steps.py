@@ -54,3 +54,32 @@ def test_launch_tiles(N, scene, pkg):
     z = op.apply(x)
     op.close()
     assert np.abs(y[0] - z).max() <= 1e-15 * np.abs(z).max() and np.abs(y[1] - z[0]).max() <= 1e-15 * np.abs(z).max()
+
+
+@pytest.mark.parametrize("scene", ["diag", "mu", "full"])
+@pytest.mark.parametrize("N", [(13, 9, 11), (66, 5, 7), (36, 21, 1)])
+def test_bicgstab_products(N, scene, pkg, O):
+    """BiCGSTAB, whose inner products end the stencils: every form of the
+    stencil (Bloch phases, reflected axes, both tile widths, the direct kernel,
+    the sparse product), a right-hand side that starts finished (b = 0)."""
+    for bloch, boundft in (((True, True, N[2] == 1), (0, 0, 0)), ((False, False, N[2] == 1), (1, 0, 0)), ((True, False, True), (0, 0, 0))):
+        if scene == "full" and any(boundft):
+            continue
+        m, rng = system(pkg, N, bloch, boundft, scene, 6)
+        pkg.set_kbloch(m, [0.02 * v for v in bloch])
+        A = O.to_scipy(O.create_A(spec_of(m), OM, m.εarr, m.μarr))
+        b = rng.normal(size=(3, A.shape[0])) + 1j * rng.normal(size=(3, A.shape[0]))
+        b[1] = 0
+        ops = [pkg.MaxwellOperator(m, OM)]
+        if scene == "diag":
+            ops.append(pkg.MaxwellOperator.from_csc(A))
+        if not any(boundft):
+            ops.append(pkg.MaxwellOperator(m, OM))
+            ops[-1].set_tile("fp64", 0, 1, 0)
+        for op in ops:
+            say("bicgstab", N, scene, bloch, boundft)
+            e, st = op.solve(b, tol=TOL, method="bicgstab")
+            op.close()
+            assert st.converged and not e[1].any()
+            for r in (0, 2):
+                assert np.linalg.norm(b[r] - A @ e[r]) <= 1.01 * TOL * np.linalg.norm(b[r])
