@@ -255,6 +255,7 @@ __global__ __launch_bounds__(BS) void k_spmv(int64_t m, const int64_t *__restric
 }
 
 #include "stencil_tiled.hpp"
+#include "stencil_plane.hpp"
 
 // finish kernel of a stencil epilogue with a reduction (nb partials per RHS)
 template <int EPI>
@@ -276,6 +277,21 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
         dim3 grid(ngrid(vs), (unsigned)nrhs);
         k_spmv<R, MODE, EPI><<<grid, BS, 0, s>>>(vs, op->csr_rowptr, op->csr_colind, op->csr_val, op->d64.qs,
                                                  op->csr_qo, x, y, b, vs, part, scal, mask);
+        if (after_main) hipEventRecord(after_main, s);
+        if (finish) launch_finish<EPI>(s, (int)grid.x, nrhs, part, scal, rn, mask);
+        return (int)grid.x;
+    }
+    if (plane_ok(op, std::is_same<R, double>::value)) {
+        const DGrid<double> &gp = op->G.d64;
+        const int ntx = (gp.N[0] + PL_TX - 1) / PL_TX;
+        const int64_t nt = ntx * (int64_t)((gp.N[1] + PL_TY - 1) / PL_TY);
+        const dim3 grid((unsigned)std::min<int64_t>(nt, NPART), (unsigned)nrhs);
+#define MFD_PLANE(OFF, TM) \
+    k_apply_plane<R, MODE, EPI, OFF, TM><<<grid, PL_TX * PL_TY, 0, s>>>(gp, op->d64, op->d64.om2, x, y, b, vs, ntx, nt, part, scal, mask)
+        if (gp.nc == 1) MFD_PLANE(false, true);   // corner ε couples Ex and Ey only
+        else if (op->full) MFD_PLANE(true, false);
+        else MFD_PLANE(false, false);
+#undef MFD_PLANE
         if (after_main) hipEventRecord(after_main, s);
         if (finish) launch_finish<EPI>(s, (int)grid.x, nrhs, part, scal, rn, mask);
         return (int)grid.x;

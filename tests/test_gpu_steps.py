@@ -2,6 +2,7 @@
 of one step, which apply every update at once."""
 import numpy as np
 import pytest
+import torch
 
 from conftest import spec_of
 from test_gpu_resident import OM, TOL, say, system
@@ -83,3 +84,58 @@ def test_bicgstab_products(N, scene, pkg, O):
             assert st.converged and not e[1].any()
             for r in (0, 2):
                 assert np.linalg.norm(b[r] - A @ e[r]) <= 1.01 * TOL * np.linalg.norm(b[r])
+
+
+@pytest.mark.parametrize("window", [(0, 2), (2, 1)])
+@pytest.mark.parametrize("N", [(1, 1), (1, 9), (64, 8), (63, 7), (65, 9), (5, 40), (130, 17)])
+def test_plane_stencil(N, window, pkg, O):
+    """The 2D stencil over the edges of its 64 × 4 tiles: the product and the
+    residual norm of a solve against the oracle's A restricted to the window,
+    every combination of ends, with and without ε_xy, FP64 and FP32 vectors."""
+    N = N + (1,)
+    c0, nc = window
+    M = int(np.prod(N))
+    for bloch in ((False, False, True), (True, False, True), (False, True, True), (True, True, True)):
+        for scene in ("diag", "full"):
+            m, rng = system(pkg, N, bloch, (0, 0, 0), scene, 7)
+            m.εarr[..., 0, 2] = m.εarr[..., 2, 0] = m.εarr[..., 1, 2] = m.εarr[..., 2, 1] = 0
+            m.order_cmpfirst = False
+            pkg.set_kbloch(m, [0.02 * bloch[0], 0.03 * bloch[1], 0])
+            A = O.to_scipy(O.create_A(spec_of(m), OM, m.εarr, m.μarr)).tocsr()
+            A = A[c0 * M:(c0 + nc) * M][:, c0 * M:(c0 + nc) * M]
+            x = rng.normal(size=(2, nc * M)) + 1j * rng.normal(size=(2, nc * M))
+            op = pkg.MaxwellOperator(m, OM)
+            op.set_components(c0, nc)
+            say("plane", N, window, bloch, scene)
+            want = np.stack([A @ v for v in x])
+            # a few sums of about ten products each: 1e-13 of the largest, FP32 storage 1e-6
+            assert np.abs(op.apply(x) - want).max() <= 1e-13 * np.abs(want).max()
+            xd = torch.from_numpy(x.astype(np.complex64)).to("cuda")
+            yd = torch.empty_like(xd)
+            torch.cuda.synchronize()
+            op.apply_dev(xd.data_ptr(), yd.data_ptr(), 2, "mixed")
+            want = np.stack([A @ v for v in xd.cpu().numpy().astype(complex)])
+            assert np.abs(yd.cpu().numpy() - want).max() <= 1e-6 * np.abs(want).max()
+            e, st = op.solve(x, tol=TOL, method="bicgstab")
+            op.close()
+            for r in range(2):
+                assert np.linalg.norm(x[r] - A @ e[r]) <= 1.01 * TOL * np.linalg.norm(x[r])
+
+
+def test_plane_steps(pkg, O):
+    """SQMR steps on a plane too large for the resident solver (131,072 cells),
+    FP64 and mixed, against the oracle's A."""
+    N = (431, 350, 1)
+    M = int(np.prod(N))
+    m, rng = system(pkg, N, (False, False, True), (0, 0, 0), "full", 8)
+    m.εarr[..., 0, 2] = m.εarr[..., 2, 0] = m.εarr[..., 1, 2] = m.εarr[..., 2, 1] = 0
+    m.order_cmpfirst = False
+    A = O.to_scipy(O.create_A(spec_of(m), OM, m.εarr, m.μarr)).tocsr()[:2 * M][:, :2 * M]
+    op = pkg.MaxwellOperator(m, OM)
+    op.set_components(0, 2)
+    b = rng.normal(size=2 * M) + 1j * rng.normal(size=2 * M)
+    for precision in ("fp64", "mixed"):
+        say("plane steps", precision)
+        e, st = op.solve(b, tol=TOL, precision=precision)
+        assert st.converged and np.linalg.norm(b - A @ e) <= 1.01 * TOL * np.linalg.norm(b)
+    op.close()
