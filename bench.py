@@ -27,7 +27,7 @@ KERNELS = ("stencil", "upd_r", "upd_dzq")
 KERNEL_NAMES = {  # device kernels as rocprofv3 lists them, template arguments abridged
     "stencil": "k_apply_tiled<{R}, 1, 2, ...> (Krylov stencil, qᵀPq epilogue)",
     "upd_r": "k_upd_r_dot<{R}, ...> (r update, α and ‖r‖², rᵀr)",
-    "upd_dzq": "k_upd_dzq<{R}, ...> (d, z, q update)",
+    "upd_dzq": "k_upd_q<{R}, ...> (q update; d, z of four steps every fourth)",
 }
 
 
@@ -38,7 +38,7 @@ def bytes_per_cell(prec):
     return {
         "stencil": 3 * sc * 2 + 3 * 16,          # read q, write t, read the FP64 complex Jacobi factors
         "upd_r": 3 * sc * 3,                     # read r, t; write r
-        "upd_dzq": 3 * sc * 7,                   # read d, z, q, r; write d, z, q
+        "upd_dzq": 3 * sc * 19 // 4,             # read q, r; write q; every 4th step d, z and 3 more q read, d, z written
     }
 
 

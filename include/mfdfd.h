@@ -256,7 +256,8 @@ int mfd_op_set_tile(mfd_op *op, int prec, int ty, int kz, int xcd_order);
 int mfd_op_bench_apply(mfd_op *op, int64_t nrhs, int prec, int iters, double *ms_per_apply);
 /* Average device time (ms) of each kernel of one SQMR iteration, in launch
  * order: ms[0] stencil with the qᵀPq epilogue, ms[1] r update with its
- * reductions, ms[2] d/z/q update.  Uses (and scribbles over) the solver
+ * reductions, ms[2] q update with its share of the d, z updates (applied every
+ * fourth iteration).  Uses (and scribbles over) the solver
  * workspace.  No reference counterpart. */
 int mfd_op_bench_iteration(mfd_op *op, int64_t nrhs, int prec, int iters, double ms[3]);
 

@@ -1207,7 +1207,8 @@ __global__ void k_bench_scal(Scal *scal, int64_t nrhs) {
 }
 
 // Average duration of each kernel of one SQMR iteration (stencil with the
-// qᵀPq epilogue, r update, d/z/q update), timed in context: `iters` complete
+// qᵀPq epilogue, r update, q update with its share of the d, z updates), timed
+// in context: `iters` complete
 // iterations (finish kernels included) run back to back on the context stream
 // with the solver's workspace and launch shapes, with events around the three
 // main kernels only.

@@ -23,7 +23,7 @@
 //     A' = Cₘ Cₑ − ω² ε − ε G W Div ε,
 // staging Y = ε ∘ X next to X and keeping ψ = W ∘ Div(Y) for planes k and k+1
 // in LDS (G: forward differences to E edges, Div: backward differences to the
-// primal nodes, the same metric as the curls).  Included by op.hip.
+// primal nodes, the same metric as the curls).  Included by stencil_impl.hpp.
 
 template <int TY, int TXW = 64>
 struct TileCfg {
@@ -131,7 +131,7 @@ __device__ inline void plane_init(const DGrid<R> &g, int vk, PlaneZ<R> &z) {
 // unbounded allocation (one wave per SIMD with AGPR overflow) by 24%.
 // OFFD: the ε tensor has corner off-diagonals (xy, xz, yz); their term is
 // formed from the staged planes k−1 (three X_z values kept in registers),
-// k and k+1, with the corner ε read from global memory.
+// k and k+1, with the corner ε staged in LDS.
 // REV: the grid g is the reflection of the operator's grid along the axes of
 // g.rmask (boundft HH there, EE in g) and the kernel works in its
 // coordinates: every per-cell global access (vectors, qs, ε, 1/μ) goes to the
