@@ -126,6 +126,13 @@ __device__ inline void bi_advance(Scal &S, const double (&tot)[3]) {
 
 template <typename R>
 __device__ inline void cell3(const DGrid<R> &g, int64_t p, int &i, int &j, int &k) {
+    if (g.M <= INT32_MAX) {   // a 64-bit division is a few hundred cycles, and there are up to four
+        const uint32_t q = (uint32_t)p, t = q / (uint32_t)g.N[0];
+        i = (int)(q - t * (uint32_t)g.N[0]);
+        k = (int)(t / (uint32_t)g.N[1]);
+        j = (int)(t - (uint32_t)k * (uint32_t)g.N[1]);
+        return;
+    }
     i = (int)(p % g.N[0]);
     int64_t t = p / g.N[0];
     j = (int)(t % g.N[1]);
@@ -133,6 +140,18 @@ __device__ inline void cell3(const DGrid<R> &g, int64_t p, int &i, int &j, int &
 }
 template <typename R>
 __device__ inline void dof2cp(const DGrid<R> &g, int64_t e, int &c, int64_t &p) {
+    if (g.M <= INT32_MAX / 3) {
+        const uint32_t u = (uint32_t)e;
+        if (g.cmpfirst) {
+            p = u / 3;
+            c = (int)(u - 3 * (uint32_t)p);
+        } else {
+            const uint32_t k = u / (uint32_t)g.M;
+            c = g.c0 + (int)k;
+            p = u - k * (uint32_t)g.M;
+        }
+        return;
+    }
     if (g.cmpfirst) { c = (int)(e % 3); p = e / 3; }
     else { const int k = (int)(e / g.M); c = g.c0 + k; p = e - (int64_t)k * g.M; }
 }
