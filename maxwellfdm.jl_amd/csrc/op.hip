@@ -614,13 +614,18 @@ __global__ void k_up(const c32 *a, c64 *b, int64_t n) {
     if (e < n) b[e] = mk<double>((double)a[e].re, (double)a[e].im);
 }
 
+void Workspace::drop_graph() {
+    if (graph) hipGraphExecDestroy(graph);
+    graph = nullptr;
+    graph_iters = 0;
+}
+
 void Workspace::release() {
     if (fixed) {   // caller-provided memory: forget it, free nothing
         *this = Workspace();
         return;
     }
-    if (graph) hipGraphExecDestroy(graph);
-    graph = nullptr;
+    drop_graph();
     if (buf) hipFree(buf);
     buf = nullptr;
     if (scal_h) hipHostFree(scal_h);
@@ -680,6 +685,7 @@ static int hbuf_ensure(mfd_op *op, int64_t nrhs) {
     if (op->hbuf_bytes >= need) return MFD_OK;
     if (op->hbuf) {
         MFD_HIP(hipStreamSynchronize(op->stream));
+        op->ws.drop_graph();   // a kept chunk graph has the scratch's address in its launches
         hipFree(op->hbuf);
         op->hbuf = nullptr;
         op->hbuf_bytes = 0;
@@ -1638,7 +1644,7 @@ static int run_cocg(mfd_op *op, const void *b, void *e, int64_t nrhs, const mfd_
         if (use_graph && (chunk & 1)) ++chunk;   // a replayed graph must end on the parity it starts with
         const int kind = sizeof(R) == 4 ? 2 : 5;
         if (use_graph && (w.graph_iters != chunk || w.graph_kind != kind)) {
-            if (w.graph) { hipGraphExecDestroy(w.graph); w.graph = nullptr; }
+            w.drop_graph();
             hipGraph_t gr;
             MFD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             for (int it = 0; it < chunk; ++it) launch_cocg_iter<R>(op, nrhs, (par + it) & 1);
@@ -1761,8 +1767,7 @@ static int chunk_graph(mfd_op *op, int64_t nrhs, int chunk) {
     Workspace &w = op->ws;
     const int kind = sizeof(R) == 4 ? 1 : 3;
     if (w.graph_iters == chunk && w.graph_kind == kind) return MFD_OK;
-    if (w.graph) { hipGraphExecDestroy(w.graph); w.graph = nullptr; }
-    w.graph_iters = 0;
+    w.drop_graph();
     hipGraph_t gr;
     MFD_HIP(hipStreamBeginCapture(op->stream, hipStreamCaptureModeThreadLocal));
     launch_steps<R>(op, nrhs, chunk);
@@ -2084,7 +2089,7 @@ static int run_inner_bicgstab(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o,
     const long long probe = std::max<long long>(chunk, 2048) / chunk * chunk;
     double cyc_best = HUGE_VAL;   // smallest worst-column probe of this cycle
     if (use_graph && (w.graph_iters != chunk || w.graph_kind != 4)) {
-        if (w.graph) { hipGraphExecDestroy(w.graph); w.graph = nullptr; }
+        w.drop_graph();
         hipGraph_t gr;
         MFD_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         for (int it = 0; it < chunk; ++it) launch_bicgstab_iter(op, nrhs);

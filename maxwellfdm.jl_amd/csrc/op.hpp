@@ -55,6 +55,7 @@ struct Workspace {
     int graph_kind = 0;       // 1/3 = SQMR FP32/FP64, 2 = COCG, 4 = BiCGSTAB iteration
     bool fixed = false;       // memory the solver must not free or reallocate (caller-provided)
     void release();
+    void drop_graph();        // the next solve captures its chunk anew
 };
 
 // Solver workspace layout (op.hip): its size for nrhs right-hand sides of n
