@@ -16,32 +16,26 @@
 //
 // Measured (FP64 SQMR, µs per step, step by step → resident): 16³ 35 → 7.3,
 // 24³ 34 → 7.8, 36³ 37 → 10, 48³ 45 → 13; μ ≠ 1 on 48³ 49 → 15, full ε 70 → 15;
-// FP32 vectors on 64³ 52 → 20.  A step takes 1.3–2 µs longer with two cells per
+// FP32 vectors on 64³ 52 → 16 (19 with d and z in registers and 45 of those spilled).  A step takes 1.3–2 µs longer with two cells per
 // thread than with one, and less with 256 threads of two cells than with 512
 // of one (14.4 → 11.6 µs on 41×36×45: half the waves at each barrier, and the
-// registers hold everything).  1,024 cells per block do not fit the registers
-// with FP64 vectors, 1/μ or corner ε: beyond 256 boxes of 512 cells those
+// registers hold everything).  1,024 cells per block hold FP32 vectors with
+// diagonal ε only, and those with d and z in LDS: no form uses scratch memory.
+// With FP64 vectors, 1/μ or corner ε they spill 90–500 registers, and a trial
+// of 16×8×8 boxes with FP64 vectors (428 spilled registers, 660 bytes of scratch
+// a lane) ended in an illegal memory access.  Its index code, which is that of
+// every form, stays inside all arrays (resident_index.hpp, host_checks.cpp);
+// what else differed was the scratch and a step's end in the step itself, and
+// no cause was shown, so it is not built: beyond 256 boxes of 512 cells those
 // problems run step by step.
 //
 // A block only ever waits for blocks of its own launch, which is cooperative
 // (every block has a place on the chip at once), and gives up after a limit.
 #include "resident.hpp"
+#include "resident_index.hpp"
 #include <algorithm>
 
 namespace mfd {
-
-template <int TX_, int TY_, int TZ_, int CPT_>
-struct BoxCfg {
-    static constexpr int TX = TX_, TY = TY_, TZ = TZ_, CPT = CPT_;   // cells of the box, cells per thread
-    static constexpr bool SLAB = TZ == 1;            // one-cell z axis: no z halo is staged
-    static constexpr int NT = TX * TY * TZ / CPT;    // threads
-    static constexpr int XH = TX + 2, YH = TY + 2, ZH = SLAB ? 1 : TZ + 2;
-    static constexpr int XS = XH * YH * ZH * 3;      // staged values
-    static constexpr int HZ = SLAB ? 0 : 2 * XH * YH, HY = 2 * TZ * XH, HX = 2 * TZ * TY;
-    static constexpr int NHALO = 3 * (HZ + HY + HX); // staged values outside the box
-    static constexpr int NHS = (NHALO + NT - 1) / NT;
-    static constexpr int NTAB = TX + TY + TZ;
-};
 
 template <typename R>
 struct ResArgs {
@@ -176,7 +170,7 @@ __device__ inline void collect(const unsigned long long *slots, int nb, unsigned
 template <typename R, bool OFFD, bool MU, int TX, int TY, int TZ, int CPT>
 __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2) void k_resident(ResArgs<R> A) {
     using C = BoxCfg<TX, TY, TZ, CPT>;
-    constexpr int NT = C::NT, XH = C::XH, YH = C::YH, NHS = C::NHS, NW = NT / 64;
+    constexpr int NT = C::NT, NHS = C::NHS, NW = NT / 64;
     // 1D factors of the box's columns, rows and planes: 1/∆l_D, 1/∆l_P, their
     // products with the plane's and the previous plane's 1/∆l_D (zero past a
     // non-Bloch end, and on a one-cell Bloch axis, where the second difference
@@ -185,10 +179,9 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
     enum { D_ = 0, P_, EP, EM, SD, SP, DM, W0 = DM + (MU ? 1 : 0), W1, NROW = W0 + (OFFD ? 2 : 0) };
     __shared__ c64 Xs[C::XS];
     __shared__ c64 tb[NROW][C::NTAB];
-    // d and z: in LDS while they fit beside the staged box, else in registers
-    constexpr bool DZL = CPT * NT <= 512;
-    constexpr int MX = TX + 1, MY = TY + 1, MZ = C::SLAB ? 1 : TZ + 1;
-    constexpr bool ML = MU && DZL;   // (MU) 1/μ of the box and one cell behind it in LDS
+    constexpr bool DZL = box_dz_lds<C>(sizeof(cx<R>));   // d and z: in LDS, else in registers
+    constexpr int MX = C::MX, MY = C::MY, MZ = C::MZ;
+    constexpr bool ML = MU && CPT * NT <= 512;   // (MU) 1/μ of the box and one cell behind it in LDS
     __shared__ cx<R> Dz[DZL ? 6 * CPT * NT : 1];
     __shared__ c64 Ms[ML ? 3 * MX * MY * MZ : 1];
     __shared__ double sh[NW][3], sh2[NW][3];
@@ -217,61 +210,32 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
             wph[tid] = f(tid % 3, g.phinv[0], g.ph[0]) * f(tid / 3 % 3, g.phinv[1], g.ph[1]) * f(tid / 9, g.phinv[2], g.ph[2]);
         }
     }
-    unsigned long long *slA = A.slots + (size_t)rl * 16 * A.nb, *slB = slA + 8 * A.nb;
+    unsigned long long *slA = A.slots + (size_t)rl * RES_SLOT_WORDS * A.nb, *slB = slA + 8 * A.nb;
     const int bx = box % A.nbx, by = (box / A.nbx) % A.nby, bz = box / (A.nbx * A.nby);
     const int i0 = bx * TX, j0 = by * TY, k0 = bz * TZ;
     const int N0 = g.N[0], N1 = g.N[1], N2 = g.N[2];
     const int64_t off = (int64_t)rhs * A.vs;
     cx<R> *rg = A.r + off, *qg = A.q + off, *dg = A.d + off, *zg = A.z + off;
-    const bool cf = g.cmpfirst != 0;
-    const int Mi = (int)g.M;
-    auto inw = [&](int c) { return (unsigned)(c - g.c0) < (unsigned)g.nc; };
-
-    // the caller's cell of (i, j, k) with its wraps (an index of wph), or −1
-    // for a non-Bloch ghost and beyond
-    auto locate = [&](int i, int j, int k, unsigned &code) -> int {
-        code = 0;
-        bool ok = true;
-        auto wrap = [&](int &v, int N, int a) {
-            const unsigned w = a == 0 ? 1u : (a == 1 ? 3u : 9u);
-            if (v < 0) { ok = ok && g.bloch[a]; v += N; code += w; }
-            else if (v >= N) { ok = ok && g.bloch[a] && v == N; v = 0; code += 2 * w; }
-        };
-        wrap(i, N0, 0);
-        wrap(j, N1, 1);
-        wrap(k, N2, 2);
-        if (g.rmask & 1) i = N0 - 1 - i;
-        if (g.rmask & 2) j = N1 - 1 - j;
-        if (g.rmask & 4) k = N2 - 1 - k;
-        return ok ? i + N0 * (j + N1 * k) : -1;
-    };
+    const BoxIndex<C> ix{N0, N1, N2, g.bloch[0], g.bloch[1], g.bloch[2], g.rmask, A.nbx, A.nby, g.cmpfirst, g.c0, g.nc, (int)g.M};
+    auto inw = [&](int c) { return ix.inw(c); };
     auto phase = [&](c64 v, unsigned code) -> c64 {
-        if (code & 63u) v = v * wph[code & 63u];
+        if (ix.slot_code(code)) v = v * wph[ix.slot_code(code)];
         return v;
     };
     // vector entries by 32-bit byte offset from the (uniform) base
     constexpr unsigned VB = sizeof(cx<R>);
     auto vent = [](auto *base, unsigned o) { return (decltype(base))((char *)base + o); };
     auto vcent = [](const c64 *base, unsigned o) { return *(const c64 *)((const char *)base + o); };
-    // place of component c of the cell at (wrapped) i, j, k among the boxes' r
-    cx<R> *xch = A.xch + (size_t)rl * A.nb * (3 * CPT * NT);
-    auto xidx = [&](int i, int j, int k, int c) -> unsigned {
-        i = i < 0 ? i + N0 : (i >= N0 ? i - N0 : i);
-        j = j < 0 ? j + N1 : (j >= N1 ? j - N1 : j);
-        k = k < 0 ? k + N2 : (k >= N2 ? k - N2 : k);
-        const int bi = i / TX, bj = j / TY, bk = k / TZ;
-        const int cell = i - bi * TX + TX * (j - bj * TY + TY * (k - bk * TZ));
-        return VB * (unsigned)((bi + A.nbx * (bj + A.nby * bk)) * (3 * CPT * NT) + 3 * cell + c);
-    };
-    auto vidx = [&](int p, int c) -> unsigned { return VB * (unsigned)(cf ? 3 * p + c : p + Mi * (c - g.c0)); };
+    cx<R> *xch = A.xch + (size_t)rl * A.nb * (3 * CPT * NT);   // the boxes' r
+    auto xidx = [&](int i, int j, int k, int c) -> unsigned { return VB * ix.xidx(i, j, k, c); };
+    auto vidx = [&](int p, int c) -> unsigned { return VB * (unsigned)ix.vidx(p, c); };
 
     // ---- this thread's cells, CPT neighbours along z (along y on a one-cell z
     // axis); one past a Bloch end (img) stands for its image
-    const int ii = tid % TX;
-    const int jq = C::SLAB ? CPT * (tid / TX) : (tid / TX) % TY, kq = C::SLAB ? 0 : CPT * (tid / (TX * TY));
-    constexpr int UJ = C::SLAB ? 1 : 0, UK = C::SLAB ? 0 : 1;   // step from one of its cells to the next
-    const int at0 = ((C::SLAB ? 0 : (kq + 1) * YH * XH) + (jq + 1) * XH + ii + 1) * 3;
-    constexpr int SX = 3, SY = 3 * XH, SZ = C::SLAB ? 0 : 3 * XH * YH, SU = C::SLAB ? SY : SZ;
+    int ii, jq, kq;
+    ix.first_cell(tid, ii, jq, kq);
+    constexpr int UJ = C::UJ, UK = C::UK, SX = C::SX, SY = C::SY, SZ = C::SZ, SU = C::SU;
+    const int at0 = ix.staged(ii, jq, kq);
     bool own[CPT], img[CPT];
     unsigned mycode[CPT];
     int p[CPT];
@@ -282,7 +246,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
     for (int u = 0; u < CPT; ++u) {
         const int jj = jq + u * UJ, kk = kq + u * UK;
         own[u] = i0 + ii < N0 && j0 + jj < N1 && k0 + kk < N2;
-        p[u] = locate(i0 + ii, j0 + jj, k0 + kk, mycode[u]);
+        p[u] = ix.locate(i0 + ii, j0 + jj, k0 + kk, mycode[u]);
         img[u] = !own[u] && p[u] >= 0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -309,38 +273,17 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
     cx<R> hq[NHS];
 #pragma unroll
     for (int s = 0; s < NHS; ++s) {
-        int h = tid + s * NT, hi, hj, hk, c;
+        const int h = tid + s * NT;
+        int hi, hj, hk, c;
         hoff[s] = hx[s] = 0;
         hpos[s] = 0;
         hq[s] = mk<R>((R)0, (R)0);
         if (h >= C::NHALO) continue;
-        if (h < 3 * C::HZ) {
-            const int pz = h / (3 * XH * YH), f = h - pz * (3 * XH * YH), row = f / (3 * XH);
-            hk = pz ? TZ : -1;
-            hj = row - 1;
-            hi = f - row * (3 * XH);
-            c = hi % 3;
-            hi = hi / 3 - 1;
-        } else if (h < 3 * (C::HZ + C::HY)) {
-            h -= 3 * C::HZ;
-            const int row = h / (3 * XH);
-            hk = row >> 1;
-            hj = (row & 1) ? TY : -1;
-            hi = h - row * (3 * XH);
-            c = hi % 3;
-            hi = hi / 3 - 1;
-        } else {
-            h -= 3 * (C::HZ + C::HY);
-            const int cell = h / 3;
-            c = h - 3 * cell;
-            hi = (cell & 1) ? TX : -1;
-            hk = (cell >> 1) / TY;
-            hj = (cell >> 1) - hk * TY;
-        }
+        ix.halo(h, hi, hj, hk, c);
         unsigned code;
-        const int ph = locate(i0 + hi, j0 + hj, k0 + hk, code);
-        const int lp = ((C::SLAB ? 0 : (hk + 1) * YH * XH) + (hj + 1) * XH + hi + 1) * 3 + c;
-        hpos[s] = 1u << 30 | (unsigned)lp << 8 | (unsigned)c << 6 | code;
+        const int ph = ix.locate(i0 + hi, j0 + hj, k0 + hk, code);
+        const int lp = ix.staged(hi, hj, hk) + c;
+        hpos[s] = ix.pack(lp, c, code);
         if (ph >= 0 && inw(c)) {
             hoff[s] = 16u * (unsigned)(3 * ph + c);
             hx[s] = xidx(i0 + hi, j0 + hj, k0 + hk, c);
@@ -381,23 +324,11 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
                 Xs[at0 + u * SU + c] = phase(neg(c, cvt<double>(q[u][c]) * qs[u][c]), img[u] ? mycode[u] : 0u);
     };
     auto stage_halo = [&](int s, c64 hqs) {
-        const int c = (int)(hpos[s] >> 6) & 3;
-        Xs[(hpos[s] >> 8) & 0xffffu] = phase(neg(c, cvt<double>(hq[s]) * hqs), hpos[s]);
+        const int c = ix.slot_comp(hpos[s]);
+        Xs[ix.slot_place(hpos[s])] = phase(neg(c, cvt<double>(hq[s]) * hqs), hpos[s]);
     };
     auto halo_qs = [&](int s) { return vcent(A.qs, hoff[s]); };
-    // 1/μ at a cell of g (clamped, so that reads past the box's end stay inside)
-    auto mu_at = [&](int x, int y, int w, int c) -> c64 {
-        x = min(x, N0 - 1);
-        y = min(y, N1 - 1);
-        w = min(w, N2 - 1);
-        if (x < 0) x += N0;
-        if (y < 0) y += N1;
-        if (w < 0) w += N2;
-        if (g.rmask & 1) x = N0 - 1 - x;
-        if (g.rmask & 2) y = N1 - 1 - y;
-        if (g.rmask & 4) w = N2 - 1 - w;
-        return A.muinv[3 * (x + N0 * (y + N1 * w)) + c];
-    };
+    auto mu_at = [&](int x, int y, int w, int c) -> c64 { return A.muinv[3 * ix.mu_cell(x, y, w) + c]; };   // 1/μ at a cell of g
     if (ML)
         for (int e = tid; e < 3 * MX * MY * MZ; e += NT) {
             const int cell = e / 3, mi = cell % MX, mj = (cell / MX) % MY, mk_ = cell / (MX * MY);
@@ -488,7 +419,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
                     auto mu = [&](int c, int a) -> c64 {   // 1/μ_c at the cell (a < 0) or one behind along a
                         const int x = tX - (a == 0), y = tY - TX - (a == 1), w = tZ - TX - TY - (a == 2);
                         if (!ML) return mu_at(i0 + x, j0 + y, k0 + w, c);
-                        return Ms[3 * (x + 1 + MX * (y + 1 + MY * (C::SLAB ? 0 : w + 1))) + c];
+                        return Ms[ix.mu_staged(x, y, w) + c];
                     };
                     const c64 hx = mu(0, -1) * (D(tY) * (ld(2, 0, 1, 0) - ld(2, 0, 0, 0)) - D(tZ) * (ld(1, 0, 0, 1) - ld(1, 0, 0, 0)));
                     const c64 hxy = mu(0, 1) * (DMt(tY) * (ld(2, 0, 0, 0) - ld(2, 0, -1, 0)) - D(tZ) * (ld(1, 0, -1, 1) - ld(1, 0, -1, 0)));
@@ -513,9 +444,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
                     // −ω² Σ_w ½ Σ_corners ε_uw · (∆l-weighted mean of X_w along w)
                     const c64 *eo = A.epso;
                     const int i = i0 + tX, j = j0 + tY - TX, k = k0 + tZ - TX - TY, pc = p[u];
-                    const int cpx = i + 1 < N0 ? pc + 1 : (g.bloch[0] ? pc - (N0 - 1) : -1);
-                    const int cpy = j + 1 < N1 ? pc + N0 : (g.bloch[1] ? pc - (N1 - 1) * N0 : -1);
-                    const int cpz = k + 1 < N2 ? pc + N0 * N1 : (g.bloch[2] ? pc - (N2 - 1) * N0 * N1 : -1);
+                    const int cpx = ix.next_x(pc, i), cpy = ix.next_y(pc, j), cpz = ix.next_z(pc, k);
                     const c64 hom = 0.5 * A.om2;
                     const c64 e0 = eo[3 * pc], e1 = eo[3 * pc + 1], e2 = eo[3 * pc + 2];
                     const c64 ax = tb[W0][tX] * ld(0, 0, 0, 0) + tb[W1][tX] * ld(0, -1, 0, 0);
@@ -600,7 +529,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
             for (int u = 0; u < CPT; ++u)
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
-                    xr[3 * (ii + TX * (jq + u * UJ + TY * (kq + u * UK))) + c] = r[u][c];
+                    xr[3 * ix.in_box(ii, jq + u * UJ, kq + u * UK) + c] = r[u][c];
             __syncthreads();
             constexpr int W = VB / 8;
             const unsigned long long *xw = (const unsigned long long *)Xs;
@@ -653,7 +582,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
             if (hpos[s] >> 31) {
                 hq[s] = cvt<R>(cvt<double>(hr[s]) + be * cvt<double>(hq[s]));
                 stage_halo(s, hqs[s]);
-            } else if (hpos[s] >> 30) Xs[(hpos[s] >> 8) & 0xffffu] = mk<double>(0, 0);   // (r went through here)
+            } else if (hpos[s] >> 30) Xs[ix.slot_place(hpos[s])] = mk<double>(0, 0);   // (r went through here)
     }
     __syncthreads();
     if (pend) {   // the last step's end
@@ -718,12 +647,12 @@ static ResPlan res_plan2(const DGrid<double> &g) {
         P.kernel = (const void *)k_resident<R, OFFD, MU, X, Y, Z, CPT>;        \
         P.threads = X * Y * Z / CPT;                                           \
         static const int c = res_capacity(P.kernel, P.threads);                \
-        P.cap = std::min(c, 256);                                              \
+        P.cap = std::min(c, RES_BOXES);                                              \
         shape(X, Y, Z);                                                        \
         if (P.nb <= P.cap) return P;                                           \
     } while (0)
-    // (four cells per thread of FP64 vectors, of 1/μ or of corner ε do not fit
-    // the registers)
+    // (four cells per thread of FP64 vectors, of 1/μ or of corner ε would need
+    // scratch memory: see above)
     constexpr bool FOUR = sizeof(R) == 4 && !MU && !OFFD;
     if (g.N[2] == 1) {
         MFD_RES(16, 8, 1, 1);
@@ -747,23 +676,18 @@ static ResPlan res_plan(const mfd_op *op) {
     return res_plan2<R, false, false>(g);
 }
 
-// Where the boxes exchange r (values per right-hand side: 3 per cell of every
-// box): the second and third slots of the partial sums, which the steps of the
-// resident kernel leave free, or the residual and probe vectors r64, et, et2,
-// free inside a cycle and consecutive; 0: neither has the room.
 template <typename R>
-static int res_xch(const Workspace &w, const ResPlan &P, int64_t n, int64_t nrhs) {
-    const size_t need = sizeof(cx<R>) * 3 * (size_t)P.nb * P.cells;
-    if (need <= 2 * sizeof(double) * NPART * 4) return 1;
-    return need <= 3 * sizeof(c64) * (size_t)n ? 2 : 0;
+static int res_xch(const ResPlan &P, int64_t n) {
+    return res_room(P.nb, P.cells, sizeof(cx<R>), sizeof(double) * NPART * 4, n);
 }
+static_assert(RES_BOXES * RES_SLOT_WORDS * sizeof(unsigned long long) <= sizeof(double) * NPART * 4, "a right-hand side's slots");
 
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs) {
     if (op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
-    if (op->G.d64.M > (1 << 22)) return false;   // 32-bit byte offsets (and far above any capacity)
+    if (op->G.d64.M > RES_MAX_CELLS) return false;
     const ResPlan P = res_plan<R>(op);
-    return P.nb <= P.cap && res_xch<R>(op->ws, P, op->n, nrhs) != 0;
+    return P.nb <= P.cap && res_xch<R>(P, op->n) != 0;
 }
 
 template <typename R>
@@ -791,12 +715,12 @@ int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) 
     A.near = near;
     A.slots = (unsigned long long *)w.part;
     A.scal = w.scal;
-    A.xch = res_xch<R>(w, P, op->n, nrhs) == 1 ? (cx<R> *)(w.part + (size_t)nrhs * NPART * 4) : (cx<R> *)w.r64;
+    A.xch = res_xch<R>(P, op->n) == 1 ? (cx<R> *)(w.part + (size_t)nrhs * NPART * 4) : (cx<R> *)w.r64;
     const int64_t group = std::max(1, P.cap / A.nb);   // right-hand sides per launch
     for (int64_t r0 = 0; r0 < nrhs; r0 += group) {
         const int nr = (int)std::min<int64_t>(group, nrhs - r0);
         A.rhs0 = (int)r0;
-        const int words = nr * 16 * A.nb;
+        const int words = nr * RES_SLOT_WORDS * A.nb;
         k_res_clear<<<(words + 255) / 256, 256, 0, s>>>(A.slots, words);
         void *args[] = {&A};
         MFD_HIP(hipLaunchCooperativeKernel(P.kernel, dim3((unsigned)(nr * A.nb)), dim3((unsigned)P.threads), args, 0, s));
