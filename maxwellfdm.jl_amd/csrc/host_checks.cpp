@@ -1,5 +1,7 @@
 // CPU checks of host- and device-shared integer code (needs no GPU and no HIP):
 //   host_checks resident    the resident solver's index code, every box shape
+//   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs
+//                           whether that many right-hand sides run resident
 // Prints what it covered; a failed check prints itself and ends with status 1.
 #include "resident_index.hpp"
 #include <cstdio>
@@ -220,6 +222,15 @@ static void resident() {
 
 int main(int argc, char **argv) {
     if (argc == 2 && !strcmp(argv[1], "resident")) { resident(); return 0; }
-    printf("usage: host_checks resident\n");
+    if (argc == 13 && !strcmp(argv[1], "pays")) {
+        int v[11];
+        for (int k = 0; k < 11; ++k) v[k] = atoi(argv[2 + k]);
+        int boxes = 1;
+        for (int a = 0; a < 3; ++a) boxes *= (v[3 + a] + v[a] - 1) / v[a];
+        const ResForm f = {v[7] != 0, v[8] != 0, v[9] != 0, v[5] == 1, v[6]};
+        printf("%d\n", (int)res_pays(f, boxes, v[0] * v[1] * v[2], RES_BOXES, (int64_t)v[3] * v[4] * v[5], v[10]));
+        return 0;
+    }
+    printf("usage: host_checks resident | pays ...\n");
     return 2;
 }

@@ -687,7 +687,10 @@ bool resident_ok(const mfd_op *op, int64_t nrhs) {
     if (op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
     if (op->G.d64.M > RES_MAX_CELLS) return false;
     const ResPlan P = res_plan<R>(op);
-    return P.nb <= P.cap && res_xch<R>(P, op->n) != 0;
+    if (P.nb > P.cap || res_xch<R>(P, op->n) == 0) return false;
+    const DGrid<double> &g = op->G.d64;
+    const ResForm f = {sizeof(R) == 8, op->has_mu != 0, op->full != 0, g.N[2] == 1, g.nc};
+    return res_pays(f, P.nb, P.cells, P.cap, g.M, nrhs);
 }
 
 template <typename R>

@@ -4,10 +4,11 @@
 
 namespace mfd {
 
-// Whether nrhs right-hand sides of the operator's system can run resident with
+// Whether nrhs right-hand sides of the operator's system run resident with
 // vectors of storage precision R: the stencil form is built (diagonal or full
-// ε with μ = 1, or μ ≠ 1 with diagonal ε; any boundft, a component window), and
-// every box of one right-hand side has a place on the chip at once.
+// ε with μ = 1, or μ ≠ 1 with diagonal ε; any boundft, a component window),
+// every box of one right-hand side has a place on the chip at once, and the
+// launches that nrhs of them take are faster than the step-by-step kernels.
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs);
 

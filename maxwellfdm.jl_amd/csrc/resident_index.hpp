@@ -157,6 +157,34 @@ MFD_HD inline int res_room(int boxes, int cells, size_t vb, size_t part_bytes, i
     return need <= 3 * 16 * (size_t)n ? 2 : 0;
 }
 
+// Whether nrhs right-hand sides run resident rather than step by step.  Boxes of
+// several right-hand sides that do not share the chip run as one launch after
+// the other, so the resident time of a step grows with the launches; step by
+// step the launches serve all right-hand sides and only the traffic grows.
+// Both sides as measured (µs per step, resident / step by step): 24³ 2 RHS 9.4 /
+// 21.6, 8 36.1 / 31.5, 16 70 / 39; 31×31×32 2 20.4 / 25.1, 4 39.6 / 30.6, 16 157 /
+// 60; 48³ 4 55 / 58, 8 110 / 97; FP32 64³ 2 41 / 48, 4 82 / 71 (1,024 cells a box
+// at 20 µs, 17 since); 180×170 (Ex, Ey) 2 9.9 / 19, 16 57 / 49.  The constants
+// below are fits to 76 systems on 15 grids, 1 to 16 right-hand sides: the choice is the
+// faster one but near the crossing (1.26 times the faster at worst).
+struct ResForm {
+    bool fp64, mu, full;   // vectors; 1/μ, corner ε
+    bool plane;            // one-cell z axis
+    int nc;                // components of the window
+};
+inline bool res_pays(const ResForm &f, int boxes, int box_cells, int cap, int64_t cells, int64_t nrhs) {
+    const bool tensor = f.mu || f.full;
+    const double launch = (f.plane ? (box_cells <= 128 ? 7.6 : (box_cells <= 512 ? 10.2 : 13.8))
+                                   : (box_cells <= 128 ? 9.2 : (box_cells <= 256 ? 10.6 : (box_cells <= 512 ? 13.2 : 17.0)))) *
+                          (tensor ? 1.1 : 1.0);
+    const int64_t per = cap / boxes < 1 ? 1 : cap / boxes, launches = (nrhs + per - 1) / per;
+    // ns per unknown and step of the four kernels: the marching stencil serves a
+    // plane of three components less well, a window's has a kernel of its own
+    const double ns = (f.fp64 ? (tensor ? 0.037 : 0.032) : (tensor ? 0.027 : 0.020)) * (f.plane && f.nc == 3 ? 1.35 : 1.0);
+    const double fixed = f.plane ? 15.5 : (f.full ? 26.0 : 20.0);
+    return (double)launches * launch <= fixed + 1e-3 * ns * (double)(f.nc * cells * nrhs);
+}
+
 // 32-bit byte offsets into the vectors (16 bytes a value) hold up to here
 constexpr int64_t RES_MAX_CELLS = 1 << 22;
 
