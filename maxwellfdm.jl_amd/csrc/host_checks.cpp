@@ -2,8 +2,11 @@
 //   host_checks resident    the resident solver's index code, every box shape
 //   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs
 //                           whether that many right-hand sides run resident
+//   host_checks fit N0 N1 N2 nrhs narrow ty_max reduces ty kz
+//                           the tile made large enough ("no": none is)
 // Prints what it covered; a failed check prints itself and ends with status 1.
 #include "resident_index.hpp"
+#include "tile_rule.hpp"
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -231,6 +234,13 @@ int main(int argc, char **argv) {
         printf("%d\n", (int)res_pays(f, boxes, v[0] * v[1] * v[2], RES_BOXES, (int64_t)v[3] * v[4] * v[5], v[10]));
         return 0;
     }
-    printf("usage: host_checks resident | pays ...\n");
+    if (argc == 11 && !strcmp(argv[1], "fit")) {
+        int v[9];
+        for (int k = 0; k < 9; ++k) v[k] = atoi(argv[2 + k]);
+        if (tile_fit(v, v[3], v[4] != 0, v[5], v[6] != 0, 16384, v[7], v[8])) printf("%d %d\n", v[7], v[8]);
+        else printf("no\n");
+        return 0;
+    }
+    printf("usage: host_checks resident | pays ... | fit ...\n");
     return 2;
 }

@@ -738,9 +738,27 @@ void ws_carve(Workspace &w, void *base, int64_t n, int64_t nrhs) {
     w.graph_iters = 0;
 }
 
+// Whether the partial sums of a solve's stencils have room: the direct kernel
+// takes over where no tile is large enough, but has no grad-div form and no
+// component window
+static bool reductions_fit(const mfd_op *op, int64_t nrhs, int prec) {
+    if (!op->gd && !op->win) return true;
+    for (bool fp64 : {true, false}) {
+        if (!fp64 && prec == MFD_FP64) continue;
+        if (plane_ok(op, fp64)) continue;
+        int ty = 4, kz = 1;
+        if (!tile_fit(op->G.d64.N, nrhs, false, op->gd ? 4 : 8, true, NPART, ty, kz)) return false;
+    }
+    return true;
+}
+
 static int ws_ensure(mfd_op *op, int64_t nrhs, int prec) {
     Workspace &w = op->ws;
     int64_t n = op->n;
+    if (!reductions_fit(op, nrhs, prec)) {
+        set_error("solve: the grid's x-y plane is too large for the grad-div form or a component window");
+        return MFD_ERR_UNSUPPORTED;
+    }
     if (w.fixed) {   // a caller-provided workspace: never reallocated here
         if (w.nrhs != nrhs || w.n != n) { set_error("fixed workspace does not match nrhs"); return MFD_ERR_ARG; }
         w.prec = prec;
@@ -1500,11 +1518,11 @@ static void launch_cocg_iter(mfd_op *op, int64_t nrhs, int par) {
     const DGrid<R> &g = op->G.view<R>();
     // the fused COCG stencil is built 64-wide only: the narrow-tile bit is ignored
     const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
-    const int ty = tile.ty, xr = tile.xr & 1;
-    if (!op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win && ty > 0) {
-        int kz = tile.kz;
-        int nx = (g.N[0] + 63) / 64, ny = (g.N[1] + ty - 1) / ty, nch = (g.N[2] + kz - 1) / kz;
-        while ((int64_t)nx * ny * nch > NPART) { kz *= 2; nch = (g.N[2] + kz - 1) / kz; }
+    const int xr = tile.xr & 1;
+    int ty = tile.ty, kz = tile.kz;
+    if (!op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win && ty > 0 &&
+        tile_fit(op->G.d64.N, nrhs, false, 8, true, NPART, ty, kz)) {
+        const int nx = (g.N[0] + 63) / 64, ny = (g.N[1] + ty - 1) / ty, nch = (g.N[2] + kz - 1) / kz;
         dim3 grid(nx, ny, (unsigned)(nch * nrhs));
         const cx<R> *rr = (const cx<R> *)w.r;
         cx<R> *xi = (cx<R> *)w.z, *t = (cx<R> *)w.t;

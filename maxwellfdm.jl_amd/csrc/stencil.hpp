@@ -1,6 +1,7 @@
 // Launches of the operator's stencils and of the sparse product.
 #pragma once
 #include "krylov_dev.hpp"
+#include "tile_rule.hpp"
 
 namespace mfd {
 
@@ -9,6 +10,13 @@ struct Tile {
     int ty, kz, xr;   // rows, planes, order (bit 0: XCD runs, bit 1: 32-wide); ty = 0: the direct kernel
 };
 Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs);
+
+// a 2D model's window on one plane of cells that k_apply_plane serves
+static inline bool plane_ok(const mfd_op *op, bool fp64) {
+    const DGrid<double> &g = op->G.d64;
+    return op->win && g.N[2] == 1 && g.bloch[2] && g.ph[2].re == 1.0 && g.ph[2].im == 0.0 && op->ee_all &&
+           ((g.c0 == 0 && g.nc == 2) || (g.c0 == 2 && g.nc == 1)) && op->tile_set[fp64 ? 0 : 1] != 1;
+}
 
 // launch one operator apply; returns the number of partial sums per RHS its
 // reduction wrote (finish = false leaves them to the next kernel)

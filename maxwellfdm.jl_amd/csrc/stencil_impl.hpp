@@ -298,17 +298,21 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
     }
     const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
     int ty = tile.ty, kz = tile.kz, xr = tile.xr;
-    if (MODE == MODE_P && op->gd && ty == 8) ty = 4;   // the grad-div tile keeps two more LDS planes
-    // μ ≠ 1 has a tiled form with diagonal ε (the grad-div form is never on with μ)
-    if ((op->ee_all || op->rev) && ty > 0 && !(op->has_mu && op->full)) {
-        // order bit 1: 32-wide tiles of 2·TY rows (same threads per block);
-        // the off-diagonal, grad-div, μ and reflected stencils are built 64-wide only
-        const bool narrow = (xr & 2) && !op->full && !(MODE == MODE_P && op->gd) && !op->has_mu && !op->rev && !op->win;
+    const bool gd = MODE == MODE_P && op->gd;
+    if (gd && ty == 8) ty = 4;   // the grad-div tile keeps two more LDS planes
+    // order bit 1: 32-wide tiles of 2·TY rows (same threads per block);
+    // the off-diagonal, grad-div, μ and reflected stencils are built 64-wide only
+    const bool narrow = (xr & 2) && !op->full && !gd && !op->has_mu && !op->rev && !op->win;
+    // μ ≠ 1 has a tiled form with diagonal ε (the grad-div form is never on with
+    // μ); a grid too large for any tile goes to the direct kernel, which has no
+    // grad-div form or window (ws_ensure refuses the reductions of those)
+    bool tiled = (op->ee_all || op->rev) && ty > 0 && !(op->has_mu && op->full);
+    if (tiled && !tile_fit(op->G.d64.N, nrhs, narrow, gd ? 4 : 8, EPI != EPI_STORE, NPART, ty, kz)) tiled = gd || op->win;
+    if (tiled) {
         xr &= 1;
         const int tw = narrow ? 32 : 64, rows = narrow ? 2 * ty : ty;
         int nx = (g.N[0] + tw - 1) / tw, ny = (g.N[1] + rows - 1) / rows;
         int nch = (g.N[2] + kz - 1) / kz;
-        while ((int64_t)nx * ny * nch > NPART) { kz *= 2; nch = (g.N[2] + kz - 1) / kz; }
         dim3 grid(nx, ny, (unsigned)(nch * nrhs));
         const DGrid<double> &gr = op->G.r64;
         if (op->win && op->full) {   // a component window (2D and 1D models), μ = 1, boundft EE
@@ -336,7 +340,7 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
             else if (ty == 2) k_apply_tiled<R, MODE, EPI, 2, false, false, true><<<grid, 128, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);
             else if (ty == 4) k_apply_tiled<R, MODE, EPI, 4, false, false, true><<<grid, 256, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);
             else k_apply_tiled<R, MODE, EPI, 1, false, false, true><<<grid, 64, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);
-        } else if (MODE == MODE_P && op->gd) {
+        } else if (gd) {
             if (ty == 2) k_apply_tiled<R, MODE, EPI, 2, true><<<grid, 128, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);
             else if (ty == 4) k_apply_tiled<R, MODE, EPI, 4, true><<<grid, 256, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);
             else k_apply_tiled<R, MODE, EPI, 1, true><<<grid, 64, 0, s>>>(op->G.d64, op->d64, op->d64.om2, x, y, b, vs, kz, nch, part, scal, mask, xr);

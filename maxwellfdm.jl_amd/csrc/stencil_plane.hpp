@@ -173,10 +173,3 @@ __global__ __launch_bounds__(PL_TX *PL_TY, 3) void k_apply_plane(DGrid<double> g
     if (EPI == EPI_STORE) return;
     block_partial<NA>(acc, part + (size_t)rhs * NPART * 4, (int)blockIdx.x);
 }
-
-// a 2D model's window on one plane of cells that the kernel above serves
-static inline bool plane_ok(const mfd_op *op, bool fp64) {
-    const DGrid<double> &g = op->G.d64;
-    return op->win && g.N[2] == 1 && g.bloch[2] && g.ph[2].re == 1.0 && g.ph[2].im == 0.0 && op->ee_all &&
-           ((g.c0 == 0 && g.nc == 2) || (g.c0 == 2 && g.nc == 1)) && op->tile_set[fp64 ? 0 : 1] != 1;
-}

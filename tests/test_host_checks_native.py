@@ -68,3 +68,23 @@ def test_resident_rhs(driver, box, N, nc, vectors, scene, nrhs, resident, steps)
     """The faster of the two solvers by the number of right-hand sides."""
     pays = run(driver, "pays", *box, *N, nc, int(vectors == "fp64"), int(scene == "mu"), int(scene == "full"), nrhs).strip()
     assert pays == ("1" if resident < steps else "0")
+
+
+@pytest.mark.parametrize("N,nrhs,narrow,ty_max,reduces,ty,kz,want", [
+    ((128, 128, 128), 1, 0, 8, 1, 4, 16, "4 16"),          # as given
+    ((203, 180, 151), 1, 0, 8, 1, 1, 1, "1 8"),            # 720 tiles a plane
+    ((700, 700, 700), 1, 0, 8, 1, 4, 1, "4 128"),
+    ((2, 174763, 1), 1, 1, 8, 0, 4, 1, "4 1"),             # no partial sums: any number of tiles
+    ((2, 174763, 1), 1, 1, 8, 1, 4, 1, "8 1"),             # one plane: only rows can grow
+    ((2, 174763, 1), 1, 0, 8, 1, 4, 1, "no"),
+    ((2, 174763, 1), 1, 0, 4, 1, 4, 16, "no"),
+    ((4096, 4096, 1), 1, 0, 8, 1, 4, 1, "no"),
+    ((1, 600000, 1), 1, 1, 8, 0, 4, 1, "8 1"),             # rows of tiles beyond a launch's 65,535
+    ((1, 1200000, 1), 1, 1, 8, 0, 4, 1, "no"),
+    ((16, 16, 200), 5000, 0, 8, 1, 4, 4, "4 16"),          # planes times right-hand sides beyond 65,535
+    ((1, 1, 1), 65535, 0, 8, 1, 1, 1, "1 1"),
+])
+def test_tile_fit(driver, N, nrhs, narrow, ty_max, reduces, ty, kz, want):
+    """Tiles of planes too large for the partial sums: the planes were doubled
+    without end, to a division by zero."""
+    assert run(driver, "fit", *N, nrhs, narrow, ty_max, reduces, ty, kz).strip() == want
