@@ -635,43 +635,13 @@ void Workspace::release() {
     nrhs = 0;
 }
 
-// Rows and planes per tile.  The stencils hold two waves per SIMD (their
-// registers), so a CU runs two 4-row blocks or one 8-row block at a time, and
-// a launch takes as many rounds of them as the fullest CU has: with 64×4 tiles
-// of 16 planes 144×120×100 is 630 tiles, three on some CUs, where 20 planes
-// make it 450, two on each.  A block costs its planes and about two more (the
-// first plane's halo and the prologue); one 4-row block alone on a CU takes
-// 0.7 of the time of two (0.5 with μ ≠ 1, where 4-row blocks never share a
-// CU); 8-row blocks read fewer halo rows.  Measured on 14 grids of 52 to 203
-// cells an axis, FP64 and FP32, one and three right-hand sides, against the
-// fastest of 26 to 52 shapes: within 2.5%, where 4 × 16 with planes halved
-// while a launch had fewer than 256 tiles lost up to 20% (µs per step: full ε
-// 144×120×100 330.6 → 274.7, μ ≠ 1 80×76×70 96.2 → 80.0, boundft HEE 100×90×96
-// 127.1 → 107.5, 110×112×90 138.6 → 121.0, 56×58×52 41.7 → 37.8).  More than
-// 20 planes lose again (203×180×151: 24 planes 618 µs, 20 planes 593).
-Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs) {
+// the caller's or the autotuner's shape, or that of tile_rule
+Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode) {
     const int *t = fp64 ? op->tile64 : op->tile32;
     Tile best = {t[0], t[1], t[2]};
     if (best.ty == 0 || op->tile_set[fp64 ? 0 : 1]) return best;
-    const int32_t *N = op->G.d64.N;
-    const bool narrow = (best.xr & 2) != 0;
-    const double alone = op->has_mu || op->gd ? 0.5 : 0.7;
-    double least = 1e300;
-    for (int ty = 8; ty >= 4; ty /= 2) {
-        if (ty == 8 && op->gd) continue;
-        const int rows = narrow ? 2 * ty : ty, per = 8 / ty;   // per: blocks of a CU at a time
-        const int64_t cols = (int64_t)((N[0] + (narrow ? 31 : 63)) / (narrow ? 32 : 64)) * ((N[1] + rows - 1) / rows);
-        for (int kz = 1; kz <= std::min<int>(N[2], 20); ++kz) {
-            const int64_t most = (cols * ((N[2] + kz - 1) / kz) * nrhs + 255) / 256;
-            const double rounds = (double)(most / per) + (most % per ? alone : 0.0);
-            const double cost = rounds * (kz + 2) * (ty == 8 ? 0.97 : 1.0);
-            if (cost < least) {
-                least = cost;
-                best.ty = ty;
-                best.kz = kz;
-            }
-        }
-    }
+    const TileKernel K = {fp64, mode == MODE_A, op->has_mu != 0, op->full != 0, op->gd != 0, op->rev != 0, op->win != 0, (best.xr & 2) != 0};
+    tile_rule(op->G.d64.N, nrhs, K, best.ty, best.kz);
     return best;
 }
 
@@ -1318,7 +1288,7 @@ int op_autotune_impl(mfd_op *op, int64_t nrhs, int iters, int *best64, int *best
     for (int prec = 0; prec < 2; ++prec) {
         int *tile = prec == 0 ? op->tile64 : op->tile32;
         op->tile_set[prec] = 0;
-        const Tile rule = stencil_tile(op, prec == 0, nrhs);   // a candidate as well
+        const Tile rule = stencil_tile(op, prec == 0, nrhs, MODE_P);   // a candidate as well
         op->tile_set[prec] = 2;
         for (int a = -1; a < 4; ++a)
             for (int b = 0; b < (a < 0 ? 1 : 4); ++b)
@@ -1517,7 +1487,7 @@ static void launch_cocg_iter(mfd_op *op, int64_t nrhs, int par) {
     cx<R> *po = cocg_p<R>(w, par), *pn = cocg_p<R>(w, par ^ 1);
     const DGrid<R> &g = op->G.view<R>();
     // the fused COCG stencil is built 64-wide only: the narrow-tile bit is ignored
-    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
+    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs, MODE_P);
     const int xr = tile.xr & 1;
     int ty = tile.ty, kz = tile.kz;
     if (!op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win && ty > 0 &&

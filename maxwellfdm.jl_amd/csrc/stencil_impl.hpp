@@ -296,7 +296,7 @@ int launch_apply(mfd_op *op, const cx<R> *x, cx<R> *y, const c64 *b, int64_t nrh
         if (finish) launch_finish<EPI>(s, (int)grid.x, nrhs, part, scal, rn, mask);
         return (int)grid.x;
     }
-    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs);
+    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs, MODE);
     int ty = tile.ty, kz = tile.kz, xr = tile.xr;
     const bool gd = MODE == MODE_P && op->gd;
     if (gd && ty == 8) ty = 4;   // the grad-div tile keeps two more LDS planes

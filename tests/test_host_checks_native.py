@@ -88,3 +88,31 @@ def test_tile_fit(driver, N, nrhs, narrow, ty_max, reduces, ty, kz, want):
     """Tiles of planes too large for the partial sums: the planes were doubled
     without end, to a division by zero."""
     assert run(driver, "fit", *N, nrhs, narrow, ty_max, reduces, ty, kz).strip() == want
+
+
+# A on one right-hand side (three: last column): µs per apply by (rows, planes) of a tile, measured; the
+# three fastest and 4 × 16
+APPLIES = [
+    ((64, 64, 64), "mu", "fp32", 1, {(8, 2): 25.4, (4, 2): 26.2, (8, 3): 27.3, (4, 16): 57.0}),
+    ((70, 66, 72), "mu", "fp32", 1, {(4, 5): 34.6, (8, 6): 35.0, (4, 6): 36.7, (4, 16): 58.5}),
+    ((56, 100, 41), "mu", "fp32", 3, {(8, 7): 38.2, (4, 7): 38.7, (8, 8): 41.0, (4, 16): 57.4}),
+    ((96, 90, 100), "mu", "fp32", 1, {(8, 10): 47.0, (4, 10): 49.1, (8, 11): 49.7, (4, 16): 66.6}),
+    ((128, 128, 128), "diag", "fp64", 1, {(4, 16): 78.3, (4, 17): 81.5, (8, 16): 82.5}),
+    ((128, 128, 128), "diag", "fp32", 1, {(4, 11): 56.6, (4, 12): 58.3, (4, 13): 59.9, (4, 16): 61.0}),
+    ((110, 112, 90), "full", "fp64", 1, {(4, 10): 72.1, (8, 10): 74.5, (4, 11): 77.1, (4, 16): 92.7}),
+    ((150, 60, 170), "mu", "fp64", 1, {(4, 16): 90.8, (4, 8): 92.7, (4, 5): 93.7}),
+    ((150, 60, 170), "hee", "fp32", 1, {(4, 10): 52.8, (4, 11): 55.2, (4, 12): 57.7, (4, 16): 61.9}),
+    ((190, 33, 120), "mu", "fp64", 1, {(4, 7): 44.7, (4, 8): 46.3, (8, 8): 47.2, (4, 16): 60.3}),
+    ((181, 62, 89), "mu", "fp32", 1, {(8, 9): 46.3, (4, 9): 47.6, (8, 10): 48.4, (4, 16): 66.7}),
+    ((27, 172, 92), "hee", "fp64", 1, {(8, 9): 39.5, (4, 9): 40.8, (8, 10): 41.6, (4, 16): 56.9}),
+]
+
+
+@pytest.mark.parametrize("N,scene,vectors,nrhs,us", APPLIES)
+def test_apply_tiles(driver, N, scene, vectors, nrhs, us):
+    """The rule's tile is one of the fastest three, within 4 % of the fastest."""
+    narrow = scene == "diag" and 64 * -(-N[0] // 64) > 32 * -(-N[0] // 32)
+    pick = run(driver, "tile", *N, nrhs, int(vectors == "fp64"), 1, int(scene == "mu"), int(scene == "full"), 0,
+               int(scene == "hee"), 0, int(narrow))
+    pick = tuple(map(int, pick.split()))
+    assert pick in us and us[pick] <= 1.04 * min(us.values())
