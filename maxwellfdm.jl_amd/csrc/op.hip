@@ -1793,6 +1793,7 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     int chunk = o->check_every > 0 ? o->check_every : 32;
     bool use_graph = o->use_graph != 0;
     const bool res = resident_ok<R>(op, nrhs);
+    if (res && getenv("MFD_SOLVE_TRACE")) resident_trace<R>(op);
     if (use_graph && !res) MFD_TRY(chunk_graph<R>(op, nrhs, chunk));
     long long done_it = 0;
     // FP32 cycles probe the true FP64 residual every `probe` steps and end after

@@ -34,6 +34,7 @@
 #include "resident.hpp"
 #include "resident_index.hpp"
 #include <algorithm>
+#include <cstdio>
 
 namespace mfd {
 
@@ -629,6 +630,7 @@ struct ResPlan {
     const void *kernel = nullptr;
     int nbx = 0, nby = 0, nb = 0, cap = 0;
     int threads = 0, cells = 0;   // per box
+    int box[3] = {0, 0, 0};
 };
 
 // the kernel and boxes for an operator: the smallest boxes that have a place on
@@ -641,6 +643,9 @@ static ResPlan res_plan2(const DGrid<double> &g) {
         P.nby = (g.N[1] + ty - 1) / ty;
         P.nb = P.nbx * P.nby * ((g.N[2] + tz - 1) / tz);
         P.cells = tx * ty * tz;
+        P.box[0] = tx;
+        P.box[1] = ty;
+        P.box[2] = tz;
     };
 #define MFD_RES(X, Y, Z, CPT)                                                  \
     do {                                                                       \
@@ -694,6 +699,13 @@ bool resident_ok(const mfd_op *op, int64_t nrhs) {
 }
 
 template <typename R>
+void resident_trace(const mfd_op *op) {
+    const ResPlan P = res_plan<R>(op);
+    fprintf(stderr, "[mfd resident] %s boxes %dx%dx%d, %d threads, %d boxes\n", sizeof(R) == 8 ? "fp64" : "fp32", P.box[0],
+            P.box[1], P.box[2], P.threads, P.nb);
+}
+
+template <typename R>
 int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) {
     Workspace &w = op->ws;
     hipStream_t s = op->stream;
@@ -733,6 +745,8 @@ int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) 
 
 template bool resident_ok<double>(const mfd_op *, int64_t);
 template bool resident_ok<float>(const mfd_op *, int64_t);
+template void resident_trace<double>(const mfd_op *);
+template void resident_trace<float>(const mfd_op *);
 template int resident_steps<double>(mfd_op *, int64_t, int, int, double);
 template int resident_steps<float>(mfd_op *, int64_t, int, int, double);
 

@@ -12,6 +12,10 @@ namespace mfd {
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs);
 
+// the boxes it runs in, to stderr
+template <typename R>
+void resident_trace(const mfd_op *op);
+
 // Runs up to `steps` SQMR steps on the operator's workspace, on its stream;
 // the state before and after is that between steps (r, q, d, z and the
 // scalars).  After each `chunk` steps a right-hand side also stops when its
