@@ -1,5 +1,6 @@
 // CPU checks of host- and device-shared integer code (needs no GPU and no HIP):
 //   host_checks resident    the resident solver's index code, every box shape
+//   host_checks scal        the store of a right-hand side's scalars
 //   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs
 //                           whether that many right-hand sides run resident
 //   host_checks tile N0 N1 N2 nrhs fp64 apply mu full gd rev win narrow
@@ -8,6 +9,7 @@
 //                           the tile made large enough ("no": none is)
 // Prints what it covered; a failed check prints itself and ends with status 1.
 #include "resident_index.hpp"
+#include "scal.hpp"
 #include "tile_rule.hpp"
 #include <cstdio>
 #include <cstdlib>
@@ -225,8 +227,22 @@ static void resident() {
     printf("resident ok: %ld grids, %ld accesses\n", n_grids, n_accesses);
 }
 
+// a mark set after the scalars were read survives their store; all else is stored
+static void scal() {
+    Scal s, to;
+    memset((void *)&s, 0x5a, sizeof s);
+    memset((void *)&to, 0, sizeof to);
+    to.stag = -1;
+    scal_store(to, s);
+    REQUIRE(to.stag == -1);
+    to.stag = s.stag;
+    REQUIRE(!memcmp((const void *)&to, (const void *)&s, sizeof s));
+    printf("scal ok\n");
+}
+
 int main(int argc, char **argv) {
     if (argc == 2 && !strcmp(argv[1], "resident")) { resident(); return 0; }
+    if (argc == 2 && !strcmp(argv[1], "scal")) { scal(); return 0; }
     if (argc == 13 && !strcmp(argv[1], "pays")) {
         int v[11];
         for (int k = 0; k < 11; ++k) v[k] = atoi(argv[2 + k]);
@@ -251,6 +267,6 @@ int main(int argc, char **argv) {
         else printf("no\n");
         return 0;
     }
-    printf("usage: host_checks resident | pays ... | tile ... | fit ...\n");
+    printf("usage: host_checks resident | scal | pays ... | tile ... | fit ...\n");
     return 2;
 }

@@ -1,24 +1,9 @@
 // Matrix-free operator and device-resident Krylov solver.
 #pragma once
 #include "grid.hpp"
+#include "scal.hpp"
 
 namespace mfd {
-
-// Per-RHS solver scalars, kept on the device.
-struct Scal {
-    double rho_re, rho_im;     // rᵀr (bilinear)
-    double sig_re, sig_im;     // qᵀ P q
-    double alpha_re, alpha_im;
-    double beta_re, beta_im;
-    double tau, theta, cn, target;
-    double c2t2, c2a_re, c2a_im;
-    double rnorm2;             // scratch: last reduced norm²
-    int conv, done, breakdown, stag;
-    long long it, itmax, it_ref;
-    double tau_ref;
-    double apend_re, apend_im;   // COCG: α of the step whose iterate update is still pending
-    double om_re, om_im;         // BiCGSTAB: ω
-};
 
 template <typename R>
 struct OpData {

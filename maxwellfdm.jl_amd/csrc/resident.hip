@@ -591,7 +591,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
         __syncthreads();
         dz_update();
     }
-    if (fail) {   // uniform over the block; the lead's scalars may miss it, the mark does not
+    if (fail) {   // uniform over the block; the solve then ends with an error, whatever the others store
         if (tid == 0) atomicMin(&A.scal[rhs].stag, RESIDENT_TIMEOUT);
         return;
     }
@@ -605,10 +605,7 @@ __global__ __launch_bounds__(TX * TY * TZ / CPT, TX *TY *TZ / CPT <= 256 ? 1 : 2
                 *vent(dg, vidx(p[u], c)) = DZL ? Dz[(6 * u + c) * NT + tid] : d[DZL ? 0 : u][c];
                 *vent(zg, vidx(p[u], c)) = DZL ? Dz[(6 * u + 3 + c) * NT + tid] : z[DZL ? 0 : u][c];
             }
-    if (lead) {
-        S.stag = A.scal[rhs].stag;
-        A.scal[rhs] = S;
-    }
+    if (lead) scal_store(A.scal[rhs], S);
 }
 
 __global__ void k_res_clear(unsigned long long *slots, int n) {

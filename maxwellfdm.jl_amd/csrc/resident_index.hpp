@@ -6,10 +6,12 @@
 #include <cstddef>
 #include <cstdint>
 
+#ifndef MFD_HD
 #ifdef __HIPCC__
 #define MFD_HD __host__ __device__
 #else
 #define MFD_HD
+#endif
 #endif
 
 namespace mfd {

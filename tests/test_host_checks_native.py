@@ -116,3 +116,9 @@ def test_apply_tiles(driver, N, scene, vectors, nrhs, us):
                int(scene == "hee"), 0, int(narrow))
     pick = tuple(map(int, pick.split()))
     assert pick in us and us[pick] <= 1.04 * min(us.values())
+
+
+def test_scal_store(driver):
+    """The lead block of a resident launch stores the scalars without the mark that
+    a block which gave up waiting may set meanwhile."""
+    assert "scal ok" in run(driver, "scal")
