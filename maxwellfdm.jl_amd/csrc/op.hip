@@ -1792,7 +1792,7 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     MFD_HIP(hipGetLastError());
     int chunk = o->check_every > 0 ? o->check_every : 32;
     bool use_graph = o->use_graph != 0;
-    const bool res = resident_ok<R>(op, nrhs);
+    bool res = resident_ok<R>(op, nrhs);
     if (res && getenv("MFD_SOLVE_TRACE")) resident_trace<R>(op);
     if (use_graph && !res) MFD_TRY(chunk_graph<R>(op, nrhs, chunk));
     long long done_it = 0;
@@ -1822,7 +1822,13 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
                 if (p64 && done_it >= next64) near = 3.0 * (tol / cyc_res);
                 steps = resident_span(chunk, done_it, p64 && done_it < next64 ? next64 : 0);
             }
-            MFD_TRY(resident_steps<R>(op, nrhs, steps, chunk, near));
+            const int rc = resident_steps<R>(op, nrhs, steps, chunk, near);
+            if (rc == RESIDENT_REFUSED) {   // nothing ran (or whole groups of right-hand sides did): go on step by step
+                res = false;
+                if (use_graph) MFD_TRY(chunk_graph<R>(op, nrhs, chunk));
+                continue;
+            }
+            MFD_TRY(rc);
         } else if (use_graph) MFD_HIP(hipGraphLaunch(w.graph, s));
         else launch_steps<R>(op, nrhs, chunk);
         MFD_HIP(hipGetLastError());
@@ -2487,6 +2493,7 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
                         r = resident_steps<double>(B.op, 1, resident_span(chunk, B.it_seen, look ? 0 : B.next64), chunk,
                                                    look ? 3.0 * o.tol / B.worst : 0.0);
                     }
+                    if (r == RESIDENT_REFUSED) r = MFD_OK;   // step by step from the next round
                 } else {
                     r = B.prec == MFD_MIXED ? chunk_graph<float>(B.op, 1, chunk) : chunk_graph<double>(B.op, 1, chunk);
                     if (!r) BCHK(hipGraphLaunch(B.op->ws.graph, s));

@@ -34,6 +34,7 @@
 #include "resident.hpp"
 #include "resident_index.hpp"
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 
 namespace mfd {
@@ -613,13 +614,21 @@ __global__ void k_res_clear(unsigned long long *slots, int n) {
     if (i < n) slots[i] = 0;
 }
 
-// boxes of one right-hand side that can be resident at once
-static int res_capacity(const void *kernel, int threads) {
-    int per = 0, dev = 0, cus = 0, coop = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
-        !coop || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess)
+constexpr int RES_DEVICES = 64;   // whose capacity is kept
+
+// blocks that can be resident on the current device at once (0: none, or the
+// query failed, which is not kept)
+static int res_capacity(std::atomic<int> *known, int dev, const void *kernel, int threads) {
+    if (dev >= 0 && dev < RES_DEVICES)
+        if (const int c = known[dev].load(std::memory_order_relaxed)) return c;
+    int per = 0, cus = 0, coop = 0;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess) {
+        hipGetLastError();
         return 0;
+    }
+    if (dev >= 0 && dev < RES_DEVICES) known[dev].store(per * cus, std::memory_order_relaxed);
     return per * cus;
 }
 
@@ -633,7 +642,7 @@ struct ResPlan {
 // the kernel and boxes for an operator: the smallest boxes that have a place on
 // the chip each
 template <typename R, bool OFFD, bool MU>
-static ResPlan res_plan2(const DGrid<double> &g) {
+static ResPlan res_plan2(const DGrid<double> &g, int dev) {
     ResPlan P;
     auto shape = [&](int tx, int ty, int tz) {
         P.nbx = (g.N[0] + tx - 1) / tx;
@@ -648,8 +657,8 @@ static ResPlan res_plan2(const DGrid<double> &g) {
     do {                                                                       \
         P.kernel = (const void *)k_resident<R, OFFD, MU, X, Y, Z, CPT>;        \
         P.threads = X * Y * Z / CPT;                                           \
-        static const int c = res_capacity(P.kernel, P.threads);                \
-        P.cap = std::min(c, RES_BOXES);                                              \
+        static std::atomic<int> known[RES_DEVICES];                            \
+        P.cap = std::min(res_capacity(known, dev, P.kernel, P.threads), RES_BOXES); \
         shape(X, Y, Z);                                                        \
         if (P.nb <= P.cap) return P;                                           \
     } while (0)
@@ -673,9 +682,10 @@ static ResPlan res_plan2(const DGrid<double> &g) {
 template <typename R>
 static ResPlan res_plan(const mfd_op *op) {
     const DGrid<double> &g = op->G.d64;
-    if (op->full) return res_plan2<R, true, false>(g);
-    if (op->has_mu) return res_plan2<R, false, true>(g);
-    return res_plan2<R, false, false>(g);
+    const int dev = op->ctx->device;
+    if (op->full) return res_plan2<R, true, false>(g, dev);
+    if (op->has_mu) return res_plan2<R, false, true>(g, dev);
+    return res_plan2<R, false, false>(g, dev);
 }
 
 template <typename R>
@@ -686,7 +696,7 @@ static_assert(RES_BOXES * RES_SLOT_WORDS * sizeof(unsigned long long) <= sizeof(
 
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs) {
-    if (op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
+    if (op->res_off || op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
     if (op->G.d64.M > RES_MAX_CELLS) return false;
     const ResPlan P = res_plan<R>(op);
     if (P.nb > P.cap || res_xch<R>(P, op->n) == 0) return false;
@@ -735,7 +745,13 @@ int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) 
         const int words = nr * RES_SLOT_WORDS * A.nb;
         k_res_clear<<<(words + 255) / 256, 256, 0, s>>>(A.slots, words);
         void *args[] = {&A};
-        MFD_HIP(hipLaunchCooperativeKernel(P.kernel, dim3((unsigned)(nr * A.nb)), dim3((unsigned)P.threads), args, 0, s));
+        const hipError_t e = hipLaunchCooperativeKernel(P.kernel, dim3((unsigned)(nr * A.nb)), dim3((unsigned)P.threads), args, 0, s);
+        if (e == hipErrorCooperativeLaunchTooLarge) {
+            hipGetLastError();
+            op->res_off = 1;
+            return RESIDENT_REFUSED;
+        }
+        MFD_HIP(e);
     }
     return MFD_OK;
 }

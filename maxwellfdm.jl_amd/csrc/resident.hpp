@@ -23,7 +23,10 @@ void resident_trace(const mfd_op *op);
 template <typename R>
 int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near);
 
-// Scal::stag of a right-hand side whose blocks gave up waiting for each other
-enum { RESIDENT_TIMEOUT = -1 };
+// Scal::stag of a right-hand side whose blocks gave up waiting for each other;
+// what resident_steps returns when the device refused the launch (fewer places
+// than it reported): the state is still that between steps, resident_ok is
+// false from then on, and the step-by-step kernels go on
+enum { RESIDENT_TIMEOUT = -1, RESIDENT_REFUSED = -2 };
 
 }  // namespace mfd

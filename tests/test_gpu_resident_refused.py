@@ -1,0 +1,64 @@
+"""A device that refuses the resident solver's cooperative launch: the solve goes
+on step by step.  The refusal is the host's: a library loaded before libmfdfd
+answers the launch with the runtime's error and starts nothing."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+pytestmark = pytest.mark.gpu
+
+SHIM = """
+int calls = 0;
+int hipLaunchCooperativeKernel(const void *f, ...) { (void)f; ++calls; return 720; }   /* hipErrorCooperativeLaunchTooLarge */
+"""
+
+PROGRAM = """
+import ctypes as C, os, sys
+shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+for p in ("maxwellfdm.jl_amd", "oracle", "tests"):
+    sys.path.insert(0, os.path.join(sys.argv[2], p))
+import numpy as np
+import maxwellfdfd as pkg, oracle as O
+from conftest import spec_of
+from test_gpu_resident import OM, TOL, system
+made = []
+for N in ((13, 9, 11), (10, 12, 7)):
+    m, rng = system(pkg, N, (False,) * 3, (0, 0, 0), "diag", 51)
+    made.append((pkg.MaxwellOperator(m, OM), O.to_scipy(O.create_A(spec_of(m), OM, m.εarr, m.μarr)), rng))
+def check(A, b, e):
+    assert np.linalg.norm(b - A @ e) <= 1.01 * TOL * np.linalg.norm(b)
+def calls():
+    return C.c_int.in_dll(shim, "calls").value
+op, A, rng = made[0]
+for precision in ("fp64", "mixed"):
+    b = rng.normal(size=(2, A.shape[0])) + 1j * rng.normal(size=(2, A.shape[0]))
+    for rhs in (b[0], b):
+        e, st = op.solve(rhs, tol=TOL, precision=precision)
+        for r, x in zip(np.atleast_2d(rhs), np.atleast_2d(e)):
+            check(A, r, x)
+print("single ok", calls(), flush=True)
+assert calls() == 1          # the operator does not ask again
+op.close()
+m, rng = system(pkg, (13, 9, 11), (False,) * 3, (0, 0, 0), "diag", 51)
+made[0] = (pkg.MaxwellOperator(m, OM), A, rng)
+bs = [rng.normal(size=A.shape[0]) + 0j for _, A, rng in made]
+es, _ = pkg.solve_batch([op for op, _, _ in made], bs, tol=TOL)
+for (_, A, _), b, e in zip(made, bs, es):
+    check(A, b, e)
+assert calls() == 3
+print("batch ok", flush=True)
+"""
+
+
+def test_refused(tmp_path):
+    c, so, py = tmp_path / "refuse.c", tmp_path / "librefuse.so", tmp_path / "program.py"
+    c.write_text(SHIM)
+    py.write_text(PROGRAM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(c)], check=True)
+    p = subprocess.run([sys.executable, "-u", str(py), str(so), ROOT], capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, PYTHONDONTWRITEBYTECODE="1"))
+    assert p.returncode == 0 and "batch ok" in p.stdout, p.stdout + p.stderr
