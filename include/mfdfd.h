@@ -237,8 +237,12 @@ int mfd_op_set_components(mfd_op *op, int c0, int nc);
  * ε is diagonal and the x size is not a multiple of 64): times each
  * candidate inside complete solver iterations for nrhs
  * right-hand sides (iters of them, on the solver workspace) and keeps the one
- * with the fastest iteration per precision; ms[] is that iteration time.
- * Outputs may be null.  No reference counterpart. */
+ * with the fastest iteration per precision; ms[] is that iteration time.  A 2D
+ * model's window ((Ex, Ey) or Ez on one periodic plane) runs a kernel without
+ * tiles: its iteration is timed once and the shape is the default rule's.
+ * Systems that solve in one kernel (mfd_op_set_tile) are tuned too, for their
+ * applies, COCG, BiCGSTAB and many right-hand sides; the shape and ms[] say
+ * nothing of their SQMR solves.  Outputs may be null.  No reference counterpart. */
 int mfd_op_autotune(mfd_op *op, int64_t nrhs, int iters, int tile64[3], int tile32[3], double ms[2]);
 /* Fix the tile shape by hand: TY in {1,2,4,8} (0 = cache-reliant direct
  * kernel; MFD_ERR_UNSUPPORTED with a component window), KZ >= 1, xcd_order

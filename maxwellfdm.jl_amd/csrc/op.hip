@@ -640,7 +640,8 @@ Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode) {
     const int *t = fp64 ? op->tile64 : op->tile32;
     Tile best = {t[0], t[1], t[2]};
     if (best.ty == 0 || op->tile_set[fp64 ? 0 : 1]) return best;
-    const TileKernel K = {fp64, mode == MODE_A, op->has_mu != 0, op->full != 0, op->gd != 0, op->rev != 0, op->win != 0, (best.xr & 2) != 0};
+    TileKernel K = {fp64, mode == MODE_A, op->has_mu != 0, op->full != 0, op->gd != 0, op->rev != 0, op->win != 0, false};
+    K.narrow = (best.xr & 2) && !K.mu && !K.full && !(K.gd && !K.apply) && !K.rev && !K.win;   // as launch_apply takes it
     tile_rule(op->G.d64.N, nrhs, K, best.ty, best.kz);
     return best;
 }
@@ -1285,17 +1286,23 @@ int op_autotune_impl(mfd_op *op, int64_t nrhs, int iters, int *best64, int *best
     double bestms[2] = {1e30, 1e30};
     int bt[2][3] = {{4, 16, 1}, {4, 16, 1}};
     const int its = std::max(2, std::min(iters, 50));
-    for (int prec = 0; prec < 2; ++prec) {
+    const int old[2][4] = {{op->tile64[0], op->tile64[1], op->tile64[2], op->tile_set[0]},
+                           {op->tile32[0], op->tile32[1], op->tile32[2], op->tile_set[1]}};
+    auto one = [&](int prec) -> int {
         int *tile = prec == 0 ? op->tile64 : op->tile32;
+        if (tile[0] == 0) tile[0] = 4;   // (the direct kernel set by hand)
         op->tile_set[prec] = 0;
         const Tile rule = stencil_tile(op, prec == 0, nrhs, MODE_P);   // a candidate as well
-        op->tile_set[prec] = 2;
-        for (int a = -1; a < 4; ++a)
+        // a 2D model's window that k_apply_plane serves runs no tiles: timed once,
+        // and the rule's shape stands
+        const bool tiles = !plane_ok(op, prec == 0);
+        if (tiles) op->tile_set[prec] = 2;
+        for (int a = -1; a < (tiles ? 4 : 0); ++a)
             for (int b = 0; b < (a < 0 ? 1 : 4); ++b)
-                for (int xo = 0; xo < norders; ++xo) {
+                for (int xo = 0; xo < (tiles ? norders : 1); ++xo) {
                     tile[0] = a < 0 ? rule.ty : tys[a];
                     tile[1] = a < 0 ? rule.kz : kzs[b];
-                    tile[2] = xo;
+                    tile[2] = tiles ? xo : rule.xr;
                     double part[3] = {0, 0, 0};
                     MFD_TRY(op_bench_iteration_impl(op, nrhs, prec == 0 ? MFD_FP64 : MFD_MIXED, its, part));
                     const double ms = part[0] + part[1] + part[2];
@@ -1304,7 +1311,19 @@ int op_autotune_impl(mfd_op *op, int64_t nrhs, int iters, int *best64, int *best
                         for (int k = 0; k < 3; ++k) bt[prec][k] = tile[k];
                     }
                 }
-    }
+        return MFD_OK;
+    };
+    for (int prec = 0; prec < 2; ++prec)
+        if (const int rc = one(prec)) {   // the shapes are those of before
+            for (int k = 0; k < 3; ++k) {
+                op->tile64[k] = old[0][k];
+                op->tile32[k] = old[1][k];
+            }
+            op->tile_set[0] = old[0][3];
+            op->tile_set[1] = old[1][3];
+            op->ws.release();
+            return rc;
+        }
     for (int k = 0; k < 3; ++k) {
         op->tile64[k] = bt[0][k];
         op->tile32[k] = bt[1][k];
