@@ -623,7 +623,7 @@ int csc_upload(mfd_ctx *ctx, const mfd_csc *h, const char *name, DevCsc &d) {
     const size_t bcp = sizeof(int64_t) * (h->n + 1), brv = sizeof(int64_t) * h->nnz, bnz = sizeof(c64) * h->nnz;
     const size_t off_rv = (bcp + 255) / 256 * 256, off_nz = off_rv + (brv + 255) / 256 * 256;
     const size_t off_fl = off_nz + (bnz + 255) / 256 * 256;
-    MFD_HIP(hipMalloc(&d.buf, off_fl + 256));
+    MFD_HIP(ctx_malloc(ctx, &d.buf, off_fl + 256));
     d.m = h->m;
     d.n = h->n;
     d.nnz = h->nnz;
@@ -765,7 +765,7 @@ int csr_of(mfd_ctx *ctx, const DevCsc &A, DevCsr &R) {
     const size_t brp = sizeof(int64_t) * (m + 1), bci = sizeof(int32_t) * nnz, bv = sizeof(c64) * nnz;
     const size_t off_ci = (brp + 255) / 256 * 256, off_v = off_ci + (bci + 255) / 256 * 256;
     const size_t off_c = off_v + (bv + 255) / 256 * 256;
-    MFD_HIP(hipMalloc(&R.buf, off_c + brp + 256));
+    MFD_HIP(ctx_malloc(ctx, &R.buf, off_c + brp + 256));
     R.m = m;
     R.n = A.n;
     R.nnz = nnz;
@@ -778,7 +778,7 @@ int csr_of(mfd_ctx *ctx, const DevCsc &A, DevCsr &R) {
     size_t tmpb = 0;
     hipcub::DeviceScan::ExclusiveSum(nullptr, tmpb, rc, R.rowptr, m + 1, s);
     void *tmp = nullptr;
-    MFD_HIP(hipMalloc(&tmp, tmpb ? tmpb : 1));
+    MFD_HIP(ctx_malloc(ctx, &tmp, tmpb ? tmpb : 1));
     hipcub::DeviceScan::ExclusiveSum(tmp, tmpb, rc, R.rowptr, m + 1, s);
     hipError_t e = hipStreamSynchronize(s);
     hipFree(tmp);

@@ -88,7 +88,7 @@ int mfd_ctx_destroy(mfd_ctx *ctx) {
 int mfd_stretched_dl(mfd_ctx *ctx, const mfd_grid *g, mfd_c64 *out) {
     CHECK_CTX(ctx);
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     MFD_HIP(hipMemcpy(out, G.sdl64, sizeof(c64) * G.total, hipMemcpyDeviceToHost));
     return MFD_OK;
 }
@@ -208,7 +208,7 @@ int mfd_curl_nnz(mfd_ctx *ctx, const mfd_grid *g, int which, int64_t *nnz) {
     CHECK_CTX(ctx);
     if (which != 0 && which != 1) { set_error("which must be 0 (Cₑ) or 1 (Cₘ)"); return MFD_ERR_ARG; }
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     return curl_csc(ctx, G, which, nnz, nullptr, nullptr, nullptr);
 }
 
@@ -217,7 +217,7 @@ int mfd_curl_csc(mfd_ctx *ctx, const mfd_grid *g, int which, int64_t *colptr, in
     if (which != 0 && which != 1) { set_error("which must be 0 (Cₑ) or 1 (Cₘ)"); return MFD_ERR_ARG; }
     if (!colptr || !rowval || !nzval) { set_error("null output buffer"); return MFD_ERR_ARG; }
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     int64_t nnz;
     return curl_csc(ctx, G, which, &nnz, colptr, rowval, nzval);
 }
@@ -226,7 +226,7 @@ int mfd_Mcs_nnz(mfd_ctx *ctx, const mfd_grid *g, int which, int64_t *nnz) {
     CHECK_CTX(ctx);
     if (which != 0 && which != 1) { set_error("which must be 0 (Mcₑ) or 1 (Mcₘ)"); return MFD_ERR_ARG; }
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     return mean_csc(ctx, G, which, nnz, nullptr, nullptr, nullptr);
 }
 
@@ -235,7 +235,7 @@ int mfd_Mcs_csc(mfd_ctx *ctx, const mfd_grid *g, int which, int64_t *colptr, int
     if (which != 0 && which != 1) { set_error("which must be 0 (Mcₑ) or 1 (Mcₘ)"); return MFD_ERR_ARG; }
     if (!colptr || !rowval || !nzval) { set_error("null output buffer"); return MFD_ERR_ARG; }
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     int64_t nnz;
     return mean_csc(ctx, G, which, &nnz, colptr, rowval, nzval);
 }
@@ -249,7 +249,7 @@ int mfd_matparams(mfd_ctx *ctx, const mfd_grid *g, int64_t nobj, const mfd_shape
 int mfd_paramop_nnz(mfd_ctx *ctx, const mfd_grid *g, int which, const mfd_c64 *parr, int64_t *nnz) {
     CHECK_CTX(ctx);
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     return param_csc(ctx, G, which, parr, nnz, nullptr, nullptr, nullptr);
 }
 
@@ -257,7 +257,7 @@ int mfd_paramop_csc(mfd_ctx *ctx, const mfd_grid *g, int which, const mfd_c64 *p
                     int64_t *rowval, mfd_c64 *nzval) {
     CHECK_CTX(ctx);
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     int64_t nnz;
     return param_csc(ctx, G, which, parr, &nnz, colptr, rowval, nzval);
 }
@@ -273,7 +273,7 @@ int mfd_A_nnz(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const mfd_
     CHECK_CTX(ctx);
     MFD_TRY(ft_check(ft));
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     return A_csc(ctx, G, ft, omega, eps_arr, mu_arr, nnz, nullptr, nullptr, nullptr);
 }
 
@@ -282,7 +282,7 @@ int mfd_A_csc(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const mfd_
     CHECK_CTX(ctx);
     MFD_TRY(ft_check(ft));
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     int64_t nnz;
     return A_csc(ctx, G, ft, omega, eps_arr, mu_arr, &nnz, colptr, rowval, nzval);
 }
@@ -292,7 +292,7 @@ int mfd_create_b(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const m
     CHECK_CTX(ctx);
     MFD_TRY(ft_check(ft));
     DevGrid G;
-    MFD_TRY(G.create(g, ctx->stream));
+    MFD_TRY(G.create(g, ctx));
     return create_b_impl(ctx, G, ft, omega, ft == MFD_EE ? mu_arr : eps_arr, je, jm, b);
 }
 

@@ -7,6 +7,7 @@
 // ghost at the negative end; ∆l[PRIM] = diff(dual incl. ghost),
 // ∆l[DUAL] = diff(primal incl. ghost).
 #include "grid.hpp"
+#include "ctxmem.hpp"
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -166,9 +167,10 @@ __global__ void k_reflect_tables(ReflectArgs a, int64_t tot, const c64 *s0, cons
     d3[e] = s3[src];
 }
 
-int DevGrid::reflect(int mask, hipStream_t stream) {
+int DevGrid::reflect(int mask, mfd_ctx *ctx) {
     if (rbuf) return MFD_OK;
-    MFD_HIP(hipMalloc(&rbuf, sizeof(c64) * 4 * total));
+    const hipStream_t stream = ctx->stream;
+    MFD_HIP(ctx_malloc(ctx, &rbuf, sizeof(c64) * 4 * total));
     c64 *dst[4];
     for (int k = 0; k < 4; ++k) dst[k] = (c64 *)rbuf + k * total;
     ReflectArgs a;
@@ -206,14 +208,15 @@ int DevGrid::reflect(int mask, hipStream_t stream) {
     return MFD_OK;
 }
 
-int DevGrid::create(const mfd_grid *g, hipStream_t stream) {
+int DevGrid::create(const mfd_grid *g, mfd_ctx *ctx) {
+    const hipStream_t stream = ctx->stream;
     MFD_TRY(build_hgrid(g, &h));
     int64_t tot = 2 * (h.N[0] + h.N[1] + h.N[2]);
     total = tot;
     // device layout: positions, dl, lprim (double); 4 complex double tables; 4 complex float tables
     int64_t nl = h.N[0] + h.N[1] + h.N[2] + 3;
     size_t bytes = sizeof(double) * (2 * tot + nl) + sizeof(c64) * 4 * tot + sizeof(c32) * 4 * tot + 256;
-    MFD_HIP(hipMalloc(&buf, bytes));
+    MFD_HIP(ctx_malloc(ctx, &buf, bytes));
     char *p = (char *)buf;
     double *pos = (double *)p; p += sizeof(double) * tot;
     double *dl = (double *)p; p += sizeof(double) * tot;

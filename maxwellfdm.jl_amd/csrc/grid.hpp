@@ -24,8 +24,8 @@ struct DevGrid {
     // Built by reflect(); null tables until then.
     DGrid<double> r64;
     void *rbuf = nullptr;
-    int create(const mfd_grid *g, hipStream_t stream);
-    int reflect(int mask, hipStream_t stream);
+    int create(const mfd_grid *g, mfd_ctx *ctx);
+    int reflect(int mask, mfd_ctx *ctx);
     void release();
     ~DevGrid();
     template <typename R> const DGrid<R> &view() const;

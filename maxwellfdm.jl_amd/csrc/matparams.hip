@@ -15,6 +15,7 @@
 //     foreground shape's nearest surface point, normal from the same point;
 //     three or more objects give the plain mean of the 8 corner tensors.
 #include "matparams.hpp"
+#include "ctxmem.hpp"
 
 namespace mfd {
 
@@ -286,7 +287,7 @@ int matparams(mfd_ctx *ctx, const mfd_grid *g, int64_t nobj, const mfd_shape *sh
     size_t bytes = sizeof(double) * ncoord + sizeof(DShape) * ds.size() + sizeof(c64) * 18 * (nobj > 0 ? nobj : 1) +
                    sizeof(int) * 8 * nl + sizeof(c64) * 9 * M + 1024;
     void *buf = nullptr;
-    MFD_HIP(hipMalloc(&buf, bytes));
+    MFD_HIP(ctx_malloc(ctx, &buf, bytes));
     char *p = (char *)buf;
     std::vector<double> hc;
     hc.reserve(ncoord);

@@ -858,8 +858,8 @@ int op_create_impl(mfd_ctx *ctx, const mfd_grid *g, int ft, mfd_c64 omega, const
             op->ee_all = 0;
             op->rev |= 1 << a;
         }
-    int rc = op->G.create(g, ctx->stream);
-    if (!rc && op->rev) rc = op->G.reflect(op->rev, ctx->stream);
+    int rc = op->G.create(g, ctx);
+    if (!rc && op->rev) rc = op->G.reflect(op->rev, ctx);
     if (rc) { delete op; return rc; }
     hipStream_t s = ctx->stream;
     int64_t M = op->G.h.M;
@@ -1008,7 +1008,7 @@ int op_create_csc_impl(mfd_ctx *ctx, const mfd_csc *A, mfd_op **out) {
     op->stream = ctx->stream;
     op->ft = MFD_EE;
     auto bail = [&](int code) { op_destroy_impl(op); return code; };
-    int rc = op->G.create(&g, ctx->stream);
+    int rc = op->G.create(&g, ctx);
     if (rc) return bail(rc);
     hipStream_t s = ctx->stream;
     op->n = n;
@@ -1032,7 +1032,7 @@ int op_create_csc_impl(mfd_ctx *ctx, const mfd_csc *A, mfd_op **out) {
     // symmetrizing scaling: breadth-first sweeps (checked every 16), a new
     // seed for each component, then the check
     void *tmp = nullptr;
-    if (hipMalloc(&tmp, 2 * sizeof(c64) * n + 256) != hipSuccess) { set_error("hipMalloc failed"); return bail(MFD_ERR_ALLOC); }
+    if (ctx_malloc(ctx, &tmp, 2 * sizeof(c64) * n + 256) != hipSuccess) { set_error("hipMalloc failed"); return bail(MFD_ERR_ALLOC); }
     c64 *w = (c64 *)tmp, *w2 = w + n;
     int *chg = (int *)(w2 + n);
     unsigned long long *first = (unsigned long long *)(chg + 32);
@@ -1169,8 +1169,8 @@ static int time_apply(mfd_op *op, int64_t nrhs, int prec, int mode, int iters, d
     int64_t n = op->n;
     size_t es = prec == MFD_FP64 ? sizeof(c64) : sizeof(c32);
     void *dx = nullptr, *dy = nullptr;
-    MFD_HIP(hipMalloc(&dx, es * n * nrhs));
-    if (hipMalloc(&dy, es * n * nrhs) != hipSuccess) { hipFree(dx); return MFD_ERR_ALLOC; }
+    MFD_HIP(ctx_malloc(op->ctx, &dx, es * n * nrhs));
+    if (ctx_malloc(op->ctx, &dy, es * n * nrhs) != hipSuccess) { hipFree(dx); return MFD_ERR_ALLOC; }
     hipStream_t s = op->stream;
     hipMemsetAsync(dx, 0, es * n * nrhs, s);
     auto one = [&]() {
@@ -2406,8 +2406,8 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
     {
         BCHK(hipEventCreate(&tev0));
         BCHK(hipEventCreate(&tev1));
-        BCHK(hipMalloc(&src_d, sizeof(Scal *) * count));
-        BCHK(hipMalloc(&all_d, sizeof(Scal) * count));
+        BCHK(ctx_malloc(ctx, (void **)&src_d, sizeof(Scal *) * count));
+        BCHK(ctx_malloc(ctx, (void **)&all_d, sizeof(Scal) * count));
         BCHK(hipHostMalloc((void **)&all_h, sizeof(Scal) * count, hipHostMallocDefault));
         {
             std::vector<Scal *> src(count);
