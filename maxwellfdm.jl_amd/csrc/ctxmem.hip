@@ -2,6 +2,7 @@
 #include "ctxmem.hpp"
 #include <algorithm>
 #include <atomic>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -77,6 +78,11 @@ hipError_t ctx_malloc(mfd_ctx *ctx, void **p, size_t bytes) {
 }
 
 int scratch_get(mfd_ctx *ctx, size_t bytes, void **p) {
+    if (bytes > SIZE_MAX - 65535) {   // (a wrapped size is not a small one)
+        *p = nullptr;
+        set_error("scratch size out of range");
+        return MFD_ERR_ALLOC;
+    }
     bytes = (std::max<size_t>(bytes, 1) + 65535) / 65536 * 65536;
     CtxMem *m = ctx->mem;
     {

@@ -1142,8 +1142,15 @@ int op_set_graddiv_impl(mfd_op *op, int enable) {
     return MFD_OK;
 }
 
+// (before a size is formed from it: a negative one would wrap)
+static int check_nrhs(int64_t nrhs) {
+    if (nrhs >= 1 && nrhs <= 65535) return MFD_OK;
+    set_error("nrhs out of range");
+    return MFD_ERR_ARG;
+}
+
 int op_apply_dev_impl(mfd_op *op, const void *x, void *y, int64_t nrhs, int prec) {
-    if (nrhs < 1 || nrhs > 65535) { set_error("nrhs out of range"); return MFD_ERR_ARG; }
+    MFD_TRY(check_nrhs(nrhs));
     MFD_TRY(hbuf_ensure(op, nrhs));
     if (prec == MFD_FP64) launch_apply<double, MODE_A, EPI_STORE>(op, (const c64 *)x, (c64 *)y, nullptr, nrhs, nullptr, nullptr, nullptr);
     else launch_apply<float, MODE_A, EPI_STORE>(op, (const c32 *)x, (c32 *)y, nullptr, nrhs, nullptr, nullptr, nullptr);
@@ -1153,6 +1160,7 @@ int op_apply_dev_impl(mfd_op *op, const void *x, void *y, int64_t nrhs, int prec
 }
 
 int op_apply_impl(mfd_op *op, const mfd_c64 *x, mfd_c64 *y, int64_t nrhs) {
+    MFD_TRY(check_nrhs(nrhs));
     int64_t n = op->n;
     size_t b = sizeof(c64) * n * nrhs;
     Scratch dx, dy;
@@ -1165,6 +1173,7 @@ int op_apply_impl(mfd_op *op, const mfd_c64 *x, mfd_c64 *y, int64_t nrhs) {
 
 // average ms of one stencil launch (EPI_STORE): MODE_A or MODE_P, FP64 or FP32 vectors
 static int time_apply(mfd_op *op, int64_t nrhs, int prec, int mode, int iters, double *ms) {
+    MFD_TRY(check_nrhs(nrhs));
     MFD_TRY(hbuf_ensure(op, nrhs));
     int64_t n = op->n;
     size_t es = prec == MFD_FP64 ? sizeof(c64) : sizeof(c32);
@@ -2162,7 +2171,7 @@ static int run_inner_bicgstab(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o,
 int solve_dev_impl(mfd_op *op, const void *b, void *e, int64_t nrhs, const mfd_solve_opts *oin, mfd_solve_stats *st) {
     mfd_solve_opts o;
     if (oin) o = *oin; else solve_opts_default(&o);
-    if (nrhs < 1 || nrhs > 65535) { set_error("nrhs out of range"); return MFD_ERR_ARG; }
+    MFD_TRY(check_nrhs(nrhs));
     int prec = o.precision == MFD_MIXED ? MFD_MIXED : MFD_FP64;
     MFD_TRY(ws_ensure(op, nrhs, prec));
     Workspace &w = op->ws;
@@ -2631,6 +2640,7 @@ int solve_batch_impl(int count, mfd_op *const *ops, const mfd_c64 *const *b, mfd
 }
 
 int solve_impl(mfd_op *op, const mfd_c64 *b, mfd_c64 *e, int64_t nrhs, const mfd_solve_opts *o, mfd_solve_stats *st) {
+    MFD_TRY(check_nrhs(nrhs));
     int64_t n = op->n;
     size_t bytes = sizeof(c64) * n * nrhs;
     Scratch db, de;
