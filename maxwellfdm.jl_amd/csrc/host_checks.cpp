@@ -1,7 +1,7 @@
 // CPU checks of host- and device-shared integer code (needs no GPU and no HIP):
 //   host_checks resident    the resident solver's index code, every box shape
 //   host_checks scal        the store of a right-hand side's scalars
-//   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs
+//   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs steps
 //                           whether that many right-hand sides run resident
 //   host_checks tile N0 N1 N2 nrhs fp64 apply mu full gd rev win narrow
 //                           rows and planes of a tile
@@ -243,13 +243,13 @@ static void scal() {
 int main(int argc, char **argv) {
     if (argc == 2 && !strcmp(argv[1], "resident")) { resident(); return 0; }
     if (argc == 2 && !strcmp(argv[1], "scal")) { scal(); return 0; }
-    if (argc == 13 && !strcmp(argv[1], "pays")) {
-        int v[11];
-        for (int k = 0; k < 11; ++k) v[k] = atoi(argv[2 + k]);
+    if (argc == 14 && !strcmp(argv[1], "pays")) {
+        int v[12];
+        for (int k = 0; k < 12; ++k) v[k] = atoi(argv[2 + k]);
         int boxes = 1;
         for (int a = 0; a < 3; ++a) boxes *= (v[3 + a] + v[a] - 1) / v[a];
         const ResForm f = {v[7] != 0, v[8] != 0, v[9] != 0, v[5] == 1, v[6]};
-        printf("%d\n", (int)res_pays(f, boxes, v[0] * v[1] * v[2], RES_BOXES, (int64_t)v[3] * v[4] * v[5], v[10]));
+        printf("%d\n", (int)res_pays(f, boxes, v[0] * v[1] * v[2], RES_BOXES, (int64_t)v[3] * v[4] * v[5], v[10], v[11]));
         return 0;
     }
     if (argc == 14 && !strcmp(argv[1], "tile")) {

@@ -1820,7 +1820,7 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     MFD_HIP(hipGetLastError());
     int chunk = o->check_every > 0 ? o->check_every : 32;
     bool use_graph = o->use_graph != 0;
-    bool res = resident_ok<R>(op, nrhs);
+    bool res = resident_ok<R>(op, nrhs, chunk);
     if (res && getenv("MFD_SOLVE_TRACE")) resident_trace<R>(op);
     if (use_graph && !res) MFD_TRY(chunk_graph<R>(op, nrhs, chunk));
     long long done_it = 0;
@@ -2370,7 +2370,7 @@ struct BatchProb {
     long long it_total = 0, it32 = 0, cycles = 0, next_probe = 0, next64 = 0;
     long long it_seen = 0;     // steps of the cycle at the last readback
     bool conv = false, done = false, stalled32 = false;   // stalled32: an FP32 cycle stagnated
-    bool res() const { return prec == MFD_MIXED ? resident_ok<float>(op, 1) : resident_ok<double>(op, 1); }
+    bool res(int chunk) const { return prec == MFD_MIXED ? resident_ok<float>(op, 1, chunk) : resident_ok<double>(op, 1, chunk); }
 };
 }  // namespace
 
@@ -2514,7 +2514,7 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
                 if (B.done) continue;
                 live = true;
                 int r;
-                if (B.res()) {   // as in run_inner: up to the next step at which the problem is looked at
+                if (B.res(chunk)) {   // as in run_inner: up to the next step at which the problem is looked at
                     if (B.prec == MFD_MIXED) r = resident_steps<float>(B.op, 1, resident_span(chunk, B.it_seen, B.next_probe), chunk, 0);
                     else {
                         const bool look = !B.op->gd && B.it_seen >= B.next64;

@@ -695,14 +695,14 @@ static int res_xch(const ResPlan &P, int64_t n) {
 static_assert(RES_BOXES * RES_SLOT_WORDS * sizeof(unsigned long long) <= sizeof(double) * NPART * 4, "a right-hand side's slots");
 
 template <typename R>
-bool resident_ok(const mfd_op *op, int64_t nrhs) {
+bool resident_ok(const mfd_op *op, int64_t nrhs, int chunk) {
     if (op->res_off || op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
     if (op->G.d64.M > RES_MAX_CELLS) return false;
     const ResPlan P = res_plan<R>(op);
     if (P.nb > P.cap || res_xch<R>(P, op->n) == 0) return false;
     const DGrid<double> &g = op->G.d64;
     const ResForm f = {sizeof(R) == 8, op->has_mu != 0, op->full != 0, g.N[2] == 1, g.nc};
-    return res_pays(f, P.nb, P.cells, P.cap, g.M, nrhs);
+    return res_pays(f, P.nb, P.cells, P.cap, g.M, nrhs, nrhs == 1 ? std::max(chunk, 512) : chunk);
 }
 
 template <typename R>
@@ -756,8 +756,8 @@ int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) 
     return MFD_OK;
 }
 
-template bool resident_ok<double>(const mfd_op *, int64_t);
-template bool resident_ok<float>(const mfd_op *, int64_t);
+template bool resident_ok<double>(const mfd_op *, int64_t, int);
+template bool resident_ok<float>(const mfd_op *, int64_t, int);
 template void resident_trace<double>(const mfd_op *);
 template void resident_trace<float>(const mfd_op *);
 template int resident_steps<double>(mfd_op *, int64_t, int, int, double);

@@ -8,9 +8,10 @@ namespace mfd {
 // vectors of storage precision R: the stencil form is built (diagonal or full
 // ε with μ = 1, or μ ≠ 1 with diagonal ε; any boundft, a component window),
 // every box of one right-hand side has a place on the chip at once, and the
-// launches that nrhs of them take are faster than the step-by-step kernels.
+// launches that nrhs of them take are faster than the step-by-step kernels
+// (chunk: steps between two looks at the scalars).
 template <typename R>
-bool resident_ok(const mfd_op *op, int64_t nrhs);
+bool resident_ok(const mfd_op *op, int64_t nrhs, int chunk);
 
 // the boxes it runs in, to stderr
 template <typename R>

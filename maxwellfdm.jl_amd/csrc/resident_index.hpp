@@ -166,19 +166,22 @@ MFD_HD inline int res_room(int boxes, int cells, size_t vb, size_t part_bytes, i
 // Both sides as measured (µs per step, resident / step by step): 24³ 2 RHS 9.4 /
 // 21.6, 8 36.1 / 31.5, 16 70 / 39; 31×31×32 2 20.4 / 25.1, 4 39.6 / 30.6, 16 157 /
 // 60; 48³ 4 55 / 58, 8 110 / 97; FP32 64³ 2 41 / 48, 4 82 / 71 (1,024 cells a box
-// at 20 µs, 17 since); 180×170 (Ex, Ey) 2 9.9 / 19, 16 57 / 49.  The constants
+// at 20 µs, 17 since), 40³ with 2 RHS and launches of one step (check_every = 1)
+// 104 / 62; 180×170 (Ex, Ey) 2 9.9 / 19, 16 57 / 49.  The constants
 // below are fits to 76 systems on 15 grids, 1 to 16 right-hand sides: the choice is the
 // faster one but near the crossing (1.26 times the faster at worst).
+// steps: of a launch (a launch takes about 26 µs beside its steps, and several
+// right-hand sides are looked at after every chunk, one only every 512 steps).
 struct ResForm {
     bool fp64, mu, full;   // vectors; 1/μ, corner ε
     bool plane;            // one-cell z axis
     int nc;                // components of the window
 };
-inline bool res_pays(const ResForm &f, int boxes, int box_cells, int cap, int64_t cells, int64_t nrhs) {
+inline bool res_pays(const ResForm &f, int boxes, int box_cells, int cap, int64_t cells, int64_t nrhs, int steps) {
     const bool tensor = f.mu || f.full;
-    const double launch = (f.plane ? (box_cells <= 128 ? 7.6 : (box_cells <= 512 ? 10.2 : 13.8))
-                                   : (box_cells <= 128 ? 9.2 : (box_cells <= 256 ? 10.6 : (box_cells <= 512 ? 13.2 : 17.0)))) *
-                          (tensor ? 1.1 : 1.0);
+    const double launch = (f.plane ? (box_cells <= 128 ? 6.8 : (box_cells <= 512 ? 9.4 : 13.0))
+                                   : (box_cells <= 128 ? 8.4 : (box_cells <= 256 ? 9.8 : (box_cells <= 512 ? 12.4 : 16.2)))) *
+                              (tensor ? 1.1 : 1.0) + 26.0 / steps;
     const int64_t per = cap / boxes < 1 ? 1 : cap / boxes, launches = (nrhs + per - 1) / per;
     // ns per unknown and step of the four kernels: the marching stencil serves a
     // plane of three components less well, a window's has a kernel of its own

@@ -66,7 +66,7 @@ MEASURED = [
 @pytest.mark.parametrize("box,N,nc,vectors,scene,nrhs,resident,steps", MEASURED)
 def test_resident_rhs(driver, box, N, nc, vectors, scene, nrhs, resident, steps):
     """The faster of the two solvers by the number of right-hand sides."""
-    pays = run(driver, "pays", *box, *N, nc, int(vectors == "fp64"), int(scene == "mu"), int(scene == "full"), nrhs).strip()
+    pays = run(driver, "pays", *box, *N, nc, int(vectors == "fp64"), int(scene == "mu"), int(scene == "full"), nrhs, 512 if nrhs == 1 else 32).strip()
     assert pays == ("1" if resident < steps else "0")
 
 
@@ -88,6 +88,16 @@ def test_tile_fit(driver, N, nrhs, narrow, ty_max, reduces, ty, kz, want):
     """Tiles of planes too large for the partial sums: the planes were doubled
     without end, to a division by zero."""
     assert run(driver, "fit", *N, nrhs, narrow, ty_max, reduces, ty, kz).strip() == want
+
+
+@pytest.mark.parametrize("box,N,nrhs,steps,resident", [
+    ((8, 8, 4), (40, 40, 40), 2, 1, 0),     # 104 against 62 µs a step (step by step), the start of each launch
+    ((8, 4, 4), (20, 20, 20), 2, 1, 0),     # 52 against 47
+    ((8, 4, 4), (20, 20, 20), 2, 8, 1),
+    ((8, 4, 4), (20, 20, 20), 1, 512, 1),   # one right-hand side: up to 512 steps a launch whatever the chunk
+])
+def test_resident_short_launches(driver, box, N, nrhs, steps, resident):
+    assert int(run(driver, "pays", *box, *N, 3, 1, 0, 0, nrhs, steps)) == resident
 
 
 # A on one right-hand side (three: last column): µs per apply by (rows, planes) of a tile, measured; the
