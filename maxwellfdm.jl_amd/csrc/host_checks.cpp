@@ -3,7 +3,7 @@
 //   host_checks scal        the store of a right-hand side's scalars
 //   host_checks pays TX TY TZ N0 N1 N2 nc fp64 mu full nrhs steps
 //                           whether that many right-hand sides run resident
-//   host_checks tile N0 N1 N2 nrhs fp64 apply mu full gd rev win narrow
+//   host_checks tile N0 N1 N2 nrhs fp64 apply mu full gd rev win narrow cocg
 //                           rows and planes of a tile
 //   host_checks fit N0 N1 N2 nrhs narrow ty_max reduces ty kz
 //                           the tile made large enough ("no": none is)
@@ -252,10 +252,10 @@ int main(int argc, char **argv) {
         printf("%d\n", (int)res_pays(f, boxes, v[0] * v[1] * v[2], RES_BOXES, (int64_t)v[3] * v[4] * v[5], v[10], v[11]));
         return 0;
     }
-    if (argc == 14 && !strcmp(argv[1], "tile")) {
-        int v[12], ty = 0, kz = 0;
-        for (int k = 0; k < 12; ++k) v[k] = atoi(argv[2 + k]);
-        const TileKernel K = {v[4] != 0, v[5] != 0, v[6] != 0, v[7] != 0, v[8] != 0, v[9] != 0, v[10] != 0, v[11] != 0};
+    if (argc == 15 && !strcmp(argv[1], "tile")) {
+        int v[13], ty = 0, kz = 0;
+        for (int k = 0; k < 13; ++k) v[k] = atoi(argv[2 + k]);
+        const TileKernel K = {v[4] != 0, v[5] != 0, v[6] != 0, v[7] != 0, v[8] != 0, v[9] != 0, v[10] != 0, v[11] != 0, v[12] != 0};
         tile_rule(v, v[3], K, ty, kz);
         printf("%d %d\n", ty, kz);
         return 0;

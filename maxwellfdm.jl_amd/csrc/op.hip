@@ -636,12 +636,12 @@ void Workspace::release() {
 }
 
 // the caller's or the autotuner's shape, or that of tile_rule
-Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode) {
+Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode, bool cocg) {
     const int *t = fp64 ? op->tile64 : op->tile32;
     Tile best = {t[0], t[1], t[2]};
     if (best.ty == 0 || op->tile_set[fp64 ? 0 : 1]) return best;
-    TileKernel K = {fp64, mode == MODE_A, op->has_mu != 0, op->full != 0, op->gd != 0, op->rev != 0, op->win != 0, false};
-    K.narrow = (best.xr & 2) && !K.mu && !K.full && !(K.gd && !K.apply) && !K.rev && !K.win;   // as launch_apply takes it
+    TileKernel K = {fp64, mode == MODE_A, op->has_mu != 0, op->full != 0, op->gd != 0, op->rev != 0, op->win != 0, false, cocg};
+    K.narrow = (best.xr & 2) && !cocg && !K.mu && !K.full && !(K.gd && !K.apply) && !K.rev && !K.win;   // as launch_apply takes it
     tile_rule(op->G.d64.N, nrhs, K, best.ty, best.kz);
     return best;
 }
@@ -1515,10 +1515,11 @@ static void launch_cocg_iter(mfd_op *op, int64_t nrhs, int par) {
     cx<R> *po = cocg_p<R>(w, par), *pn = cocg_p<R>(w, par ^ 1);
     const DGrid<R> &g = op->G.view<R>();
     // the fused COCG stencil is built 64-wide only: the narrow-tile bit is ignored
-    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs, MODE_P);
+    const bool fused = !op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win;
+    const Tile tile = stencil_tile(op, std::is_same<R, double>::value, nrhs, MODE_P, fused);
     const int xr = tile.xr & 1;
     int ty = tile.ty, kz = tile.kz;
-    if (!op->csr && !op->full && !op->has_mu && !op->gd && op->ee_all && !op->win && ty > 0 &&
+    if (fused && ty > 0 &&
         tile_fit(op->G.d64.N, nrhs, false, 8, true, NPART, ty, kz)) {
         const int nx = (g.N[0] + 63) / 64, ny = (g.N[1] + ty - 1) / ty, nch = (g.N[2] + kz - 1) / kz;
         dim3 grid(nx, ny, (unsigned)(nch * nrhs));

@@ -5,11 +5,12 @@
 
 namespace mfd {
 
-// the tile shape of a stencil launch over nrhs right-hand sides (mode: A or P)
+// the tile shape of a stencil launch over nrhs right-hand sides (mode: A or P;
+// cocg: COCG's fused P)
 struct Tile {
     int ty, kz, xr;   // rows, planes, order (bit 0: XCD runs, bit 1: 32-wide); ty = 0: the direct kernel
 };
-Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode);
+Tile stencil_tile(const mfd_op *op, bool fp64, int64_t nrhs, int mode, bool cocg = false);
 
 // a 2D model's window on one plane of cells that k_apply_plane serves
 static inline bool plane_ok(const mfd_op *op, bool fp64) {

@@ -32,6 +32,7 @@ struct TileKernel {
     bool rev;               // a reflected grid (boundft HH on some axis)
     bool win;               // a component window
     bool narrow;            // 32-wide tiles of twice the rows
+    bool cocg;              // COCG's fused P (64-wide only)
 };
 
 // A launch takes as many rounds of blocks as the fullest CU has, so its time is
@@ -55,15 +56,21 @@ struct TileKernel {
 // well, lost up to 48% there (µs per apply, 4 × 16 → those → these: μ ≠ 1
 // 190×33×120 47.1 → 57.1 → 44.1, FP32 96×90×100 65.9 → 69.4 → 46.8, FP32 HEE
 // 150×60×170 61.3 → 62.3 → 52.7).
+// COCG's fused P, which moves four more vectors, on 10 grids of 24 to 170 cells:
+// 2.5% (FP64) and 0.4% slower than the fastest; with P's constants and the width
+// of tiles that it does not have it lost up to 33% (µs per step, 4 × 16 → those →
+// these: 150×60×170 229.4 → 303.2 → 228.7, FP32 146.7 → 220.0 → 146.2; 70×66×72
+// with three right-hand sides 159.1 → 175.5 → 139.9; 190×33×120 99.1 → 108.2 →
+// 106.4, where 8 planes would take 99.7).
 // P against 4 × 16 with planes halved while a launch had fewer than 256 tiles (µs
 // per step): full ε 144×120×100 330.6 → 274.7, μ ≠ 1 80×76×70 96.2 → 80.0, boundft
 // HEE 100×90×96 127.1 → 107.5, 110×112×90 138.6 → 121.0, 56×58×52 41.7 → 37.8.
 // More than 20 planes lose again (203×180×151: 24 planes 618 µs, 20 planes 593).
 inline void tile_rule(const int *N, int64_t nrhs, const TileKernel &K, int &ty_out, int &kz_out) {
     const int per4 = !K.apply && (K.mu || K.gd) ? 1 : (K.apply && !K.fp64 && !K.mu && !K.full && !K.win ? 3 : 2);
-    const double alone = K.apply ? 0.8 : (per4 == 1 ? 0.5 : 0.7);
+    const double alone = K.apply || (K.cocg && !K.fp64) ? 0.8 : (K.cocg ? 0.65 : (per4 == 1 ? 0.5 : 0.7));
     const int nx = (N[0] + (K.narrow ? 31 : 63)) / (K.narrow ? 32 : 64);
-    const bool eight_pays = !K.apply || per4 == 3 || (K.mu && !K.fp64) || ((K.mu || K.rev) && nx == 1);
+    const bool eight_pays = !(K.apply || K.cocg) || per4 == 3 || (K.mu && !K.fp64) || ((K.mu || K.rev) && nx == 1);
     const double eight = eight_pays ? 0.97 : 1.03;
     double least = 1e300;
     for (int ty = 8; ty >= 4; ty /= 2) {

@@ -123,7 +123,7 @@ def test_apply_tiles(driver, N, scene, vectors, nrhs, us):
     """The rule's tile is one of the fastest three, within 4 % of the fastest."""
     narrow = scene == "diag" and 64 * -(-N[0] // 64) > 32 * -(-N[0] // 32)
     pick = run(driver, "tile", *N, nrhs, int(vectors == "fp64"), 1, int(scene == "mu"), int(scene == "full"), 0,
-               int(scene == "hee"), 0, int(narrow))
+               int(scene == "hee"), 0, int(narrow), 0)
     pick = tuple(map(int, pick.split()))
     assert pick in us and us[pick] <= 1.04 * min(us.values())
 
@@ -132,3 +132,22 @@ def test_scal_store(driver):
     """The lead block of a resident launch stores the scalars without the mark that
     a block which gave up waiting may set meanwhile."""
     assert "scal ok" in run(driver, "scal")
+
+
+# COCG's fused step: µs by (rows, planes), measured; the three fastest and 4 × 16
+COCG = [
+    ((64, 64, 64), "fp64", 1, {(4, 4): 54.1, (4, 3): 54.7, (8, 3): 56.2, (4, 16): 97.1}),
+    ((70, 66, 72), "fp64", 3, {(4, 15): 139.9, (4, 16): 146.5, (4, 8): 146.8, (4, 9): 151.1}),
+    ((70, 66, 72), "fp32", 1, {(4, 5): 57.0, (4, 6): 61.2, (8, 6): 64.1, (4, 16): 96.5}),
+    ((100, 90, 96), "fp32", 1, {(4, 9): 82.8, (4, 10): 86.2, (8, 10): 89.7, (4, 16): 113.6}),
+    ((150, 60, 170), "fp64", 1, {(4, 16): 228.7, (8, 18): 231.2, (4, 18): 239.8}),
+    ((150, 60, 170), "fp32", 1, {(4, 16): 146.2, (4, 18): 155.6, (4, 8): 156.2}),
+    ((30, 170, 60), "fp64", 1, {(4, 6): 60.8, (8, 6): 63.9, (4, 7): 64.4, (4, 16): 91.6}),
+]
+
+
+@pytest.mark.parametrize("N,vectors,nrhs,us", COCG)
+def test_cocg_tiles(driver, N, vectors, nrhs, us):
+    pick = run(driver, "tile", *N, nrhs, int(vectors == "fp64"), 0, 0, 0, 0, 0, 0, 0, 1)
+    pick = tuple(map(int, pick.split()))
+    assert pick in us and us[pick] <= 1.07 * min(us.values())
