@@ -37,6 +37,7 @@ struct CtxMem {
         size_t bytes = 0;
         bool used = false;
     } blk[NBLK];
+    hipStream_t side = nullptr;   // (under m)
     std::mutex copying;   // the slots
     char *pin = nullptr;
     hipEvent_t ev[2 * COPY_THREADS] = {};
@@ -60,6 +61,7 @@ static void drop_unused(CtxMem *m) {
 void ctxmem_destroy(CtxMem *m) {
     if (!m) return;
     drop_unused(m);
+    if (m->side) hipStreamDestroy(m->side);
     for (auto &e : m->ev)
         if (e) hipEventDestroy(e);
     if (m->pin) hipHostFree(m->pin);
@@ -145,6 +147,16 @@ void scratch_put(mfd_ctx *ctx, void *p) {
         }
     }
     for (int i = 0; i < nd; ++i) hipFree(drop[i]);   // waits for the device
+}
+
+hipStream_t ctx_side_stream(mfd_ctx *ctx) {
+    CtxMem *m = ctx->mem;
+    std::lock_guard<std::mutex> lock(m->m);
+    if (!m->side && hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking) != hipSuccess) {
+        hipGetLastError();
+        m->side = nullptr;
+    }
+    return m->side;
 }
 
 static bool slots_ready(CtxMem *m) {

@@ -31,6 +31,11 @@ struct Scratch {
 // hipMalloc that gives the context's unused blocks back before it fails
 hipError_t ctx_malloc(mfd_ctx *ctx, void **p, size_t bytes);
 
+// The context's second stream, made when first asked for (null: it could not be).
+// Work there is forked from and joined to the context's stream by events, so that
+// nothing else needs to know of it.
+hipStream_t ctx_side_stream(mfd_ctx *ctx);
+
 // Copies on the context's stream.  src of copy_in stays the caller's until the
 // stream is waited for; copy_out has written dst (and waited for the stream).
 int copy_in(mfd_ctx *ctx, void *dst, const void *src, size_t bytes);

@@ -2381,9 +2381,13 @@ struct BatchProb {
 // workspace from call to call) otherwise; between rounds the host reads all
 // solver scalars in one copy and runs the FP64 refinement step of each
 // problem whose inner cycle ended (same rules as solve_dev_impl's SQMR path).
-// One graph with a branch and a stream per problem was captured and
-// instantiated on every call, and its branches did not overlap: eight
-// problems of 20³ to 64³ took 312 µs per step, the sum of their own steps.
+// The graphs go to two streams, which overlap the small launches of two problems
+// (µs per step of all, one stream → two, 256 steps): eight of 54³ 285 → 179, three
+// of 64³ 132 → 109, six of 70³ 317 → 250, 70³, 66³ and 60³ 140 → 120.  Three streams
+// take 161, 98, 243 and 108, but a process that has used three queues runs every
+// resident launch 3% longer from then on.  One graph of all problems with a branch
+// and a stream each, captured and instantiated in every call, took 218, 113, 299
+// and 125.
 int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, void *const *e,
                          const mfd_solve_opts *oin, mfd_solve_stats *st) {
     if (count < 1 || count > 1024 || !ops || !b || !e) { set_error("count must be in [1, 1024] with non-null arrays"); return MFD_ERR_ARG; }
@@ -2407,7 +2411,8 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
         P[p].prec = prec0;
         MFD_TRY(ws_ensure(ops[p], 1, prec0));
     }
-    hipEvent_t tev0 = nullptr, tev1 = nullptr;
+    hipEvent_t tev0 = nullptr, tev1 = nullptr, fork = nullptr, join = nullptr;
+    hipStream_t forked = nullptr;
     Scal **src_d = nullptr;
     Scal *all_d = nullptr, *all_h = nullptr;
     int rc = MFD_OK;
@@ -2416,6 +2421,8 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
     {
         BCHK(hipEventCreate(&tev0));
         BCHK(hipEventCreate(&tev1));
+        BCHK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+        BCHK(hipEventCreateWithFlags(&join, hipEventDisableTiming));
         BCHK(ctx_malloc(ctx, (void **)&src_d, sizeof(Scal *) * count));
         BCHK(ctx_malloc(ctx, (void **)&all_d, sizeof(Scal) * count));
         BCHK(hipHostMalloc((void **)&all_h, sizeof(Scal) * count, hipHostMallocDefault));
@@ -2509,27 +2516,44 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
             if (r) { rc = r; goto cleanup; }
         }
         while (true) {
-            bool live = false;
+            int live = 0, steps = 0;   // problems; those of them that run step by step
             for (int p = 0; p < count; ++p) {
                 BatchProb &B = P[p];
                 if (B.done) continue;
-                live = true;
+                ++live;
+                if (!B.res(chunk)) { ++steps; continue; }
+                // as in run_inner: up to the next step at which the problem is looked at
                 int r;
-                if (B.res(chunk)) {   // as in run_inner: up to the next step at which the problem is looked at
-                    if (B.prec == MFD_MIXED) r = resident_steps<float>(B.op, 1, resident_span(chunk, B.it_seen, B.next_probe), chunk, 0);
-                    else {
-                        const bool look = !B.op->gd && B.it_seen >= B.next64;
-                        r = resident_steps<double>(B.op, 1, resident_span(chunk, B.it_seen, look ? 0 : B.next64), chunk,
-                                                   look ? 3.0 * o.tol / B.worst : 0.0);
-                    }
-                    if (r == RESIDENT_REFUSED) r = MFD_OK;   // step by step from the next round
-                } else {
-                    r = B.prec == MFD_MIXED ? chunk_graph<float>(B.op, 1, chunk) : chunk_graph<double>(B.op, 1, chunk);
-                    if (!r) BCHK(hipGraphLaunch(B.op->ws.graph, s));
+                if (B.prec == MFD_MIXED) r = resident_steps<float>(B.op, 1, resident_span(chunk, B.it_seen, B.next_probe), chunk, 0);
+                else {
+                    const bool look = !B.op->gd && B.it_seen >= B.next64;
+                    r = resident_steps<double>(B.op, 1, resident_span(chunk, B.it_seen, look ? 0 : B.next64), chunk,
+                                               look ? 3.0 * o.tol / B.worst : 0.0);
                 }
-                if (r) { rc = r; goto cleanup; }
+                if (r && r != RESIDENT_REFUSED) { rc = r; goto cleanup; }   // (refused: step by step below)
             }
             if (!live) break;
+            // the chunk graphs of several problems on two streams, side by side
+            hipStream_t side = steps > 1 ? ctx_side_stream(ctx) : nullptr;
+            if (side) {
+                BCHK(hipEventRecord(fork, s));
+                BCHK(hipStreamWaitEvent(side, fork, 0));
+                forked = side;
+            }
+            int64_t load[2] = {0, 0};
+            for (int p = 0; p < count; ++p) {
+                BatchProb &B = P[p];
+                if (B.done || B.res(chunk)) continue;
+                const int r = B.prec == MFD_MIXED ? chunk_graph<float>(B.op, 1, chunk) : chunk_graph<double>(B.op, 1, chunk);
+                if (r) { rc = r; goto cleanup; }
+                const int k = side && load[1] < load[0];
+                load[k] += B.op->n;
+                BCHK(hipGraphLaunch(B.op->ws.graph, k ? side : s));
+            }
+            if (side) {
+                BCHK(hipEventRecord(join, side));
+                BCHK(hipStreamWaitEvent(s, join, 0));
+            }
             k_gather_scal<<<(count + 63) / 64, 64, 0, s>>>(src_d, all_d, count);
             BCHK(hipMemcpyAsync(all_h, all_d, sizeof(Scal) * count, hipMemcpyDeviceToHost, s));
             BCHK(hipStreamSynchronize(s));
@@ -2602,6 +2626,9 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
 cleanup:
 #undef BCHK
     hipStreamSynchronize(s);
+    if (forked) hipStreamSynchronize(forked);   // (an error between fork and join)
+    if (fork) hipEventDestroy(fork);
+    if (join) hipEventDestroy(join);
     if (tev0) hipEventDestroy(tev0);
     if (tev1) hipEventDestroy(tev1);
     if (src_d) hipFree(src_d);
