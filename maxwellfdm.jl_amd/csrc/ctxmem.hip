@@ -11,8 +11,10 @@
 namespace mfd {
 
 // An allocation and its release cost 60–800 µs of a call (the release waits
-// for the device and unmaps the pages), so blocks are kept from call to call,
-// within a bound that holds the arrays of a 56×48×50 assembly (172 MB).
+// for the device and unmaps the pages), so blocks are kept from call to call:
+// 0.1% of the device's memory at most.  A call whose arrays need more (an
+// assembly of more than some 200,000 cells) allocates as it did, beside tens of
+// ms of copies (90×80×70: 29 ms).
 constexpr size_t CTXMEM_KEEP = 256u << 20;
 constexpr int NBLK = 32;
 
@@ -21,9 +23,10 @@ constexpr int NBLK = 32;
 // Here a thread per 4 MB does that (eight at most), each with two pinned slots
 // of its own, so that one slot fills while the other drains.  The assembled
 // 56×48×50 A (126 MB out) takes 17.1 ms the plain way and 10.5, 9.8 and 8.7 ms
-// with 2, 4 and 8 threads.  Below 16 MB the plain way stays: an apply with
-// 11 MB in and out gains 0.2 of 1.3 ms, but the caller's fresh pages end up on
-// other NUMA nodes, and a 2D solve that reorders them afterwards loses 1 of 11 ms.
+// with 2, 4 and 8 threads.  Below 16 MB (four threads' worth) the plain way stays:
+// an apply with 11 MB in and out would gain 0.2 of 1.3 ms, but the pages that the
+// threads touch first end up on other NUMA nodes, and a caller that goes through
+// them afterwards loses more (a 2D solve that reorders 11 MB: 1 of 11 ms).
 constexpr int COPY_THREADS = 8;
 constexpr size_t CHUNK = 1u << 20;
 constexpr size_t PER_THREAD = 4u << 20;

@@ -1237,8 +1237,6 @@ int op_bench_iteration_impl(mfd_op *op, int64_t nrhs, int prec, int iters, doubl
     size_t es = prec == MFD_FP64 ? sizeof(c64) : sizeof(c32);
     // bounded nonzero contents (every byte 0x3c: ~1e-2 in FP32, ~2e-19 in FP64)
     for (void *v : {w.r, w.q, w.t, w.d, w.z}) MFD_HIP(hipMemsetAsync(v, 0x3c, es * n * nrhs, s));
-    dim3 gv(ngrid(n), (unsigned)nrhs);
-    const size_t ps = (size_t)nrhs * NPART * 4;
     std::vector<hipEvent_t> ev(6 * (size_t)iters, nullptr);
     int rc = MFD_OK;
     for (auto &e : ev)
@@ -1595,8 +1593,6 @@ static int run_cocg(mfd_op *op, const void *b, void *e, int64_t nrhs, const mfd_
     int64_t n = w.n;
     dim3 gv(ngrid(n), (unsigned)nrhs);
     size_t pslot = (size_t)nrhs * NPART * 4;
-    const DGrid<R> &g = op->G.view<R>();
-    const OpData<R> &od = opd<R>(op);
     std::vector<double> bn(nrhs);
     MFD_TRY(rhs_norms(op, b, e, nrhs, bn.data()));
     k_scal_reset<<<(unsigned)((nrhs + 63) / 64), 64, 0, s>>>(w.scal, nrhs);
@@ -1813,10 +1809,6 @@ static int run_inner(mfd_op *op, int64_t nrhs, const mfd_solve_opts *o, double r
     Workspace &w = op->ws;
     hipStream_t s = op->stream;
     int64_t n = w.n;
-    dim3 gv(ngrid(n), (unsigned)nrhs);
-    size_t pslot = (size_t)nrhs * NPART * 4;
-    const DGrid<R> &g = op->G.view<R>();
-    const OpData<R> &od = opd<R>(op);
     launch_init<R>(op, nrhs, rel_target, active_d, budget);
     MFD_HIP(hipGetLastError());
     int chunk = o->check_every > 0 ? o->check_every : 32;
