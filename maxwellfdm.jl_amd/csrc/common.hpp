@@ -2,6 +2,7 @@
 // staggered grid, and HIP error plumbing.  gfx950 only.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -134,4 +135,6 @@ struct mfd_ctx {
     int device;
     hipStream_t stream;
     mfd::CtxMem *mem = nullptr;   // scratch memory and copy slots (ctxmem.hpp)
+    // after a refused resident launch: when to ask again (ns of the steady clock)
+    std::atomic<int64_t> res_retry{0};
 };

@@ -2363,6 +2363,7 @@ struct BatchProb {
     long long it_total = 0, it32 = 0, cycles = 0, next_probe = 0, next64 = 0;
     long long it_seen = 0;     // steps of the cycle at the last readback
     bool conv = false, done = false, stalled32 = false;   // stalled32: an FP32 cycle stagnated
+    bool on_chip = false;      // this round's steps run resident
     bool res(int chunk) const { return prec == MFD_MIXED ? resident_ok<float>(op, 1, chunk) : resident_ok<double>(op, 1, chunk); }
 };
 }  // namespace
@@ -2513,7 +2514,8 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
                 BatchProb &B = P[p];
                 if (B.done) continue;
                 ++live;
-                if (!B.res(chunk)) { ++steps; continue; }
+                B.on_chip = B.res(chunk);
+                if (!B.on_chip) { ++steps; continue; }
                 // as in run_inner: up to the next step at which the problem is looked at
                 int r;
                 if (B.prec == MFD_MIXED) r = resident_steps<float>(B.op, 1, resident_span(chunk, B.it_seen, B.next_probe), chunk, 0);
@@ -2522,7 +2524,10 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
                     r = resident_steps<double>(B.op, 1, resident_span(chunk, B.it_seen, look ? 0 : B.next64), chunk,
                                                look ? 3.0 * o.tol / B.worst : 0.0);
                 }
-                if (r && r != RESIDENT_REFUSED) { rc = r; goto cleanup; }   // (refused: step by step below)
+                if (r == RESIDENT_REFUSED) {
+                    B.on_chip = false;
+                    ++steps;
+                } else if (r) { rc = r; goto cleanup; }
             }
             if (!live) break;
             // the chunk graphs of several problems on two streams, side by side
@@ -2535,7 +2540,7 @@ int solve_batch_dev_impl(int count, mfd_op *const *ops, const void *const *b, vo
             int64_t load[2] = {0, 0};
             for (int p = 0; p < count; ++p) {
                 BatchProb &B = P[p];
-                if (B.done || B.res(chunk)) continue;
+                if (B.done || B.on_chip) continue;
                 const int r = B.prec == MFD_MIXED ? chunk_graph<float>(B.op, 1, chunk) : chunk_graph<double>(B.op, 1, chunk);
                 if (r) { rc = r; goto cleanup; }
                 const int k = side && load[1] < load[0];

@@ -70,7 +70,6 @@ struct mfd_op {
     // 1 = fixed by the caller, whose solves then march through the tiles even
     // where the resident kernel would serve, 2 = fixed by the autotuner
     int tile_set[2] = {0, 0};
-    int res_off = 0;          // a resident launch was refused: step by step from then on
     int sym = 1;              // complex-symmetric up to S_E (no complex Bloch phase)
     int gd = 0;               // grad-div augmented inner operator in use
     int gd_ok = 0;            // eligible (diagonal ε, μ = 1)

@@ -35,6 +35,7 @@
 #include "resident_index.hpp"
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 
 namespace mfd {
@@ -694,9 +695,15 @@ static int res_xch(const ResPlan &P, int64_t n) {
 }
 static_assert(RES_BOXES * RES_SLOT_WORDS * sizeof(unsigned long long) <= sizeof(double) * NPART * 4, "a right-hand side's slots");
 
+// A refused launch costs 38 ms (the runtime tries to make the cooperative queue),
+// so a context asks again after 10 s only
+constexpr int64_t RES_RETRY_NS = 10000000000ll;
+static int64_t now_ns() { return std::chrono::steady_clock::now().time_since_epoch() / std::chrono::nanoseconds(1); }
+
 template <typename R>
 bool resident_ok(const mfd_op *op, int64_t nrhs, int chunk) {
-    if (op->res_off || op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
+    if (now_ns() < op->ctx->res_retry.load(std::memory_order_relaxed)) return false;
+    if (op->tile_set[0] == 1 || op->tile_set[1] == 1 || op->csr || op->gd || !(op->ee_all || op->rev) || (op->has_mu && op->full)) return false;
     if (op->G.d64.M > RES_MAX_CELLS) return false;
     const ResPlan P = res_plan<R>(op);
     if (P.nb > P.cap || res_xch<R>(P, op->n) == 0) return false;
@@ -746,12 +753,14 @@ int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near) 
         k_res_clear<<<(words + 255) / 256, 256, 0, s>>>(A.slots, words);
         void *args[] = {&A};
         const hipError_t e = hipLaunchCooperativeKernel(P.kernel, dim3((unsigned)(nr * A.nb)), dim3((unsigned)P.threads), args, 0, s);
-        if (e == hipErrorCooperativeLaunchTooLarge) {
+        // whatever the reason: too few places, or another process has the device's
+        // one cooperative queue (hipErrorIllegalState).  An error of earlier work
+        // comes up again in the step-by-step launches.
+        if (e != hipSuccess) {
             hipGetLastError();
-            op->res_off = 1;
+            op->ctx->res_retry.store(now_ns() + RES_RETRY_NS, std::memory_order_relaxed);
             return RESIDENT_REFUSED;
         }
-        MFD_HIP(e);
     }
     return MFD_OK;
 }

@@ -25,9 +25,10 @@ template <typename R>
 int resident_steps(mfd_op *op, int64_t nrhs, int steps, int chunk, double near);
 
 // Scal::stag of a right-hand side whose blocks gave up waiting for each other;
-// what resident_steps returns when the device refused the launch (fewer places
-// than it reported): the state is still that between steps, resident_ok is
-// false from then on, and the step-by-step kernels go on
+// what resident_steps returns when the launch was refused (fewer places than the
+// device reported, or another process holds its cooperative queue): the state is
+// still that between steps, resident_ok is false for the context's operators for
+// some seconds, and the step-by-step kernels go on
 enum { RESIDENT_TIMEOUT = -1, RESIDENT_REFUSED = -2 };
 
 }  // namespace mfd
