@@ -252,8 +252,10 @@ int mfd_op_autotune(mfd_op *op, int64_t nrhs, int iters, int tile64[3], int tile
  * launch chooses TY in {4, 8} and KZ from 1 to 20 by how many rounds of tiles
  * the fullest CU runs, XCD order, and 32-wide tiles (xcd_order 3) when that
  * stencil serves and they leave fewer lanes of the last x tile idle than
- * 64-wide ones.  Small SQMR solves do not use the
- * tiles (one kernel keeps the whole grid on chip) unless they were set here. */
+ * 64-wide ones, with constants of the kernel that runs.  Small SQMR solves of one
+ * or a few right-hand sides do not use the tiles (one kernel keeps the whole grid
+ * on chip) unless they were set here.  A grid whose x-y plane has too many tiles
+ * for a solve's reductions gets taller ones, or the direct kernel. */
 int mfd_op_set_tile(mfd_op *op, int prec, int ty, int kz, int xcd_order);
 /* Average device time (ms) of one apply of the solver's stencil kernel
  * (MFD_FP64: A; MFD_MIXED: the complex-FP32 inner operator) */
