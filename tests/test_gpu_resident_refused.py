@@ -18,7 +18,8 @@ int hipLaunchCooperativeKernel(const void *f, ...) { (void)f; ++calls; return ER
 """
 
 PROGRAM = """
-import ctypes as C, os, sys
+import ctypes as C, os, sys, time
+start = time.monotonic()
 shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 for p in ("maxwellfdm.jl_amd", "oracle", "tests"):
     sys.path.insert(0, os.path.join(sys.argv[2], p))
@@ -32,8 +33,9 @@ for N in ((13, 9, 11), (10, 12, 7)):
     made.append((pkg.MaxwellOperator(m, OM), O.to_scipy(O.create_A(spec_of(m), OM, m.εarr, m.μarr)), rng))
 def check(A, b, e):
     assert np.linalg.norm(b - A @ e) <= 1.01 * TOL * np.linalg.norm(b)
-def calls():
-    return C.c_int.in_dll(shim, "calls").value
+def asked():   # once, and again after 10 s only
+    n = C.c_int.in_dll(shim, "calls").value
+    return 1 <= n <= 1 + (time.monotonic() - start) / 10
 op, A, rng = made[0]
 for precision in ("fp64", "mixed"):
     b = rng.normal(size=(2, A.shape[0])) + 1j * rng.normal(size=(2, A.shape[0]))
@@ -41,8 +43,8 @@ for precision in ("fp64", "mixed"):
         e, st = op.solve(rhs, tol=TOL, precision=precision)
         for r, x in zip(np.atleast_2d(rhs), np.atleast_2d(e)):
             check(A, r, x)
-print("single ok", calls(), flush=True)
-assert calls() == 1          # nobody asks again for some seconds
+print("single ok", flush=True)
+assert asked()
 op.close()
 m, rng = system(pkg, (13, 9, 11), (False,) * 3, (0, 0, 0), "diag", 51)
 made[0] = (pkg.MaxwellOperator(m, OM), A, rng)
@@ -50,7 +52,7 @@ bs = [rng.normal(size=A.shape[0]) + 0j for _, A, rng in made]
 es, _ = pkg.solve_batch([op for op, _, _ in made], bs, tol=TOL)
 for (_, A, _), b, e in zip(made, bs, es):
     check(A, b, e)
-assert calls() == 1
+assert asked()
 print("batch ok", flush=True)
 """
 
